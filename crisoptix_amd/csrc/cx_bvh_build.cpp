@@ -461,6 +461,7 @@ bool collapse_bvh(const BvhHost& bin, int width, uint32_t stackLimit, std::vecto
               collapse_with(bin, width, true, stackLimit, out, root, stackBound);
     // Every reference must be empty, an inner node of `out` or a leaf inside the triangle slots.
     const size_t nodeWords = 2 * (size_t)width, numNodes = out.size() / nodeWords;
+    ok = ok && out.size() * sizeof(float4) <= WIDE_BYTES_MAX;
     const uint64_t slots = bin.tris.size() >= TRI_PAD ? (bin.tris.size() - TRI_PAD) / 3 : 0;
     for (size_t i = 0; ok && i < numNodes; i++)
         for (int g = 0; g < width / 4; g++) {

@@ -1035,7 +1035,8 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
         };
         e = collapse(dp);
         if (e == hipSuccess && sc[1] + 1 > (uint32_t)STACK_DEPTH) e = collapse(WideDP{nullptr, nullptr, nullptr});
-        if (e == hipSuccess && sc[1] + 1 <= (uint32_t)STACK_DEPTH) {
+        if (e == hipSuccess && sc[1] + 1 <= (uint32_t)STACK_DEPTH &&
+            (uint64_t)numWide * words * sizeof(float4) <= WIDE_BYTES_MAX) {
             hipLaunchKernelGGL(k_check_refs, blocks(numWide), dim3(BB), 0, s, wnodes, numWide, words, n, bad);
             allocs.push_back(wnodes);
             out.wnodes = wnodes;

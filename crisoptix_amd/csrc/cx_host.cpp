@@ -950,9 +950,18 @@ int cx_bvh_host_trace(const cx_scene_desc* d, const float* rays, uint32_t n, int
     S.wroot = wroot;
     S.width = width;
     struct HostStack {
-        int e[STACK_DEPTH];
+        int e[STACK_DEPTH] = {};
         void put(int i, int x) { e[i] = x; }
-        int get(int i) const { return e[i]; }
+        int peek(int sp) const { return e[sp > 0 ? sp - 1 : 0]; }
+        int pop(int& sp, int peeked) const {
+            --sp;
+            return peeked;
+        }
+        void push3(int& sp, int c1, int c2, int c3, bool h1, bool h2, bool h3) {
+            if (h3) put(sp++, c3);
+            if (h2) put(sp++, c2);
+            if (h1) put(sp++, c1);
+        }
     };
     // The stepped traversal of the queue-trace kernel (trav_init / trav_step), one ray at a time.
     auto run = [&](auto widthTag, auto anyTag, TravRay& tr, HostStack& st) {

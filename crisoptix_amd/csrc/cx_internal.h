@@ -108,10 +108,12 @@ hipError_t wave_launch(int kernel, const WaveArgs& W, uint32_t threads, hipStrea
 static constexpr uint32_t DEFAULT_MAX_LEAF = 2;
 
 // Host BVH build output (binary SAH BVH in the node format of cx_scene_dev.h).
-// Zero float4 after the last triangle slot of every triangle array the traversal reads: the
-// 4-wide traversal step loads 7 float4 from a leaf's first slot whatever the leaf's size, so the
-// loads of a last leaf of one triangle end 4 float4 past the slots.
+// Zero float4 after the last triangle slot of every triangle array the traversal reads.
 static constexpr size_t TRI_PAD = 4;
+
+// Most bytes of a wide node array: the traversal addresses its nodes by 32-bit byte offsets.  A
+// larger one (more than 33 M 4-wide nodes) is replaced by the binary tree.
+static constexpr uint64_t WIDE_BYTES_MAX = uint64_t(1) << 32;
 
 struct BvhHost {
     std::vector<float4> nodes;   // 4 per inner node

@@ -8,6 +8,7 @@
 namespace cx {
 
 static constexpr int BLOCK = 128;
+static_assert(BLOCK == TRACE_BLOCK, "the traversal stack's column stride");
 static constexpr int TILE_X = 16;
 static constexpr int TILE_Y = 8;
 
@@ -925,9 +926,9 @@ __global__ __launch_bounds__(BLOCK) void k_trace(DScene S, const float* rays, ui
     Hit h;
     const V3 o = V3{r[0], r[1], r[2]}, d = V3{r[3], r[4], r[5]};
     if (anyHit) {
-        occ[i] = traverse<true>(S, o, d, r[6], r[7], h, s_stack + threadIdx.x, BLOCK) ? 1u : 0u;
+        occ[i] = traverse<true>(S, o, d, r[6], r[7], h, s_stack + threadIdx.x) ? 1u : 0u;
     } else {
-        traverse<false>(S, o, d, r[6], r[7], h, s_stack + threadIdx.x, BLOCK);
+        traverse<false>(S, o, d, r[6], r[7], h, s_stack + threadIdx.x);
         const bool hit = h.prim != INVALID_PRIM;
         prim[i] = h.prim;
         t[i] = hit ? h.t : 0.0f;

@@ -127,56 +127,92 @@ struct Hit {
     float t, u, v;
 };
 
-// Slab test of both children of a node; the far plane carries a relative slack so that a
-// triangle whose computed t equals the current best is never pruned.
-CX_HD void box2(const float4 a, const float4 b, const float4 c, V3 o, V3 inv, float tmin,
-                                     float tcap, bool& hit0, bool& hit1, float& tn0, float& tn1) {
-    const float l0x = (a.x - o.x) * inv.x, h0x = (a.y - o.x) * inv.x;
-    const float l0y = (a.z - o.y) * inv.y, h0y = (a.w - o.y) * inv.y;
-    const float l0z = (c.x - o.z) * inv.z, h0z = (c.y - o.z) * inv.z;
-    const float l1x = (b.x - o.x) * inv.x, h1x = (b.y - o.x) * inv.x;
-    const float l1y = (b.z - o.y) * inv.y, h1y = (b.w - o.y) * inv.y;
-    const float l1z = (c.z - o.z) * inv.z, h1z = (c.w - o.z) * inv.z;
-    const float n0 = fmaxf(fmaxf(fminf(l0x, h0x), fminf(l0y, h0y)), fmaxf(fminf(l0z, h0z), tmin));
-    const float f0 = fminf(fminf(fmaxf(l0x, h0x), fmaxf(l0y, h0y)), fminf(fmaxf(l0z, h0z), tcap));
-    const float n1 = fmaxf(fmaxf(fminf(l1x, h1x), fminf(l1y, h1y)), fmaxf(fminf(l1z, h1z), tmin));
-    const float f1 = fminf(fminf(fmaxf(l1x, h1x), fmaxf(l1y, h1y)), fminf(fmaxf(l1z, h1z), tcap));
-    hit0 = n0 <= f0 * 1.00002f + 1e-30f;
-    hit1 = n1 <= f1 * 1.00002f + 1e-30f;
-    tn0 = n0;
-    tn1 = n1;
+// The slab tests of a ray: the plane x_i = c is crossed at fma(c, inv_i, -o_i inv_i), one operation
+// per plane.  The rounding of the product o_i inv_i is an absolute error in t, so it is kept as an
+// interval: nn_i (used for the near planes) lies below it, nf_i (far planes) above it, and the one
+// rounding of the fma is relative and covered by the far plane's slack; every box the ray enters
+// is so reported as entered.  A ray with d_i = 0 never changes x_i: its inv_i is a large power of
+// two (the product is then exact) and its interval is widened by 2^-40 in x_i, so that a box
+// whose face holds the origin is entered.  A component that overflows makes nn_i or nf_i infinite
+// or NaN, which fmaxf / fminf pass over: the axis then constrains nothing.
+struct RaySlab {
+    V3 inv, nn, nf;
+};
+
+CX_HD void slab_axis(float o, float d, float big, float& inv, float& nn, float& nf) {
+    inv = d == 0.0f ? copysignf(big, d) : 1.0f / d;
+    const float noi = -(o * inv);
+    const float e = (fabsf(noi) * 1.1920929e-7f + 1e-30f) + (d == 0.0f ? big * 9.094947e-13f : 0.0f);
+    nn = noi - e;
+    nf = noi + e;
+}
+
+CX_HD RaySlab slab_init(V3 o, V3 d) {
+    const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+    // 2^96 over the power of two at or below the largest component (0 and denormals as they are)
+    const float p = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, m) & 0x7f800000u);
+    const float big = 7.9228163e28f / (p > 0.0f ? p : 1.0f);
+    RaySlab r;
+    slab_axis(o.x, d.x, big, r.inv.x, r.nn.x, r.nf.x);
+    slab_axis(o.y, d.y, big, r.inv.y, r.nn.y, r.nf.y);
+    slab_axis(o.z, d.z, big, r.inv.z, r.nn.z, r.nf.z);
+    return r;
+}
+
+// Entry distance of a box whose near and far planes (by the signs of inv) are given, and whether
+// the ray enters it in [tmin, tcap].  The far plane carries a relative slack so that a triangle
+// whose computed t equals the current best is never pruned.
+CX_HD float slab_box(float nx, float fx, float ny, float fy, float nz, float fz, const RaySlab& r, float tmin,
+                     float tcap, bool& hit) {
+    const float n = fmaxf(fmaxf(fmaf(nx, r.inv.x, r.nn.x), fmaf(ny, r.inv.y, r.nn.y)),
+                          fmaxf(fmaf(nz, r.inv.z, r.nn.z), tmin));
+    const float f = fminf(fminf(fmaf(fx, r.inv.x, r.nf.x), fmaf(fy, r.inv.y, r.nf.y)),
+                          fminf(fmaf(fz, r.inv.z, r.nf.z), tcap));
+    hit = n <= fmaf(fabsf(f), 2e-5f, f);
+    return n;
 }
 
 __device__ __forceinline__ V3 load_v3(const float* p, uint32_t i) { return V3{p[3 * i], p[3 * i + 1], p[3 * i + 2]}; }
 
-// Traversal stack: the first SHORT entries in a per-thread LDS column (lds[i * stride]), deeper
-// entries in a per-lane private array.
+// Traversal stack: the first SHORT entries in a per-thread LDS column (lds[i * STRIDE]), deeper
+// entries in a per-lane private array that the caller declares beside it (STACK_OVF entries; an
+// array inside this struct would pin the whole struct in private memory).
 template <int SHORT>
+static constexpr int STACK_OVF = STACK_DEPTH - SHORT > 0 ? STACK_DEPTH - SHORT : 1;
+
+template <int SHORT, int STRIDE>
 struct TravStack {
     int* lds;
-    int stride;
-    int ovf[STACK_DEPTH - SHORT > 0 ? STACK_DEPTH - SHORT : 1];
+    int* ovf;
     CX_HD void put(int i, int v) {
-        if (SHORT >= STACK_DEPTH || i < SHORT) lds[i * stride] = v;
+        if (SHORT >= STACK_DEPTH || i < SHORT) lds[i * STRIDE] = v;
         else ovf[i - SHORT] = v;
     }
-    CX_HD int get(int i) const {
-        if (SHORT >= STACK_DEPTH || i < SHORT) return lds[i * stride];
-        return ovf[i - SHORT];
+    // The entry below depth sp, read ahead of its use (any value when sp is 0 or the entry lies in
+    // private memory), and the pop of it.
+    CX_HD int peek(int sp) const { return lds[(sp > 0 && (SHORT >= STACK_DEPTH || sp <= SHORT) ? sp - 1 : 0) * STRIDE]; }
+    CX_HD int pop(int& sp, int peeked) const {
+        --sp;
+        int v = peeked;
+        if (SHORT < STACK_DEPTH && sp >= SHORT) v = ovf[sp - SHORT];
+        return v;
     }
-};
-
-// A traversal stack with its top entry in a register: a pop takes the register,
-// and the stack read that refills it is needed only at the next push or pop, so it is not on
-// the path from a pop to the fetch of the popped node.
-template <typename Stack>
-struct TopStack {
-    Stack& st;
-    int& top;
-    // push of entry i (= the current depth)
-    CX_HD void put(int i, int v) {
-        if (i > 0) st.put(i - 1, top);
-        top = v;
+    // Pushes c3, c2, c1 in this order, of which only the first n entries of (c1, c2, c3) are
+    // valid; sp becomes sp + n.  While all three fit in LDS they are stored without branches, the
+    // invalid ones above the new top.
+    CX_HD void push3(int& sp, int c1, int c2, int c3, bool h1, bool h2, bool h3) {
+        if (sp + 3 <= SHORT) {
+            int* const b = lds + sp * STRIDE;
+            const int a2 = h2 ? 1 : 0, a3 = h3 ? 1 : 0;
+            b[(a2 + a3) * STRIDE] = c1;
+            b[h2 && !h3 ? 0 : STRIDE] = c2;
+            b[h3 ? 0 : 2 * STRIDE] = c3;
+            sp += (h1 ? 1 : 0) + a2 + a3;
+        } else {
+            if (h3) put(sp++, c3);
+            if (h2) put(sp++, c2);
+            if (h1) put(sp++, c1);
+        }
     }
 };
 
@@ -227,15 +263,21 @@ CX_HD bool leaf_hits(const DScene& S, int32_t ref, V3 o, const RayPre& rp, float
     return leaf_hits_rt(S, ref, o, rp, tmin, best, ANY);
 }
 
-// One triangle of a leaf, its slot already loaded in q[0..2]: leaf_hits' test of that triangle.
+// One triangle of a leaf, its slot already loaded in q0..q2: leaf_hits' test of that triangle.
 // Returns true when an any-hit query is answered.
-CX_HD bool tri_hits_q(const float4* q, V3 o, const RayPre& rp, float tmin, Hit& best, bool any) {
-    if (__builtin_bit_cast(uint32_t, q[1].w) & (any ? 2u : 1u)) return false;   // invisible to this ray kind
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// The bits of a value.  By value: __builtin_bit_cast applied directly to an element of a vector
+// reads the vector's first element.
+CX_HD uint32_t bits_of(float x) { return __builtin_bit_cast(uint32_t, x); }
+
+CX_HD bool tri_hits_q(f32x4 q0, f32x4 q1, f32x4 q2, V3 o, const RayPre& rp, float tmin, Hit& best, bool any) {
+    if (bits_of(q1[3]) & (any ? 2u : 1u)) return false;   // invisible to this ray kind
     float t, u, v;
-    if (!tri_hit(o, rp, V3{q[0].x, q[0].y, q[0].z}, V3{q[1].x, q[1].y, q[1].z}, V3{q[2].x, q[2].y, q[2].z}, tmin,
-                 best.t, t, u, v))
+    if (!tri_hit(o, rp, V3{q0[0], q0[1], q0[2]}, V3{q1[0], q1[1], q1[2]}, V3{q2[0], q2[1], q2[2]}, tmin, best.t, t, u,
+                 v))
         return false;
-    const uint32_t prim = __builtin_bit_cast(uint32_t, q[0].w);
+    const uint32_t prim = bits_of(q0[3]);
     if (any) {
         best.prim = prim;
         best.t = t;
@@ -250,64 +292,115 @@ CX_HD bool tri_hits_q(const float4* q, V3 o, const RayPre& rp, float tmin, Hit& 
     return false;
 }
 
-// Slab test of one child of a wide node (same arithmetic and slack as box2).
-CX_HD float box1(float lx, float hx, float ly, float hy, float lz, float hz, V3 o, V3 inv,
-                                      float tmin, float tcap, bool& hit) {
-    const float ax = (lx - o.x) * inv.x, bx = (hx - o.x) * inv.x;
-    const float ay = (ly - o.y) * inv.y, by = (hy - o.y) * inv.y;
-    const float az = (lz - o.z) * inv.z, bz = (hz - o.z) * inv.z;
-    const float n = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fmaxf(fminf(az, bz), tmin));
-    const float f = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fminf(fmaxf(az, bz), tcap));
-    hit = n <= f * 1.00002f + 1e-30f;
-    return n;
+// A child box's entry distance and reference as one double, the distance's bits in the high word:
+// for the distances of hit boxes (any float but NaN, +inf marking a miss) the order of the doubles
+// is the order of the distances, so a compare-exchange is a minimum and a maximum (v_min_f64 and
+// v_max_f64 issue at the rate of the 32-bit operations on gfx950) instead of a comparison and four
+// selects.  The low word only breaks ties.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+CX_HD double hit_key(float t, int ref) {
+    return __builtin_bit_cast(double, u32x2{(uint32_t)ref, __builtin_bit_cast(uint32_t, t)});
 }
 
-CX_HD void cswap(float& ta, int& ra, float& tb, int& rb) {
-    const bool sw = tb < ta;
-    const float t = sw ? tb : ta;
-    const int r = sw ? rb : ra;
-    tb = sw ? ta : tb;
-    rb = sw ? ra : rb;
-    ta = t;
-    ra = r;
+CX_HD int key_ref(double k) {
+    const u32x2 b = __builtin_bit_cast(u32x2, k);
+    return (int)b.x;
+}
+CX_HD bool key_miss(double k) {
+    const u32x2 b = __builtin_bit_cast(u32x2, k);
+    return b.y == 0x7f800000u;
 }
 
-// One wide node: test the N child boxes, sort the hit ones by entry distance (a fixed
-// compare-exchange network on registers, misses at +inf), push all but the nearest, farthest
-// first, and return the nearest in ref; false (ref unchanged) when no child box is hit.  q holds
-// the node's first 7 float4 per group of 4 children (bounds lo.x, hi.x, lo.y, hi.y, lo.z, hi.z
-// of the 4 children, then their references), already loaded.
-template <int N, typename Stack>
-CX_HD bool wide_visit_q(const float4* q, int& ref, V3 o, V3 inv, float tmin, float tcap, Stack& st, int& sp) {
-    float tn[N];
-    int cr[N];
-#pragma unroll
-    for (int g = 0; g < N / 4; g++) {
-        const float4 lx = q[7 * g + 0], hx = q[7 * g + 1], ly = q[7 * g + 2], hy = q[7 * g + 3];
-        const float4 lz = q[7 * g + 4], hz = q[7 * g + 5];
-        const int4 rr = __builtin_bit_cast(int4, q[7 * g + 6]);
-        const float lxa[4] = {lx.x, lx.y, lx.z, lx.w}, hxa[4] = {hx.x, hx.y, hx.z, hx.w};
-        const float lya[4] = {ly.x, ly.y, ly.z, ly.w}, hya[4] = {hy.x, hy.y, hy.z, hy.w};
-        const float lza[4] = {lz.x, lz.y, lz.z, lz.w}, hza[4] = {hz.x, hz.y, hz.z, hz.w};
-        const int ra[4] = {rr.x, rr.y, rr.z, rr.w};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            bool h;
-            const float t = box1(lxa[j], hxa[j], lya[j], hya[j], lza[j], hza[j], o, inv, tmin, tcap, h);
-            const bool use = h && ra[j] != WIDE_EMPTY;
-            tn[4 * g + j] = use ? t : INFINITY;
-            cr[4 * g + j] = ra[j];
-        }
+CX_HD void key_cswap(double& a, double& b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    // the instructions themselves: fmin and fmax would quiet their operands first
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
+#else
+    if (b < a) {
+        const double t = a;
+        a = b;
+        b = t;
     }
+#endif
+}
+
+// One wide node (2 N float4 per node, the 8th of each group of 4 children unused): test the N
+// child boxes, sort the hit ones by entry distance (a fixed compare-exchange network on
+// registers, misses last), push all but the nearest, farthest first, and return the nearest in
+// ref; false (ref unchanged) when no child box is hit.  The near and far planes of an axis are
+// chosen by address, from the sign of the ray's direction, so no minimum or maximum is needed per
+// plane pair: a node's offset is a 32-bit number of bytes (cx_scene_build keeps the array below
+// 4 GiB), and a far plane lies 16 bytes from its near plane.
+#ifdef __HIP_DEVICE_COMPILE__
+typedef const f32x4 __attribute__((address_space(1)))* gf32x4;   // a global-memory address
+#else
+typedef const f32x4* gf32x4;
+#endif
+
+struct WideLoads {
+    f32x4 nx, fx, ny, fy, nz, fz, ref;
+};
+
+CX_HD f32x4 load_at(const float4* base, uint32_t bytes) { return *(const f32x4*)((const char*)base + bytes); }
+
+CX_HD WideLoads wide_load(const float4* nodes, uint32_t off, const RaySlab& r) {
+    const uint32_t ax = off + ((__builtin_bit_cast(uint32_t, r.inv.x) >> 27) & 16u);
+    const uint32_t ay = off + ((__builtin_bit_cast(uint32_t, r.inv.y) >> 27) & 16u);
+    const uint32_t az = off + ((__builtin_bit_cast(uint32_t, r.inv.z) >> 27) & 16u);
+    WideLoads w;
+    w.nx = load_at(nodes, ax);
+    w.fx = load_at(nodes, ax ^ 16u);
+    w.ny = load_at(nodes + 2, ay);
+    w.fy = load_at(nodes + 2, ay ^ 16u);
+    w.nz = load_at(nodes + 4, az);
+    w.fz = load_at(nodes + 4, az ^ 16u);
+    w.ref = load_at(nodes + 6, off);
+    return w;
+}
+
+CX_HD void wide_keys(const WideLoads& w, const RaySlab& r, float tmin, float tcap, double* k) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        bool h;
+        const float t = slab_box(w.nx[j], w.fx[j], w.ny[j], w.fy[j], w.nz[j], w.fz[j], r, tmin, tcap, h);
+        const int ref = (int)bits_of(w.ref[j]);
+        k[j] = hit_key(h && ref != WIDE_EMPTY ? t : INFINITY, ref);
+    }
+}
+
+// wide_visit of a 4-wide node whose float4 are loaded.
+template <typename Stack>
+CX_HD bool wide_visit4(const WideLoads& w, int& ref, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
+    double k[4];
+    wide_keys(w, r, tmin, tcap, k);
+    key_cswap(k[0], k[1]);
+    key_cswap(k[2], k[3]);
+    key_cswap(k[0], k[2]);
+    key_cswap(k[1], k[3]);
+    key_cswap(k[1], k[2]);
+    if (key_miss(k[0])) return false;
+    st.push3(sp, key_ref(k[1]), key_ref(k[2]), key_ref(k[3]), !key_miss(k[1]), !key_miss(k[2]), !key_miss(k[3]));
+    ref = key_ref(k[0]);
+    return true;
+}
+
+template <int N, typename Stack>
+CX_HD bool wide_visit(const DScene& S, int& ref, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
     if constexpr (N == 4) {
-        cswap(tn[0], cr[0], tn[1], cr[1]);
-        cswap(tn[2], cr[2], tn[3], cr[3]);
-        cswap(tn[0], cr[0], tn[2], cr[2]);
-        cswap(tn[1], cr[1], tn[3], cr[3]);
-        cswap(tn[1], cr[1], tn[2], cr[2]);
+        return wide_visit4(wide_load(S.wnodes, (uint32_t)ref * 128u, r), ref, r, tmin, tcap, st, sp);
     } else {
+        double k[8];
+        const WideLoads w0 = wide_load(S.wnodes, (uint32_t)ref * 256u, r);
+        const WideLoads w1 = wide_load(S.wnodes, (uint32_t)ref * 256u + 128u, r);
+        wide_keys(w0, r, tmin, tcap, k);
+        wide_keys(w1, r, tmin, tcap, k + 4);
         // Batcher's odd-even merge sort of 8 keys (19 compare-exchanges).
-#define CX_CS(a, b) cswap(tn[a], cr[a], tn[b], cr[b])
+#define CX_CS(a, b) key_cswap(k[a], k[b])
         CX_CS(0, 1); CX_CS(2, 3); CX_CS(4, 5); CX_CS(6, 7);
         CX_CS(0, 2); CX_CS(1, 3); CX_CS(4, 6); CX_CS(5, 7);
         CX_CS(1, 2); CX_CS(5, 6);
@@ -315,43 +408,28 @@ CX_HD bool wide_visit_q(const float4* q, int& ref, V3 o, V3 inv, float tmin, flo
         CX_CS(2, 4); CX_CS(3, 5);
         CX_CS(1, 2); CX_CS(3, 4); CX_CS(5, 6);
 #undef CX_CS
-    }
-    if (tn[0] == INFINITY) return false;
+        if (key_miss(k[0])) return false;
 #pragma unroll
-    for (int i = N - 1; i >= 1; i--) {
-        if (tn[i] != INFINITY) {
-            st.put(sp, cr[i]);
-            ++sp;
-        }
+        for (int i = 7; i >= 1; i--)
+            if (!key_miss(k[i])) st.put(sp++, key_ref(k[i]));
+        ref = key_ref(k[0]);
+        return true;
     }
-    ref = cr[0];
-    return true;
-}
-
-// wide_visit_q on node `ref` of the wide array (2 N float4 per node, the 8th of each group of
-// 4 children unused).
-template <int N, typename Stack>
-CX_HD bool wide_visit(const DScene& S, int& ref, V3 o, V3 inv, float tmin, float tcap, Stack& st, int& sp) {
-    const float4* n = S.wnodes + (size_t)ref * (2 * N);
-    float4 q[7 * (N / 4)];
-#pragma unroll
-    for (int g = 0; g < N / 4; g++) {
-#pragma unroll
-        for (int k = 0; k < 7; k++) q[7 * g + k] = n[8 * g + k];
-    }
-    return wide_visit_q<N>(q, ref, o, inv, tmin, tcap, st, sp);
 }
 
 // One binary node: the nearer hit child in ref (the farther one pushed); false when neither
 // child box is hit.
 template <typename Stack>
-CX_HD bool bin_visit(const DScene& S, int& ref, V3 o, V3 inv, float tmin, float tcap, Stack& st, int& sp) {
+CX_HD bool bin_visit(const DScene& S, int& ref, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
     const float4* n = S.nodes + 4 * (size_t)ref;
     const float4 a = n[0], b = n[1], c = n[2];
     const int4 dd = __builtin_bit_cast(int4, n[3]);
+    const bool sx = __builtin_signbitf(r.inv.x), sy = __builtin_signbitf(r.inv.y), sz = __builtin_signbitf(r.inv.z);
     bool h0, h1;
-    float t0, t1;
-    box2(a, b, c, o, inv, tmin, tcap, h0, h1, t0, t1);
+    const float t0 = slab_box(sx ? a.y : a.x, sx ? a.x : a.y, sy ? a.w : a.z, sy ? a.z : a.w, sz ? c.y : c.x,
+                              sz ? c.x : c.y, r, tmin, tcap, h0);
+    const float t1 = slab_box(sx ? b.y : b.x, sx ? b.x : b.y, sy ? b.w : b.z, sy ? b.z : b.w, sz ? c.w : c.z,
+                              sz ? c.z : c.w, r, tmin, tcap, h1);
     if (h0 && h1) {
         const bool first0 = t0 <= t1;
         st.put(sp, first0 ? dd.y : dd.x);
@@ -368,18 +446,17 @@ template <bool ANY, int N, typename Stack>
 CX_HD bool traverse_wide(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& best,
                                               Stack& st) {
     const RayPre rp = ray_pre(d);
-    const V3 inv = V3{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+    const RaySlab sl = slab_init(o, d);
     int sp = 0;
     int ref = S.wroot;
     while (true) {
         if (ref >= 0) {
-            if (wide_visit<N>(S, ref, o, inv, tmin, best.t, st, sp)) continue;
+            if (wide_visit<N>(S, ref, sl, tmin, best.t, st, sp)) continue;
         } else {
             if (leaf_hits<ANY>(S, ref, o, rp, tmin, best)) return true;
         }
         if (sp == 0) break;
-        --sp;
-        ref = st.get(sp);
+        ref = st.pop(sp, st.peek(sp));
     }
     return best.prim != INVALID_PRIM;
 }
@@ -393,18 +470,17 @@ CX_HD bool traverse_bin(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit
     best.v = 0.0f;
     if (S.numTris == 0) return false;
     const RayPre rp = ray_pre(d);
-    const V3 inv = V3{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+    const RaySlab sl = slab_init(o, d);
     int sp = 0;
     int ref = S.root;
     while (true) {
         if (ref >= 0) {
-            if (bin_visit(S, ref, o, inv, tmin, best.t, st, sp)) continue;
+            if (bin_visit(S, ref, sl, tmin, best.t, st, sp)) continue;
         } else {
             if (leaf_hits<ANY>(S, ref, o, rp, tmin, best)) return true;
         }
         if (sp == 0) break;
-        --sp;
-        ref = st.get(sp);
+        ref = st.pop(sp, st.peek(sp));
     }
     return best.prim != INVALID_PRIM;
 }
@@ -414,55 +490,65 @@ CX_HD bool traverse_bin(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit
 // without waiting for the rest of its wavefront).  The answer is the loop's: the same nodes in
 // the same order.
 struct TravRay {
-    V3 o, inv;
+    V3 o;
+    RaySlab sl;
     RayPre rp;
     float tmin;
     Hit best;   // best.t: the ray's tmax until a hit lowers it
     int ref;
     int sp;
-    int top;   // stack entry sp - 1 (valid when sp > 0); the stack holds entries 0 .. sp - 2
 };
 
 
 template <int WIDTH>
 CX_HD void trav_init(const DScene& S, TravRay& r, V3 o, V3 d, float tmin, float tmax) {
     r.o = o;
-    r.inv = V3{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+    r.sl = slab_init(o, d);
     r.rp = ray_pre(d);
     r.tmin = tmin;
     r.best = Hit{INVALID_PRIM, tmax, 0.0f, 0.0f};
     r.ref = WIDTH == 2 ? S.root : S.wroot;
     r.sp = 0;
-    r.top = 0;
 }
 
 // One step; true when the ray is answered: closest hit in r.best (prim INVALID_PRIM: a miss),
 // occlusion as r.best.prim != INVALID_PRIM.  A scene without triangles answers at once.
 //
-// At width 4 a step makes one fetch for both kinds of lane: a lane at an inner node loads the
-// node's 7 float4, a lane at a leaf the 7 float4 from the slot of its next triangle (that
-// triangle's 3, then 4 unused), in the same load instructions, before either kind is processed.
-// A leaf step tests one triangle and leaves the lane on the rest of the leaf, so the leaf branch
-// of a wavefront split between nodes and leaves costs one triangle test per step.  A wavefront whose
-// lanes are split between nodes and leaves so waits once per step instead of once for the node
-// fetches and again for the triangle fetches.
+// The stack's top entry is read at the start of the step, with the node or triangle fetch, so a
+// pop at its end finds it in a register.  At width 4 the lanes at inner nodes and the lanes at
+// leaves issue their fetches (7 and 3 float4) before either kind is processed, so a wavefront
+// split between the two waits once per step; a leaf step tests one triangle and leaves the lane
+// on the rest of the leaf, so the leaf branch costs one triangle test per step.
 template <int WIDTH, typename Stack>
-CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& stack, bool any) {
+CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& st, bool any) {
     if (S.numTris == 0) return true;
-    TopStack<Stack> st{stack, r.top};
+    const int top = st.peek(r.sp);
     if constexpr (WIDTH == 4) {
         const bool inner = r.ref >= 0;
         const uint32_t code = ~(uint32_t)r.ref;
-        // a leaf's 7 loads run past its next triangle into the following slots, or into the
-        // TRI_PAD float4 after the last slot; one base address, seven immediate offsets
-        const float4* base = inner ? S.wnodes + (size_t)r.ref * 8 : S.tris + 3 * (size_t)(code >> 4);
-        float4 q[7];
-#pragma unroll
-        for (uint32_t k = 0; k < 7; k++) q[k] = base[k];
+        gf32x4 tv = (gf32x4)S.tris + 3 * (size_t)(code >> 4);
+        int kind = inner ? 1 : 0;
+#ifdef __HIP_DEVICE_COMPILE__
+        // the triangle's address is formed ahead of the node's loads, so that both kinds of lane
+        // load into the same registers without a wait between them
+        asm("" : "+v"(tv));
+        asm("" : "+v"(kind));
+#endif
+        WideLoads w;
+        if (inner) w = wide_load(S.wnodes, (uint32_t)r.ref * 128u, r.sl);
+        if (!kind) {
+            w.nx = tv[0];
+            w.fx = tv[1];
+            w.ny = tv[2];
+        }
+#ifdef __HIP_DEVICE_COMPILE__
+        // one wait for the loads of both kinds, here
+        asm("" : "+v"(w.nx), "+v"(w.fx), "+v"(w.ny), "+v"(w.fy), "+v"(w.nz), "+v"(w.fz), "+v"(w.ref));
+#endif
         if (inner) {
-            if (wide_visit_q<4>(q, r.ref, r.o, r.inv, r.tmin, r.best.t, st, r.sp)) return false;
+            if (wide_visit4(w, r.ref, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
         } else {
-            if (tri_hits_q(q, r.o, r.rp, r.tmin, r.best, any)) return true;
+            if (tri_hits_q(w.nx, w.fx, w.ny, r.o, r.rp, r.tmin, r.best, any)) return true;
             if ((code & 15u) > 1u) {
                 r.ref = (int32_t)~(code + 15u);   // the rest of the leaf, from its next slot
                 return false;
@@ -470,17 +556,15 @@ CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& stack, bool any) {
         }
     } else if (r.ref >= 0) {
         if constexpr (WIDTH == 2) {
-            if (bin_visit(S, r.ref, r.o, r.inv, r.tmin, r.best.t, st, r.sp)) return false;
+            if (bin_visit(S, r.ref, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
         } else {
-            if (wide_visit<WIDTH>(S, r.ref, r.o, r.inv, r.tmin, r.best.t, st, r.sp)) return false;
+            if (wide_visit<WIDTH>(S, r.ref, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
         }
     } else {
         if (leaf_hits_rt(S, r.ref, r.o, r.rp, r.tmin, r.best, any)) return true;
     }
     if (r.sp == 0) return true;
-    --r.sp;
-    r.ref = r.top;
-    if (r.sp > 0) r.top = stack.get(r.sp - 1);
+    r.ref = st.pop(r.sp, top);
     return false;
 }
 
@@ -509,13 +593,13 @@ CX_HD bool traverse_s(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& 
     return traverse_w<ANY, 2>(S, o, d, tmin, tmax, best, st);
 }
 
-// Traversal with the whole stack in a per-thread LDS column (stack[i * stride]).
+// Traversal with the whole stack in a per-thread LDS column (stack[i * TRACE_BLOCK]).
+static constexpr int TRACE_BLOCK = 128;   // threads per block (the column stride) of the kernels that use it
+
 template <bool ANY>
 __device__ __forceinline__ bool traverse(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& best,
-                                         int* stack, int stride) {
-    TravStack<STACK_DEPTH> st;
-    st.lds = stack;
-    st.stride = stride;
+                                         int* stack) {
+    TravStack<STACK_DEPTH, TRACE_BLOCK> st{stack, nullptr};
     return traverse_s<ANY>(S, o, d, tmin, tmax, best, st);
 }
 
@@ -579,7 +663,7 @@ __device__ __forceinline__ void trace_surface(const DScene& S, TraceCtx& tc, V3 
                                               Inter& io) {
     Hit h;
     tc.closest++;
-    traverse<false>(S, o, d, tmin, tmax, h, tc.stack, tc.stride);
+    traverse<false>(S, o, d, tmin, tmax, h, tc.stack);
     io.dir = d;
     if (h.prim == INVALID_PRIM) {
         io.valid = false;
@@ -598,7 +682,7 @@ __device__ __forceinline__ void trace_surface(const DScene& S, TraceCtx& tc, V3 
 __device__ __forceinline__ bool trace_occluded(const DScene& S, TraceCtx& tc, V3 o, V3 d, float tmin, float tmax) {
     Hit h;
     tc.shadow++;
-    return traverse<true>(S, o, d, tmin, tmax, h, tc.stack, tc.stride);
+    return traverse<true>(S, o, d, tmin, tmax, h, tc.stack);
 }
 
 // ---- BSDF (shader/brdf.cu) ----

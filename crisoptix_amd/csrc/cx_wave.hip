@@ -128,9 +128,13 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, 
 // zeroes the stripe counts of qout (the next step kernel's output queue) and adds the rays to
 // the pass counters.  Each wavefront traces its chunks of the closest rays and then of the
 // shadow rays in one refill loop (trace_chunks), and the grid is what fits on the device at
-// once.  The 4-wide kernel is held to at least 7 waves per SIMD: 72 VGPRs, 8 bytes per lane
-// more of private stack than at its natural 74 VGPRs and 6 waves (1080p frame 22.75-22.82 ms at
-// 7 waves, 22.91 at 6, 23.57-23.61 at 8, 25.6 held to exactly 5).  The 2-wide kernel keeps at
+// once.  What bounds it is the issue of vector instructions (two thirds of the SIMDs' cycles on
+// the 1080p frame's long launches) and, where a queue is short, the slowest ray's chain of
+// steps; so a step is kept short: planes by one fma each, near and far planes chosen by address,
+// children sorted as 64-bit keys, branch-free pushes (trav_step_rt).  About 110 vector
+// instructions for a node and 90 for a triangle against 190 and 110 before (1080p frame 21.8 ->
+// 19.3 ms, the 720p path tracer 2.39 -> 1.87 ms, a 160x90 frame 3.56 -> 3.09 ms).  The 4-wide
+// kernel is held to at least 7 waves per SIMD (72 VGPRs, no spills); the 2-wide kernel keeps at
 // least 5.
 template <int WIDTH>
 __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH == 8 ? 1 : (WIDTH == 4 ? 7 : 5), 8))) void k_q_trace(
@@ -147,9 +151,8 @@ __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH ==
             if (ns) atomicAdd(&counters[1], (unsigned long long)ns);
         }
     }
-    TravStack<SHORT_STACK> st;
-    st.lds = s_st + threadIdx.x;
-    st.stride = WBLOCK;
+    int ovf[STACK_OVF<SHORT_STACK>];
+    TravStack<SHORT_STACK, WBLOCK> st{s_st + threadIdx.x, ovf};
     const uint32_t waves = gridDim.x * (WBLOCK / 64), w = blockIdx.x * (WBLOCK / 64) + (threadIdx.x >> 6);
     trace_chunks<WIDTH>(S, qin, qi, nc, ns, w, waves, minChunk, st);
 }
@@ -1268,9 +1271,8 @@ struct Mach<WK_FG_STEP> {
 template <int M, int WIDTH>
 __global__ __launch_bounds__(WBLOCK) void k_w_tail(WaveArgs W, uint32_t maxSteps, int pass) {
     __shared__ int s_st[SHORT_STACK * WBLOCK];
-    TravStack<SHORT_STACK> st;
-    st.lds = s_st + threadIdx.x;
-    st.stride = WBLOCK;
+    int ovf[STACK_OVF<SHORT_STACK>];
+    TravStack<SHORT_STACK, WBLOCK> st{s_st + threadIdx.x, ovf};
     const DScene& S = W.A.S;
     uint32_t nClosest = 0, nShadow = 0;
     CX_FOR_JOBS(W) {

@@ -29,6 +29,53 @@ def test_host_traversal_matches_oracle(name, width, max_leaf, orc):
     assert np.array_equal(oo.astype(np.uint32), og)
 
 
+def axis_rays(sc, n, seed):
+    """Rays at the edges of the slab test's arithmetic: one or two direction components exactly
+    zero or far below the others (1e-9, 1e-20, 1e-40), of either sign, origins on vertex
+    coordinates (so on box faces, the ground plane y = 0 among them) or up to 1000 scene sizes
+    away along the ray's main axis, directions scaled by 1e-6 .. 1e6, tmax infinite or limited,
+    tmin 0 or 1e-3 over the scale (an origin on a surface has a rounding error of about 1e-8 in
+    space, which a tmin below it in space would let through as a hit at a point that the box of
+    its triangle does not hold)."""
+    rng = np.random.default_rng(seed)
+    pos = sc.positions.astype(np.float32)
+    size = np.float32(sc.scene_size())
+    rays = np.zeros((n, 8), np.float32)
+    for a in range(3):   # each coordinate that of a random vertex
+        rays[:, a] = pos[rng.integers(0, len(pos), n), a]
+    main = rng.integers(0, 3, n)
+    d = rng.choice([0.0, -0.0, 1e-9, -1e-9, 1e-20, -1e-20, 1e-40, -0.3, 0.4], size=(n, 3)).astype(np.float32)
+    sign = rng.choice([-1.0, 1.0], n).astype(np.float32)
+    d[np.arange(n), main] = sign
+    far = rng.random(n) < 0.4
+    away = (size * 10.0 ** rng.uniform(0, 3, n)).astype(np.float32)
+    straight = np.abs(d).sum(1) < 1.1          # a tilted far ray would pass the scene by
+    pick = far & straight
+    rays[pick, main[pick]] = -sign[pick] * away[pick]
+    rays[:, 3:6] = d * (10.0 ** rng.uniform(-6, 6, n)).astype(np.float32)[:, None]
+    rays[:, 6] = np.where(rng.random(n) < 0.5, 0.0, 1e-3 / np.abs(rays[:, 3:6]).max(1))
+    rays[:, 7] = np.where(rng.random(n) < 0.7, np.inf, size / np.abs(rays[:, 3:6]).max(1))
+    return rays
+
+
+@pytest.mark.parametrize("name", ["cornell", "grid3"])
+def test_axis_parallel_and_far_rays_match_brute_force(name, orc):
+    """The slab test's interval arithmetic loses no hit: closest hits and occlusion of every width
+    equal the oracle's loop over all triangles, bit for bit."""
+    sc = scenes.cornell_box(1, 8) if name == "cornell" else small_grid_scene()
+    rays = axis_rays(sc, 6000, seed=23)
+    brute = orc.OracleScene(sc, brute_force=True)
+    ref = brute.trace_closest(rays)
+    occ = brute.trace_occluded(rays).astype(np.uint32)
+    assert 0.2 < np.mean(ref[0] != 0xFFFFFFFF) < 0.98
+    for width in (2, 4, 8):
+        *got, _ = runtime.host_trace(sc, rays, width=width)
+        for x, y in zip(ref, got):
+            assert np.array_equal(bits(x), bits(y)), width
+        og, _ = runtime.host_trace(sc, rays, any_hit=True, width=width)
+        assert np.array_equal(occ, og), width
+
+
 def test_wide8_collapse_falls_back_to_greedy_on_large_scene():
     """The 1.06 M-triangle object grid of the 1080p benchmark: the least-area collapse at width 8
     needs more than 64 traversal-stack entries, so the collapse takes the greedy rule, which fits;
