@@ -502,7 +502,7 @@ hipError_t run_machine(cx_renderer* r, WaveArgs W, int setup, int step, uint32_t
     for (uint32_t i = 0; i < waveRounds && e == hipSuccess; i++) {
         const Queue qin = queue_view(r, cur, cap), qout = queue_view(r, 1 - cur, cap);
         trace_rec(r, s);
-        e = wave_trace(W.A.S, qin, qout, W.A.counters + 2 * pass, r->concurrent ? ~0u : 1u, s);
+        e = wave_trace(step, W, qin, qout, W.A.counters + 2 * pass, r->concurrent ? ~0u : 1u, s);
         trace_rec(r, s);
         W.qin = qin;
         W.qout = qout;

@@ -22,7 +22,15 @@ namespace cx {
 
 // ---- queues ----
 
-static constexpr uint32_t EMIT_NONE = 0, EMIT_CLOSEST = 1, EMIT_SHADOW = 2;
+// What a step of a job ends in: nothing more, a closest-hit ray, a shadow ray whose answer the
+// job's next step reads, or a final shadow ray.  A job that emits a final shadow ray has already
+// stored its result as it is if the ray is unoccluded; the kernel that answers the ray takes the
+// result back if it is occluded (final_answer), and the job has no further step and no context.
+static constexpr uint32_t EMIT_NONE = 0, EMIT_CLOSEST = 1, EMIT_SHADOW = 2, EMIT_FINAL = 3;
+
+// Bit of a queued job number that marks a final shadow ray where a machine has both kinds (the
+// suffix walk, whose job is a pixel below 2^28).
+static constexpr uint32_t JOB_FINAL = 0x80000000u;
 
 static constexpr uint32_t QSTRIPES = 64;       // one per lane of the wavefront that scans them
 static constexpr uint32_t QCOUNT_STRIDE = 16;  // words between stripes' counters (64 bytes)
@@ -119,6 +127,7 @@ struct Emit {
 CX_HD Emit emit_none() { return Emit{EMIT_NONE, v3(0.0f), v3(0.0f), 0.0f, 0.0f}; }
 CX_HD Emit emit_closest(V3 o, V3 d) { return Emit{EMIT_CLOSEST, o, d, 1e-3f, 1e16f}; }
 CX_HD Emit emit_shadow(V3 o, V3 d, float tmax) { return Emit{EMIT_SHADOW, o, d, 1e-3f, tmax}; }
+CX_HD Emit emit_final(V3 o, V3 d, float tmax) { return Emit{EMIT_FINAL, o, d, 1e-3f, tmax}; }
 
 // Slot of the input queue handled by thread i: the closest range [0, nc) first, then the
 // shadow range, each walked stripe by stripe.
@@ -141,7 +150,7 @@ __device__ __forceinline__ uint32_t in_slot(const Queue& q, const QIndex& x, uin
 // leaves the queue.
 __device__ __forceinline__ uint32_t append(const Queue& q, uint32_t kind) {
     const uint64_t mc = __ballot(kind == EMIT_CLOSEST);
-    const uint64_t ms = __ballot(kind == EMIT_SHADOW);
+    const uint64_t ms = __ballot(kind >= EMIT_SHADOW);
     const uint32_t lane = __lane_id();
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     const uint32_t stripe = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) % QSTRIPES;
@@ -159,7 +168,7 @@ __device__ __forceinline__ uint32_t append(const Queue& q, uint32_t kind) {
     bs = __shfl(bs, 0, 64);
     const uint32_t base = stripe * q.stripeCap;
     if (kind == EMIT_CLOSEST) return base + (bc + (uint32_t)__popcll(mc & lt)) % q.stripeCap;
-    if (kind == EMIT_SHADOW) return base + q.stripeCap - 1u - (bs + (uint32_t)__popcll(ms & lt)) % q.stripeCap;
+    if (kind >= EMIT_SHADOW) return base + q.stripeCap - 1u - (bs + (uint32_t)__popcll(ms & lt)) % q.stripeCap;
     return 0xFFFFFFFFu;
 }
 
@@ -278,24 +287,16 @@ struct Rd {
 // PrefixGen: TracePrefix (path_gen.h:74-250)
 // ======================================================================================
 
-static constexpr uint32_t PG_TRACE = 1, PG_NEE = 2;
-// The queued context of a walk (11 chunks, 176 bytes): the prefix record, the generator, the
-// state word, and the traced interaction and emitter colour of a pending NEE ray.  The rest of
-// PgState is rebuilt from the job's queued ray (pg_unpack): while a closest-hit ray is pending,
-// cur and dir are its origin and direction; while an NEE ray is pending, lightDir and dist are its
-// direction and tmax, and dir (the direction that reached the interaction) is the interaction's
-// stored incoming direction.
-static constexpr int PG_CHUNKS = 11;
+static constexpr uint32_t PG_TRACE = 1;
+// The queued context of a walk (9 chunks, 144 bytes): the prefix record, the generator and the
+// state word.  cur and dir are the origin and direction of the job's queued ray (pg_unpack).
+static constexpr int PG_CHUNKS = 9;
 
 struct PgState {
     Prefix pre;
     uint64_t rng;
     V3 cur, dir;
     uint32_t traceIdx, postRecon, state;
-    Packed it;            // traced interaction (normalised normal)
-    V3 lightDir;
-    float dist;
-    V3 color;
 };
 
 __device__ __forceinline__ Ctx<PG_CHUNKS> pg_pack(const PgState& s) {
@@ -304,7 +305,6 @@ __device__ __forceinline__ Ctx<PG_CHUNKS> pg_pack(const PgState& s) {
     w.u64(p.rng); w.u(p.flags); w.f(p.p); w.v(p.f); w.f(p.pathLen); w.v(p.postReconF); w.v(p.reconOutDir);
     w.pk(p.primary); w.pk(p.recon); w.pk(p.last);
     w.u64(s.rng); w.u(s.traceIdx | (s.postRecon << 8) | (s.state << 16));
-    w.pk(s.it); w.v(s.color);
     return w.ctx();
 }
 
@@ -320,17 +320,8 @@ __device__ __forceinline__ PgState pg_unpack(const Ctx<PG_CHUNKS>& c, float4 ra,
     s.traceIdx = m & 0xFFu;
     s.postRecon = (m >> 8) & 1u;
     s.state = m >> 16;
-    s.it = r.pk(); s.color = r.v();
     s.cur = V3{ra.x, ra.y, ra.z};
-    if (s.state == PG_NEE) {
-        s.dir = s.it.dir;
-        s.lightDir = V3{rb.x, rb.y, rb.z};
-        s.dist = rb.w;
-    } else {
-        s.dir = V3{rb.x, rb.y, rb.z};
-        s.lightDir = v3(0.0f);
-        s.dist = 0.0f;
-    }
+    s.dir = V3{rb.x, rb.y, rb.z};
     return s;
 }
 
@@ -345,9 +336,6 @@ __device__ __forceinline__ void pg_reset(PgState& s, uint64_t rng) {
     s.pre.recon = packed_invalid();
     s.pre.last = packed_invalid();
     s.pre.reconOutDir = v3(0.0f);
-    s.lightDir = v3(0.0f);
-    s.dist = 0.0f;
-    s.color = v3(0.0f);
 }
 
 // Start of TracePrefix with the camera ray: returns the first emission.
@@ -363,13 +351,41 @@ __device__ __forceinline__ Emit pg_start(const cx_launch_params& lp, PgState& s,
     s.dir = dir;
     s.traceIdx = 0;
     s.postRecon = 0;
-    s.it = packed_invalid();
     if (pg_max_len(lp) == 0) {   // loop body never runs: lastInt stays the default (invalid)
         s.pre.last = packed_invalid();
         return emit_none();
     }
     s.state = PG_TRACE;
     return emit_closest(origin, dir);
+}
+
+// The NEE vertex (path_gen.h:151-210): the record as it is if the light is visible.  A light with
+// no BSDF density towards it leaves the record invalid whatever its visibility, so no ray is
+// traced for it; an occluded final ray clears the record's valid flag, which is all that is read
+// of an invalid record.
+__device__ __forceinline__ Emit pg_nee(const DScene& S, PgState& s, const Inter& it, const EmitterSample& es) {
+    Prefix& pre = s.pre;
+    const V3 lightDir = normalize(es.pos - it.pos);
+    const float dist = length(es.pos - it.pos);
+    const BrdfEval be = ggx_eval(S, it, lightDir);
+    if (be.pdf <= 0.0f) {
+        pre.set_valid(false);
+        return emit_none();
+    }
+    if (!s.postRecon) {   // the re-trace of the same ray returns this same hit
+        pre.recon = it.pack();
+        pre.set_recon_idx(pre.length());
+        pre.reconOutDir = s.dir;
+        s.postRecon = 1;
+    }
+    const float distFactor = 1.0f / (dist * dist);
+    pre.f = pre.f * (be.brdf * es.color * distFactor);
+    if (s.postRecon) pre.postReconF = pre.postReconF * (be.brdf * es.color * distFactor);
+    if (pre.length() == 1) pre.f = pre.f + be.emission * distFactor;
+    pre.set_nee(true);
+    pre.set_valid(true);
+    pre.last = it.pack();
+    return emit_final(it.pos, lightDir, dist);
 }
 
 // After the closest hit of the current vertex (path_gen.h:100-247).
@@ -399,13 +415,8 @@ __device__ __forceinline__ Emit pg_on_hit(const DScene& S, const cx_launch_param
     if (rng.f() < lp.neeProb || forceNee) {
         pre.p *= lp.neeProb;
         const EmitterSample es = sample_emitter(S, rng);
-        s.lightDir = normalize(es.pos - it.pos);
-        s.dist = length(es.pos - it.pos);
-        s.color = es.color;
-        s.it = it.pack();
         s.rng = rng.s;
-        s.state = PG_NEE;
-        return emit_shadow(it.pos, s.lightDir, s.dist);
+        return pg_nee(S, s, it, es);
     }
     const BrdfSample bs = ggx_sample(S, it, rng);
     s.rng = rng.s;
@@ -436,52 +447,20 @@ __device__ __forceinline__ Emit pg_on_hit(const DScene& S, const cx_launch_param
     return emit_none();
 }
 
-// After the NEE shadow ray (path_gen.h:158-210).
-__device__ __forceinline__ Emit pg_on_shadow(const DScene& S, const cx_launch_params& lp, PgState& s, bool occluded) {
-    Prefix& pre = s.pre;
-    if (occluded) {
-        pre.set_valid(false);
-        return emit_none();
-    }
-    const Inter it = inter_restore(S, s.it, true);
-    if (!s.postRecon) {   // the re-trace of the same ray returns this same hit
-        pre.recon = s.it;
-        pre.set_recon_idx(pre.length());
-        pre.reconOutDir = s.dir;
-        s.postRecon = 1;
-    }
-    const BrdfEval be = ggx_eval(S, it, s.lightDir);
-    if (be.pdf <= 0.0f) {
-        pre.set_valid(false);
-        return emit_none();
-    }
-    const float distFactor = 1.0f / (s.dist * s.dist);
-    pre.f = pre.f * (be.brdf * s.color * distFactor);
-    if (s.postRecon) pre.postReconF = pre.postReconF * (be.brdf * s.color * distFactor);
-    if (pre.length() == 1) pre.f = pre.f + be.emission * distFactor;
-    pre.set_nee(true);
-    pre.set_valid(true);
-    pre.last = s.it;
-    return emit_none();
-}
-
 // ======================================================================================
 // SuffixGen: TraceSuffix (path_gen.h:252-387)
 // ======================================================================================
 
 static constexpr uint32_t SG_TRACE = 1, SG_NEE = 2, SG_RECON = 3;
-// The queued context of a suffix walk (10 chunks): the suffix record, the generator, the state
-// words and the emitter colour, then 6 words whose use depends on the pending ray: the NEE ray's
-// interaction (SG_NEE), or the BSDF value and the light distance (SG_RECON).  The rest of SgState
-// is rebuilt from the job's queued ray (sg_unpack): lastDir is a closest-hit ray's direction
-// (SG_TRACE), lightDir the NEE or reconnection ray's direction, lightLen the NEE ray's tmax.
-static constexpr int SG_CHUNKS = 10;
+// The queued context of a suffix walk (9 chunks): the suffix record, the generator, the state
+// words, the emitter colour, and the BSDF value and light distance of a sampled light.  lastDir is
+// a closest-hit ray's direction (SG_TRACE), lightDir the NEE or reconnection ray's direction.
+static constexpr int SG_CHUNKS = 9;
 
 struct SgState {
     Suffix suf;
     uint64_t rng;
-    uint32_t vertIdx, maxLen, prefixLen, postRecon, state, itTraced;
-    Packed it;
+    uint32_t vertIdx, maxLen, prefixLen, postRecon, state;
     V3 lastDir;
     V3 lightDir;
     float lightLen;
@@ -495,19 +474,14 @@ __device__ __forceinline__ Ctx<SG_CHUNKS> sg_pack(const SgState& s) {
     w.u64(u.rng); w.u(u.flags); w.f(u.p); w.v(u.f); w.v(u.postReconF); w.v(u.reconOutDir);
     w.pk(u.recon); w.pk(u.lastPrefix);
     w.u64(s.rng);
-    w.u(s.vertIdx | (s.maxLen << 8) | (s.prefixLen << 16) | (s.postRecon << 24) | (s.itTraced << 25));
+    w.u(s.vertIdx | (s.maxLen << 8) | (s.prefixLen << 16) | (s.postRecon << 24));
     w.u(s.state);
-    w.v(s.color);
-    if (s.state == SG_RECON) {
-        w.v(s.brdf); w.f(s.lightLen);
-    } else {
-        w.pk(s.it);
-    }
+    w.v(s.color); w.v(s.brdf); w.f(s.lightLen);
     return w.ctx();
 }
 
-// ra, rb: the job's queued ray {origin, tmin}, {direction, tmax}.
-__device__ __forceinline__ SgState sg_unpack(const Ctx<SG_CHUNKS>& c, float4 ra, float4 rb) {
+// rb: the job's queued ray's {direction, tmax}.
+__device__ __forceinline__ SgState sg_unpack(const Ctx<SG_CHUNKS>& c, float4 rb) {
     Rd<SG_CHUNKS> r(c);
     SgState s;
     Suffix& u = s.suf;
@@ -519,22 +493,21 @@ __device__ __forceinline__ SgState sg_unpack(const Ctx<SG_CHUNKS>& c, float4 ra,
     s.maxLen = (m >> 8) & 0xFFu;
     s.prefixLen = (m >> 16) & 0xFFu;
     s.postRecon = (m >> 24) & 1u;
-    s.itTraced = (m >> 25) & 1u;
     s.state = r.u();
-    s.color = r.v();
+    s.color = r.v(); s.brdf = r.v(); s.lightLen = r.f();
     const V3 d = V3{rb.x, rb.y, rb.z};
     s.lastDir = d;
     s.lightDir = d;
-    s.brdf = v3(0.0f);
-    s.lightLen = rb.w;
-    if (s.state == SG_RECON) {
-        s.brdf = r.v(); s.lightLen = r.f();
-        s.it = packed_invalid();
-    } else {
-        s.it = r.pk();
-    }
-    (void)ra;
     return s;
+}
+
+__device__ __forceinline__ void sg_finish(SgState& s) {
+    Suffix& suf = s.suf;
+    const float distFactor = 1.0f / (s.lightLen * s.lightLen);
+    suf.f = suf.f * (s.brdf * s.color * distFactor);
+    suf.postReconF = suf.postReconF * (s.color * distFactor);
+    if (suf.recon_idx() < suf.length()) suf.postReconF = suf.postReconF * s.brdf;
+    suf.set_valid(true);
 }
 
 // One vertex of the suffix loop once its interaction is known (path_gen.h:296-385).
@@ -553,7 +526,17 @@ __device__ __forceinline__ Emit sg_vertex(const DScene& S, const cx_launch_param
         s.lightDir = normalize(lightVec);
         if (any_bad(s.lightDir)) return emit_none();
         s.color = em.color;
-        s.it = it.pack();
+        // the BSDF towards the light before its visibility: without density the suffix stays
+        // invalid either way; a suffix that is reconnected already is stored as it is if the
+        // light is visible
+        const BrdfEval be = ggx_eval(S, it, s.lightDir);
+        if (be.pdf <= 0.0f) return emit_none();
+        suf.set_length(suf.length() + 1);
+        s.brdf = be.brdf;
+        if (s.postRecon) {
+            sg_finish(s);
+            return emit_final(it.pos, s.lightDir, s.lightLen);
+        }
         s.state = SG_NEE;
         return emit_shadow(it.pos, s.lightDir, s.lightLen);
     }
@@ -595,7 +578,6 @@ __device__ __forceinline__ Emit sg_start(const DScene& S, const cx_launch_params
     s.vertIdx = 0;
     s.lastDir = v3(0.0f);
     s.state = 0;
-    s.itTraced = 0;
     s.prefixLen = pre.length();
     if (!pre.valid() || pre.nee()) return emit_none();
     const uint32_t maxLen = (uint32_t)lp.maxPathLen - pre.length();
@@ -608,33 +590,16 @@ __device__ __forceinline__ Emit sg_start(const DScene& S, const cx_launch_params
 
 __device__ __forceinline__ Emit sg_on_hit(const DScene& S, const cx_launch_params& lp, SgState& s, const Inter& it,
                                           V3 rayOrigin) {
-    s.itTraced = 1;
     if (!it.valid) return emit_none();
     return sg_vertex(S, lp, s, it, rayOrigin);
 }
 
-__device__ __forceinline__ Emit sg_finish(SgState& s) {
-    Suffix& suf = s.suf;
-    const float distFactor = 1.0f / (s.lightLen * s.lightLen);
-    suf.f = suf.f * (s.brdf * s.color * distFactor);
-    suf.postReconF = suf.postReconF * (s.color * distFactor);
-    if (suf.recon_idx() < suf.length()) suf.postReconF = suf.postReconF * s.brdf;
-    suf.set_valid(true);
-    return emit_none();
-}
-
-__device__ __forceinline__ Emit sg_on_shadow(const DScene& S, SgState& s, bool occluded) {
+// After the shadow ray (origin o) of a light sampled before any reconnection vertex: the
+// reconnection ray along it (path_gen.h:318-335).
+__device__ __forceinline__ Emit sg_on_shadow(SgState& s, bool occluded, V3 o) {
     if (occluded) return emit_none();
-    const Inter it = inter_restore(S, s.it, s.itTraced != 0);
-    const BrdfEval be = ggx_eval(S, it, s.lightDir);
-    if (be.pdf <= 0.0f) return emit_none();
-    s.suf.set_length(s.suf.length() + 1);
-    s.brdf = be.brdf;
-    if (!s.postRecon) {
-        s.state = SG_RECON;
-        return emit_closest(it.pos, s.lightDir);
-    }
-    return sg_finish(s);
+    s.state = SG_RECON;
+    return emit_closest(o, s.lightDir);
 }
 
 __device__ __forceinline__ Emit sg_on_recon(SgState& s, const Inter& ri) {
@@ -643,30 +608,25 @@ __device__ __forceinline__ Emit sg_on_recon(SgState& s, const Inter& ri) {
     s.suf.set_recon_idx(s.suf.length());
     s.suf.reconOutDir = v3(0.0f);
     s.postRecon = 1;
-    return sg_finish(s);
+    sg_finish(s);
+    return emit_none();
 }
 
 // ======================================================================================
 // CompletePath: TraceCompletePath (path_gen.h:389-472)
 // ======================================================================================
 
-static constexpr uint32_t CP_TRACE = 1, CP_NEE = 2;
-static constexpr int CP_CHUNKS = 7;
+static constexpr int CP_CHUNKS = 2;   // the generator, the counters and the throughput
 
 struct CpState {
     uint64_t rng;
-    uint32_t traceIdx, depth, state;
-    V3 cur, dir, thr, radiance;
-    Packed it;
-    V3 lightDir;
-    float dist;
-    V3 color;
+    uint32_t traceIdx, depth;
+    V3 thr, radiance;
 };
 
 __device__ __forceinline__ Ctx<CP_CHUNKS> cp_pack(const CpState& s) {
     Wr<CP_CHUNKS> w;
-    w.u64(s.rng); w.u(s.traceIdx | (s.depth << 8) | (s.state << 16));
-    w.v(s.cur); w.v(s.dir); w.v(s.thr); w.pk(s.it); w.v(s.lightDir); w.f(s.dist); w.v(s.color);
+    w.u64(s.rng); w.u(s.traceIdx | (s.depth << 8)); w.v(s.thr);
     return w.ctx();
 }
 
@@ -677,26 +637,18 @@ __device__ __forceinline__ CpState cp_unpack(const Ctx<CP_CHUNKS>& c) {
     const uint32_t m = r.u();
     s.traceIdx = m & 0xFFu;
     s.depth = (m >> 8) & 0xFFu;
-    s.state = m >> 16;
-    s.cur = r.v(); s.dir = r.v(); s.thr = r.v(); s.it = r.pk(); s.lightDir = r.v(); s.dist = r.f(); s.color = r.v();
+    s.thr = r.v();
     s.radiance = v3(0.0f);
     return s;
 }
 
 // The state of a complete path before its first trace.
-__device__ __forceinline__ void cp_reset(CpState& s, uint64_t rng, V3 origin, V3 dir) {
+__device__ __forceinline__ void cp_reset(CpState& s, uint64_t rng) {
     s.rng = rng;
     s.traceIdx = 0;
     s.depth = 0;
-    s.state = CP_TRACE;
-    s.cur = origin;
-    s.dir = dir;
     s.thr = v3(1.0f);
     s.radiance = v3(0.0f);
-    s.it = packed_invalid();
-    s.lightDir = v3(0.0f);
-    s.dist = 0.0f;
-    s.color = v3(0.0f);
 }
 
 // ---- fresh contexts: a walk before its first trace is a function of its generator state and
@@ -730,9 +682,7 @@ __device__ __forceinline__ CpState cp_load(const Queue& q, uint32_t slot) {
     const uint4 c0 = q.ctx[slot];
     CpState s;
     if (c0.z & CTX_FRESH) {
-        V3 o, d;
-        get_ray(q, slot, o, d);
-        cp_reset(s, (uint64_t)c0.x | ((uint64_t)c0.y << 32), o, d);
+        cp_reset(s, (uint64_t)c0.x | ((uint64_t)c0.y << 32));
         return s;
     }
     Ctx<CP_CHUNKS> c;
@@ -742,7 +692,8 @@ __device__ __forceinline__ CpState cp_load(const Queue& q, uint32_t slot) {
     return cp_unpack(c);
 }
 
-// Returns an emission; when none, `done` holds the radiance in s.radiance.
+// Returns an emission; when none or a final shadow ray, s.radiance holds the path's radiance (0 if
+// the final ray is occluded).
 __device__ __forceinline__ Emit cp_on_hit(const DScene& S, const cx_launch_params& lp, CpState& s, const Inter& it) {
     if (!it.valid) {
         s.radiance = v3(0.0f);
@@ -755,12 +706,17 @@ __device__ __forceinline__ Emit cp_on_hit(const DScene& S, const cx_launch_param
         s.thr = s.thr / lp.neeProb;
         const EmitterSample es = sample_emitter(S, rng);
         s.rng = rng.s;
-        s.lightDir = normalize(es.pos - it.pos);
-        s.dist = length(es.pos - it.pos);
-        s.color = es.color;
-        s.it = it.pack();
-        s.state = CP_NEE;
-        return emit_shadow(it.pos, s.lightDir, s.dist);
+        // the radiance if the light is visible (path_gen.h:430-455); an occluded light gives 0, so
+        // a radiance of 0 needs no ray
+        const V3 lightDir = normalize(es.pos - it.pos);
+        const float dist = length(es.pos - it.pos);
+        const BrdfEval be = ggx_eval(S, it, lightDir);
+        const float distFactor = 1.0f / (dist * dist);
+        s.radiance = s.thr * be.brdf * es.color * distFactor;
+        if (s.depth == 1) s.radiance = s.radiance + be.emission;
+        if (any_bad(s.radiance)) s.radiance = v3(0.0f);
+        if (is_zero(s.radiance)) return emit_none();
+        return emit_final(it.pos, lightDir, dist);
     }
     const BrdfSample bs = ggx_sample(S, it, rng);
     s.rng = rng.s;
@@ -768,29 +724,11 @@ __device__ __forceinline__ Emit cp_on_hit(const DScene& S, const cx_launch_param
         s.radiance = v3(0.0f);
         return emit_none();
     }
-    s.cur = it.pos;
-    s.dir = bs.outDir;
     s.thr = s.thr * (bs.brdf / bs.pdf);
     s.thr = s.thr / (1.0f - lp.neeProb);
     s.traceIdx++;
-    if (s.traceIdx < (uint32_t)lp.maxPathLen) {
-        s.state = CP_TRACE;
-        return emit_closest(s.cur, s.dir);
-    }
+    if (s.traceIdx < (uint32_t)lp.maxPathLen) return emit_closest(it.pos, bs.outDir);
     s.radiance = v3(0.0f);
-    return emit_none();
-}
-
-__device__ __forceinline__ Emit cp_on_shadow(const DScene& S, CpState& s, bool occluded) {
-    if (occluded) {
-        s.radiance = v3(0.0f);
-        return emit_none();
-    }
-    const Inter it = inter_restore(S, s.it, true);
-    const BrdfEval be = ggx_eval(S, it, s.lightDir);
-    const float distFactor = 1.0f / (s.dist * s.dist);
-    s.radiance = s.thr * be.brdf * s.color * distFactor;
-    if (s.depth == 1) s.radiance = s.radiance + be.emission;
     return emit_none();
 }
 
@@ -867,6 +805,20 @@ __device__ __forceinline__ Inter load_suffix_dst(const DScene& S, const RecordSe
     return rehydrate(S, load_suffix_ref(R, ref).lastPrefix);
 }
 
+// What the answer to a final shadow ray does (final_answer), per machine.
+static constexpr uint32_t FINAL_NONE = 0, FINAL_SHIFT = 1, FINAL_PREFIX = 2, FINAL_SUFFIX = 3, FINAL_PATH = 4;
+
+struct FinalArgs {
+    uint32_t mode;
+    uint32_t accum;           // FINAL_PATH: blend into the output (enableAccum)
+    float4* shiftRes;         // FINAL_SHIFT
+    uint4* records;           // FINAL_PREFIX, FINAL_SUFFIX: first chunk of the canonical records
+    const float4* radiance;   // FINAL_PATH: radiance if visible, per pixel
+    float* out;
+    uint64_t frameIdx;
+    const FrameDyn* dyn;      // frame index of a graph replay, or null
+};
+
 // Everything a wavefront kernel reads or writes.  qin is the queue whose rays were just
 // answered, qout the queue the kernel appends to; both share one allocation per side and are
 // viewed with the capacity and chunk count of the machine in flight.
@@ -902,21 +854,27 @@ struct WaveArgs {
     uint32_t gIdx;          // final-gather prefix index (0 = canonical)
 };
 
-static constexpr uint32_t SH_TRACE = 1, SH_SHADOW = 2;
-static constexpr int SH_CHUNKS = 4;
+// The queued context of a shift that replays vertices (2 chunks): its source, the replay's
+// position and generator and the throughput.  Only closest-hit rays have one.
+static constexpr int SH_CHUNKS = 2;
 
 struct ShState {
-    uint32_t srcRef, isSuffix, idx, count, state, currTraced;
+    uint32_t srcRef, isSuffix, idx, count;
     uint64_t srng;
     V3 thr;
-    Packed curr;
+};
+
+// A shift's result: the shifted integrand and the Jacobian.
+struct ShiftOut {
+    V3 f;
+    float J;
 };
 
 __device__ __forceinline__ Ctx<SH_CHUNKS> sh_pack(const ShState& s) {
     Wr<SH_CHUNKS> w;
     w.u(s.srcRef);
-    w.u(s.idx | (s.count << 8) | (s.state << 16) | (s.isSuffix << 24) | (s.currTraced << 25));
-    w.u64(s.srng); w.v(s.thr); w.pk(s.curr);
+    w.u(s.idx | (s.count << 8) | (s.isSuffix << 16));
+    w.u64(s.srng); w.v(s.thr);
     return w.ctx();
 }
 
@@ -927,15 +885,59 @@ __device__ __forceinline__ ShState sh_unpack(const Ctx<SH_CHUNKS>& c) {
     const uint32_t m = r.u();
     s.idx = m & 0xFFu;
     s.count = (m >> 8) & 0xFFu;
-    s.state = (m >> 16) & 0xFFu;
-    s.isSuffix = (m >> 24) & 1u;
-    s.currTraced = (m >> 25) & 1u;
-    s.srng = r.u64(); s.thr = r.v(); s.curr = r.pk();
+    s.isSuffix = (m >> 16) & 1u;
+    s.srng = r.u64(); s.thr = r.v();
     return s;
 }
 
-// Replay step or reconnection ray, from the current interaction.
-__device__ __forceinline__ Emit sh_continue(const DScene& S, const RecordSet& R, ShState& s, const Inter& curr) {
+// The end of a shift once the vertex before the reconnection is known: BSDFs at both ends of the
+// reconnection and the Jacobian, as they are if the reconnection is visible (prefix_reuse.h:66-99,
+// suffix_reuse.h:76-108).  (0, 0) where no ray could make them anything else.
+__device__ __forceinline__ ShiftOut sh_reconnect(const DScene& S, const ShState& s, const Prefix& src, Inter srcRecon,
+                                                 const Inter& curr, V3 reconDir) {
+    const ShiftOut none{v3(0.0f), 0.0f};
+    V3 thr = s.thr;
+    const Inter srcPrimary = rehydrate(S, src.primary);
+    const BrdfEval b1 = ggx_eval(S, curr, reconDir);
+    if (b1.pdf <= 0.0f) return none;
+    thr = thr * b1.brdf;
+    srcRecon.dir = reconDir;
+    const BrdfEval b2 = ggx_eval(S, srcRecon, src.reconOutDir);
+    if (b2.pdf <= 0.0f) return none;
+    thr = thr * b2.brdf;
+    const V3 ff = thr * src.postReconF;
+    return ShiftOut{V3{gmax(0.0f, ff.x), gmax(0.0f, ff.y), gmax(0.0f, ff.z)},
+                    recon_jacobian(srcPrimary.pos, curr.pos, srcRecon.pos, srcRecon.nrm)};
+}
+
+__device__ __forceinline__ ShiftOut sh_reconnect(const DScene& S, const ShState& s, const Suffix& src, Inter srcRecon,
+                                                 const Inter& curr, V3 reconDir) {
+    const ShiftOut none{v3(0.0f), 0.0f};
+    V3 thr = s.thr;
+    const Inter srcLast = rehydrate(S, src.lastPrefix);
+    const BrdfEval b1 = ggx_eval(S, curr, reconDir);
+    if (b1.pdf <= 0.0f) return none;
+    thr = thr * b1.brdf;
+    if (src.recon_idx() < src.length()) {
+        srcRecon.dir = reconDir;
+        if (is_zero(src.reconOutDir)) return none;
+        const BrdfEval b2 = ggx_eval(S, srcRecon, src.reconOutDir);
+        if (b2.pdf <= 0.0f) return none;
+        thr = thr * b2.brdf;
+    }
+    return ShiftOut{thr * src.postReconF, recon_jacobian(srcLast.pos, curr.pos, srcRecon.pos, srcRecon.nrm)};
+}
+
+// Replay step or reconnection ray, from the current interaction.  The reconnection is evaluated
+// before its ray is traced: `out` is the shift's result if the (final) ray is unoccluded.  A shift
+// whose integrand is 0 in every channel is finished as (0, 0) without a ray, for every use of a
+// result multiplies its luminance by the (finite) Jacobian: a third of the reconnections point
+// below one of the two surfaces, and those between two points of one plane run along it, the
+// slowest rays of all, which pass every triangle on their way.
+template <typename R>
+__device__ __forceinline__ Emit sh_continue(const DScene& S, ShState& s, const R& src, const Inter& curr,
+                                            ShiftOut& out) {
+    out = ShiftOut{v3(0.0f), 0.0f};
     if (s.idx < s.count) {
         Rng srng;
         srng.s = s.srng;
@@ -944,37 +946,31 @@ __device__ __forceinline__ Emit sh_continue(const DScene& S, const RecordSet& R,
         s.srng = srng.s;
         if (bs.pdf <= 0.0f) return emit_none();
         s.thr = s.thr * bs.brdf;
-        s.curr = curr.pack();
-        s.state = SH_TRACE;
         return emit_closest(curr.pos, bs.outDir);
     }
-    // an if, not ?: over the two records: the conditional operator on whole records made the
-    // compiler load both into private memory and read the field back from there
-    Packed reconP;
-    if (s.isSuffix) reconP = load_suffix_ref(R, s.srcRef).recon;
-    else reconP = load_prefix_ref(R, s.srcRef).recon;
-    const Inter srcRecon = rehydrate(S, reconP);
+    const Inter srcRecon = rehydrate(S, src.recon);
     const V3 reconVec = srcRecon.pos - curr.pos;
     const float reconLen = length(reconVec);
     const V3 reconDir = normalize(reconVec);
     if (!s.isSuffix && isinf(reconLen)) return emit_none();
     if (any_bad(reconDir)) return emit_none();
-    s.curr = curr.pack();
-    s.state = SH_SHADOW;
-    return emit_shadow(curr.pos, reconDir, reconLen);
+    out = sh_reconnect(S, s, src, srcRecon, curr, reconDir);
+    if (is_zero(out.f)) {
+        out = ShiftOut{v3(0.0f), 0.0f};
+        return emit_none();
+    }
+    return emit_final(curr.pos, reconDir, reconLen);
 }
 
-// Start of a shift: returns the first emission (none = finished with f = 0, J = 0).
+// Start of a shift: returns the first emission (none = finished with `out`).
 __device__ __forceinline__ Emit sh_start_prefix(const DScene& S, const RecordSet& R, ShState& s, uint32_t srcRef,
-                                                uint32_t dstRef) {
+                                                uint32_t dstRef, ShiftOut& out) {
+    out = ShiftOut{v3(0.0f), 0.0f};
     s.srcRef = srcRef;
     s.isSuffix = 0;
     s.idx = 0;
     s.count = 0;
-    s.state = 0;
-    s.currTraced = 0;
     s.thr = v3(1.0f);
-    s.curr = packed_invalid();
     const Prefix src = load_prefix_ref(R, srcRef);
     s.srng = src.rng;
     if (!src.valid() || src.recon_idx() < 2) return emit_none();
@@ -984,19 +980,17 @@ __device__ __forceinline__ Emit sh_start_prefix(const DScene& S, const RecordSet
     if (!rehydrate(S, src.recon).valid) return emit_none();
     const int rvc = (int)(src.recon_idx() - 2u);
     s.count = rvc > 0 ? (uint32_t)rvc : 0u;
-    return sh_continue(S, R, s, curr);
+    return sh_continue(S, s, src, curr, out);
 }
 
 __device__ __forceinline__ Emit sh_start_suffix(const DScene& S, const RecordSet& R, ShState& s, uint32_t srcRef,
-                                                uint32_t dstRef) {
+                                                uint32_t dstRef, ShiftOut& out) {
+    out = ShiftOut{v3(0.0f), 0.0f};
     s.srcRef = srcRef;
     s.isSuffix = 1;
     s.idx = 0;
     s.count = 0;
-    s.state = 0;
-    s.currTraced = (dstRef >> 28) == REF_PACKED_TRACED ? 1u : 0u;
     s.thr = v3(1.0f);
-    s.curr = packed_invalid();
     const Inter dst = load_suffix_dst(S, R, dstRef);
     const Suffix src = load_suffix_ref(R, srcRef);
     s.srng = src.rng;
@@ -1006,57 +1000,18 @@ __device__ __forceinline__ Emit sh_start_suffix(const DScene& S, const RecordSet
     if (!rehydrate(S, src.recon).valid) return emit_none();
     const int rvc = (int)(src.recon_idx() - 1u);
     s.count = rvc > 0 ? (uint32_t)rvc : 0u;
-    return sh_continue(S, R, s, dst);
+    return sh_continue(S, s, src, dst, out);
 }
 
-__device__ __forceinline__ Emit sh_on_hit(const DScene& S, const RecordSet& R, ShState& s, const Inter& it) {
+__device__ __forceinline__ Emit sh_on_hit(const DScene& S, const RecordSet& R, ShState& s, const Inter& it,
+                                          ShiftOut& out) {
+    out = ShiftOut{v3(0.0f), 0.0f};
     if (!it.valid) return emit_none();
-    s.currTraced = 1;
     s.idx++;
-    return sh_continue(S, R, s, it);
-}
-
-// Final step: BSDFs at both ends of the reconnection and the Jacobian.  Writes f and J.
-__device__ __forceinline__ void sh_on_shadow(const DScene& S, const RecordSet& R, const ShState& s, bool occluded,
-                                             V3& f, float& J) {
-    f = v3(0.0f);
-    J = 0.0f;
-    if (occluded) return;
-    const Inter curr = inter_restore(S, s.curr, s.currTraced != 0);
-    V3 thr = s.thr;
-    if (!s.isSuffix) {
-        const Prefix src = load_prefix_ref(R, s.srcRef);
-        const Inter srcPrimary = rehydrate(S, src.primary);
-        Inter srcRecon = rehydrate(S, src.recon);
-        const V3 reconDir = normalize(srcRecon.pos - curr.pos);
-        const BrdfEval b1 = ggx_eval(S, curr, reconDir);
-        if (b1.pdf <= 0.0f) return;
-        thr = thr * b1.brdf;
-        srcRecon.dir = reconDir;
-        const BrdfEval b2 = ggx_eval(S, srcRecon, src.reconOutDir);
-        if (b2.pdf <= 0.0f) return;
-        thr = thr * b2.brdf;
-        J = recon_jacobian(srcPrimary.pos, curr.pos, srcRecon.pos, srcRecon.nrm);
-        const V3 ff = thr * src.postReconF;
-        f = V3{gmax(0.0f, ff.x), gmax(0.0f, ff.y), gmax(0.0f, ff.z)};
-        return;
-    }
-    const Suffix src = load_suffix_ref(R, s.srcRef);
-    const Inter srcLast = rehydrate(S, src.lastPrefix);
-    Inter srcRecon = rehydrate(S, src.recon);
-    const V3 reconDir = normalize(srcRecon.pos - curr.pos);
-    const BrdfEval b1 = ggx_eval(S, curr, reconDir);
-    if (b1.pdf <= 0.0f) return;
-    thr = thr * b1.brdf;
-    if (src.recon_idx() < src.length()) {
-        srcRecon.dir = reconDir;
-        if (is_zero(src.reconOutDir)) return;
-        const BrdfEval b2 = ggx_eval(S, srcRecon, src.reconOutDir);
-        if (b2.pdf <= 0.0f) return;
-        thr = thr * b2.brdf;
-    }
-    J = recon_jacobian(srcLast.pos, curr.pos, srcRecon.pos, srcRecon.nrm);
-    f = thr * src.postReconF;
+    // an if, not ?: over the two records: the conditional operator on whole records made the
+    // compiler load both into private memory and read the fields back from there
+    if (s.isSuffix) return sh_continue(S, s, load_suffix_ref(R, s.srcRef), it, out);
+    return sh_continue(S, s, load_prefix_ref(R, s.srcRef), it, out);
 }
 
 }  // namespace cx

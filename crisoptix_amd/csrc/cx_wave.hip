@@ -22,6 +22,45 @@ static constexpr int SHORT_STACK = 16;
 
 __device__ __forceinline__ uint32_t gid() { return blockIdx.x * blockDim.x + threadIdx.x; }
 
+// ---- final shadow rays ----
+
+__device__ __forceinline__ void write_radiance(float* out, bool accum, uint64_t frameIdx, uint32_t p, V3 rad) {
+    float* o = out + 3 * (size_t)p;
+    V3 r = rad;
+    if (accum) {
+        const V3 old = V3{o[0], o[1], o[2]};
+        const float blend = 1.0f / (float)(frameIdx + 1);
+        r = blend * rad + (1.0f - blend) * old;
+    }
+    o[0] = r.x;
+    o[1] = r.y;
+    o[2] = r.z;
+}
+
+// The answer to a shadow ray of job `job`, if it is a final one (false: the job's next step reads
+// the answer): the job's stored result stands if the ray is unoccluded and is taken back if not.
+__device__ __forceinline__ bool final_answer(const FinalArgs& F, uint32_t job, bool occluded) {
+    switch (F.mode) {
+        case FINAL_SHIFT:
+            if (occluded) F.shiftRes[job] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+            return true;
+        case FINAL_SUFFIX:
+            if (!(job & JOB_FINAL)) return false;
+            [[fallthrough]];
+        case FINAL_PREFIX:
+            // the valid flag of the canonical record (word 2 of its first chunk)
+            if (occluded) ((uint32_t*)(F.records + (job & ~JOB_FINAL)))[2] &= ~(1u << 16);
+            return true;
+        case FINAL_PATH: {
+            const float4 r = F.radiance[job];
+            write_radiance(F.out, F.accum != 0, F.dyn ? F.dyn->frameIdx : F.frameIdx, job,
+                           occluded ? v3(0.0f) : V3{r.x, r.y, r.z});
+            return true;
+        }
+        default: return false;
+    }
+}
+
 // ---- traversal of a queue ----
 
 // The rays of wavefront w among `waves`, out of the n rays [base, base + n) of qin's index space:
@@ -83,7 +122,7 @@ __device__ __forceinline__ uint32_t chunk_ray(const ChunkRange& c, uint32_t v, u
 template <int WIDTH, typename Stack>
 __device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, const QIndex& qi, uint32_t nc,
                                              uint32_t ns, uint32_t w, uint32_t waves, uint32_t minChunk,
-                                             Stack& st) {
+                                             const FinalArgs& F, Stack& st) {
     const ChunkRange cc = chunk_range(0u, nc, w, waves, minChunk), cs = chunk_range(nc, ns, w, waves, minChunk);
     const uint32_t cnt = cc.cnt + cs.cnt;
     const uint64_t below = (1ull << (threadIdx.x & 63)) - 1ull;
@@ -117,8 +156,9 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, 
         if (trav_step_rt<WIDTH>(S, r, st, any)) {
             const Hit& h = r.best;
             const bool hit = h.prim != INVALID_PRIM;
-            qin.res[slot] = any ? uint4{hit ? 1u : 0u, 0u, 0u, 0u}
-                                : uint4{h.prim, fb(hit ? h.t : 0.0f), fb(hit ? h.u : 0.0f), fb(hit ? h.v : 0.0f)};
+            if (!any || !final_answer(F, qin.job[slot], hit))
+                qin.res[slot] = any ? uint4{hit ? 1u : 0u, 0u, 0u, 0u}
+                                    : uint4{h.prim, fb(hit ? h.t : 0.0f), fb(hit ? h.u : 0.0f), fb(hit ? h.v : 0.0f)};
             has = false;
         }
     }
@@ -138,7 +178,7 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, 
 // least 5.
 template <int WIDTH>
 __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH == 8 ? 1 : (WIDTH == 4 ? 7 : 5), 8))) void k_q_trace(
-    DScene S, Queue qin, Queue qout, unsigned long long* counters, uint32_t minChunk) {
+    DScene S, Queue qin, Queue qout, unsigned long long* counters, uint32_t minChunk, FinalArgs F) {
     __shared__ int s_st[SHORT_STACK * WBLOCK];
     __shared__ QIndex qi;
     qindex_load(qin, qi);
@@ -154,22 +194,26 @@ __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH ==
     int ovf[STACK_OVF<SHORT_STACK>];
     TravStack<SHORT_STACK, WBLOCK> st{s_st + threadIdx.x, ovf};
     const uint32_t waves = gridDim.x * (WBLOCK / 64), w = blockIdx.x * (WBLOCK / 64) + (threadIdx.x >> 6);
-    trace_chunks<WIDTH>(S, qin, qi, nc, ns, w, waves, minChunk, st);
+    trace_chunks<WIDTH>(S, qin, qi, nc, ns, w, waves, minChunk, F, st);
 }
 
 // Grid-stride loop over the jobs of qin whose bound is uniform per block, so every lane of a
-// wavefront reaches each wave-aggregated append.
-#define CX_FOR_JOBS(W)                                                         \
+// wavefront reaches each wave-aggregated append.  A machine whose shadow rays are all final has
+// nothing to step for them: `shadows` false leaves them out.
+#define CX_FOR_JOBS(W, shadows)                                                \
     __shared__ QIndex _qi;                                                    \
     qindex_load((W).qin, _qi);                                                \
     const uint32_t _nc = _qi.pc[QSTRIPES], _ns = _qi.ps[QSTRIPES];            \
-    const uint32_t _n = _nc + _ns;                                            \
+    const uint32_t _n = _nc + ((shadows) ? _ns : 0u);                         \
     for (uint32_t _base = blockIdx.x * WBLOCK; _base < _n; _base += gridDim.x * WBLOCK)
 
 __device__ __forceinline__ void emit_job(const Queue& q, uint32_t slot, uint32_t job, const Emit& e) {
     q.job[slot] = job;
     put_ray(q, slot, e);
 }
+
+// A context is stored for the rays that a later step answers, not for final ones.
+__device__ __forceinline__ bool keeps_context(uint32_t kind) { return kind == EMIT_CLOSEST || kind == EMIT_SHADOW; }
 
 __device__ __forceinline__ uint64_t gbuf_rng(const uint4& g) { return (uint64_t)g.x | ((uint64_t)g.y << 32); }
 
@@ -191,19 +235,15 @@ __device__ __forceinline__ void pg_finish(const WaveArgs& W, uint32_t p, const P
     W.rngScratch[p] = s.rng;
 }
 
-__device__ __forceinline__ void cp_finish(const WaveArgs& W, uint32_t p, const CpState& s) {
-    V3 rad = s.radiance;
-    if (any_bad(rad)) rad = v3(0.0f);
-    float* o = W.A.out + 3 * (size_t)p;
-    V3 r = rad;
-    if (W.A.lp.enableAccum) {
-        const V3 old = V3{o[0], o[1], o[2]};
-        const float blend = 1.0f / (float)(frame_index(W.A) + 1);
-        r = blend * rad + (1.0f - blend) * old;
-    }
-    o[0] = r.x;
-    o[1] = r.y;
-    o[2] = r.z;
+__device__ __forceinline__ void write_out(const FrameArgs& A, uint32_t p, V3 rad) {
+    write_radiance(A.out, A.lp.enableAccum != 0, frame_index(A), p, rad);
+}
+
+// A path without a further ray is written at once; one with a final shadow ray leaves its
+// radiance for the ray's answer.
+__device__ __forceinline__ void cp_finish(const WaveArgs& W, uint32_t p, const CpState& s, uint32_t kind) {
+    if (kind == EMIT_FINAL) W.radScratch[p] = float4{s.radiance.x, s.radiance.y, s.radiance.z, 0.0f};
+    else if (kind == EMIT_NONE) write_out(W.A, p, any_bad(s.radiance) ? v3(0.0f) : s.radiance);
 }
 
 // Camera ray, then the first ray of TracePrefix (ReSTIR modes) or TraceCompletePath.
@@ -233,9 +273,9 @@ __global__ __launch_bounds__(WBLOCK) void k_w_prefix_init(WaveArgs W) {
             e = pg_start(A.lp, pg, origin, dir);
             if (e.kind == EMIT_NONE) pg_finish(W, p, pg);
         } else {
-            cp_reset(cp, rng.s, origin, dir);
+            cp_reset(cp, rng.s);
             if (A.lp.maxPathLen > 0) e = emit_closest(origin, dir);
-            else cp_finish(W, p, cp);
+            else cp_finish(W, p, cp, EMIT_NONE);
         }
     }
     const uint32_t slot = append(W.qout, e.kind);
@@ -249,14 +289,13 @@ __global__ __launch_bounds__(WBLOCK) void k_w_prefix_init(WaveArgs W) {
 // reference's logic up to the job's next trace call or its end, where it stores the result.
 // Shared by the step kernels and the tail kernel.
 __device__ __forceinline__ Emit pg_advance(const WaveArgs& W, uint32_t job, PgState& s, uint4 r, V3 o, V3 d) {
-    const Emit e = s.state == PG_TRACE ? pg_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d))
-                                       : pg_on_shadow(W.A.S, W.A.lp, s, r.x != 0);
-    if (e.kind == EMIT_NONE) pg_finish(W, job, s);
+    const Emit e = pg_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d));
+    if (e.kind != EMIT_CLOSEST) pg_finish(W, job, s);
     return e;
 }
 
 __global__ __launch_bounds__(WBLOCK) void k_w_pg_step(WaveArgs W) {
-    CX_FOR_JOBS(W) {
+    CX_FOR_JOBS(W, false) {
     const uint32_t i = _base + threadIdx.x;
     const bool active = i < _n;
     Emit e = emit_none();
@@ -272,21 +311,20 @@ __global__ __launch_bounds__(WBLOCK) void k_w_pg_step(WaveArgs W) {
     }
     const uint32_t slot = append(W.qout, e.kind);
     if (active && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, pg_pack(s));
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, pg_pack(s));
         emit_job(W.qout, slot, job, e);
     }
     }
 }
 
 __device__ __forceinline__ Emit cp_advance(const WaveArgs& W, uint32_t job, CpState& s, uint4 r, V3 o, V3 d) {
-    const Emit e = s.state == CP_TRACE ? cp_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d))
-                                       : cp_on_shadow(W.A.S, s, r.x != 0);
-    if (e.kind == EMIT_NONE) cp_finish(W, job, s);
+    const Emit e = cp_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d));
+    cp_finish(W, job, s, e.kind);
     return e;
 }
 
 __global__ __launch_bounds__(WBLOCK) void k_w_cp_step(WaveArgs W) {
-    CX_FOR_JOBS(W) {
+    CX_FOR_JOBS(W, false) {
     const uint32_t i = _base + threadIdx.x;
     const bool active = i < _n;
     Emit e = emit_none();
@@ -302,7 +340,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_cp_step(WaveArgs W) {
     }
     const uint32_t slot = append(W.qout, e.kind);
     if (active && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, cp_pack(s));
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, cp_pack(s));
         emit_job(W.qout, slot, job, e);
     }
     }
@@ -316,8 +354,8 @@ __device__ __forceinline__ bool prefix_temporal(const WaveArgs& W, uint32_t p, c
     return !(prev.wSum <= 0.0f || !prev.s.valid() || skipNee);
 }
 
-__device__ __forceinline__ void shift_finish(const WaveArgs& W, uint32_t job, V3 f, float J) {
-    W.shiftRes[job] = float4{f.x, f.y, f.z, J};
+__device__ __forceinline__ void shift_finish(const WaveArgs& W, uint32_t job, const ShiftOut& r) {
+    W.shiftRes[job] = float4{r.f.x, r.f.y, r.f.z, r.J};
 }
 
 // Both temporal shifts of a pixel (prefix_gen_temp_reuse.cu:58-61).
@@ -333,35 +371,30 @@ __global__ __launch_bounds__(WBLOCK) void k_w_prefix_temporal_setup(WaveArgs W) 
     for (uint32_t d = 0; d < 2; d++) {
         Emit e = emit_none();
         ShState s;
+        ShiftOut out;
         const uint32_t job = 2 * p + d;
         if (temporal) {
             const uint32_t back = make_ref(REF_PREFIX_BACK, p), canon = make_ref(REF_PREFIX_SCRATCH, p);
-            e = d == 0 ? sh_start_prefix(W.A.S, W.R, s, back, canon) : sh_start_prefix(W.A.S, W.R, s, canon, back);
-            if (e.kind == EMIT_NONE) shift_finish(W, job, v3(0.0f), 0.0f);
+            e = d == 0 ? sh_start_prefix(W.A.S, W.R, s, back, canon, out) : sh_start_prefix(W.A.S, W.R, s, canon, back, out);
+            if (e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
         }
         const uint32_t slot = append(W.qout, e.kind);
         if (temporal && e.kind != EMIT_NONE) {
-            store_ctx(W.qout, slot, sh_pack(s));
+            if (keeps_context(e.kind)) store_ctx(W.qout, slot, sh_pack(s));
             emit_job(W.qout, slot, job, e);
         }
     }
 }
 
 __device__ __forceinline__ Emit sh_advance(const WaveArgs& W, uint32_t job, ShState& s, uint4 r, V3 o, V3 d) {
-    if (s.state == SH_TRACE) {
-        const Emit e = sh_on_hit(W.A.S, W.R, s, inter_from_hit(W.A.S, r, d));
-        if (e.kind == EMIT_NONE) shift_finish(W, job, v3(0.0f), 0.0f);
-        return e;
-    }
-    V3 f;
-    float J;
-    sh_on_shadow(W.A.S, W.R, s, r.x != 0, f, J);
-    shift_finish(W, job, f, J);
-    return emit_none();
+    ShiftOut out;
+    const Emit e = sh_on_hit(W.A.S, W.R, s, inter_from_hit(W.A.S, r, d), out);
+    if (e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
+    return e;
 }
 
 __global__ __launch_bounds__(WBLOCK) void k_w_sh_step(WaveArgs W) {
-    CX_FOR_JOBS(W) {
+    CX_FOR_JOBS(W, false) {
     const uint32_t i = _base + threadIdx.x;
     const bool active = i < _n;
     Emit e = emit_none();
@@ -377,23 +410,10 @@ __global__ __launch_bounds__(WBLOCK) void k_w_sh_step(WaveArgs W) {
     }
     const uint32_t slot = append(W.qout, e.kind);
     if (active && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, sh_pack(s));
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, sh_pack(s));
         emit_job(W.qout, slot, job, e);
     }
     }
-}
-
-__device__ __forceinline__ void write_out(const FrameArgs& A, uint32_t p, V3 rad) {
-    float* o = A.out + 3 * (size_t)p;
-    V3 r = rad;
-    if (A.lp.enableAccum) {
-        const V3 old = V3{o[0], o[1], o[2]};
-        const float blend = 1.0f / (float)(frame_index(A) + 1);
-        r = blend * rad + (1.0f - blend) * old;
-    }
-    o[0] = r.x;
-    o[1] = r.y;
-    o[2] = r.z;
 }
 
 // Reservoir updates of PrefixGenTempReuse and the raygen epilogue (prefix_gen_temp_reuse.cu:24-172).
@@ -511,22 +531,23 @@ __global__ __launch_bounds__(WBLOCK) void k_w_spatial_setup(WaveArgs W) {
         for (uint32_t d = 0; d < 2; d++) {
             Emit e = emit_none();
             ShState s;
+            ShiftOut out;
             const uint32_t job = ((uint32_t)p * S + i) * 2 + d;
             const bool want = ok && ((validFlags >> i) & 1u);
             if (want) {
                 const uint32_t np = W.nbr[(size_t)p * S + i];
                 if (!SUFFIX) {
                     const uint32_t neigh = make_ref(REF_PREFIX_BACK, np), curr = make_ref(REF_PREFIX_FRONT, p);
-                    e = d == 0 ? sh_start_prefix(A.S, W.R, s, neigh, curr) : sh_start_prefix(A.S, W.R, s, curr, neigh);
+                    e = d == 0 ? sh_start_prefix(A.S, W.R, s, neigh, curr, out) : sh_start_prefix(A.S, W.R, s, curr, neigh, out);
                 } else {
                     const uint32_t neigh = make_ref(REF_SUFFIX_BACK, np), curr = make_ref(REF_SUFFIX_FRONT, p);
-                    e = d == 0 ? sh_start_suffix(A.S, W.R, s, neigh, curr) : sh_start_suffix(A.S, W.R, s, curr, neigh);
+                    e = d == 0 ? sh_start_suffix(A.S, W.R, s, neigh, curr, out) : sh_start_suffix(A.S, W.R, s, curr, neigh, out);
                 }
-                if (e.kind == EMIT_NONE) shift_finish(W, job, v3(0.0f), 0.0f);
+                if (e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
             }
             const uint32_t slot = append(W.qout, e.kind);
             if (want && e.kind != EMIT_NONE) {
-                store_ctx(W.qout, slot, sh_pack(s));
+                if (keeps_context(e.kind)) store_ctx(W.qout, slot, sh_pack(s));
                 emit_job(W.qout, slot, job, e);
             }
         }
@@ -667,7 +688,6 @@ __device__ __forceinline__ void sg_init_state(SgState& s, uint64_t rng) {
     s.rng = rng;
     s.suf.recon = packed_invalid();
     s.suf.reconOutDir = v3(0.0f);
-    s.it = packed_invalid();
     s.lightDir = v3(0.0f);
     s.lightLen = 0.0f;
     s.color = v3(0.0f);
@@ -701,43 +721,44 @@ __global__ __launch_bounds__(WBLOCK) void k_w_suffix_init(WaveArgs W, int gather
                 e = sg_start(A.S, A.lp, s, load_prefix(W.prefixScratch, A.P, p).s);
             }
         }
-        if (run && e.kind == EMIT_NONE) sg_finish_store(W, p, s);
+        if (run && !keeps_context(e.kind)) sg_finish_store(W, p, s);
     }
     const uint32_t slot = append(W.qout, e.kind);
     if (run && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, sg_pack(s));
-        emit_job(W.qout, slot, p, e);
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, sg_pack(s));
+        emit_job(W.qout, slot, e.kind == EMIT_FINAL ? p | JOB_FINAL : p, e);
     }
 }
 
 __device__ __forceinline__ Emit sg_advance(const WaveArgs& W, uint32_t job, SgState& s, uint4 r, V3 o, V3 d) {
     Emit e;
     if (s.state == SG_TRACE) e = sg_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d), o);
-    else if (s.state == SG_NEE) e = sg_on_shadow(W.A.S, s, r.x != 0);
+    else if (s.state == SG_NEE) e = sg_on_shadow(s, r.x != 0, o);
     else e = sg_on_recon(s, inter_from_hit(W.A.S, r, d));
-    if (e.kind == EMIT_NONE) sg_finish_store(W, job, s);
+    if (!keeps_context(e.kind)) sg_finish_store(W, job, s);
     return e;
 }
 
 __global__ __launch_bounds__(WBLOCK) void k_w_sg_step(WaveArgs W) {
-    CX_FOR_JOBS(W) {
+    CX_FOR_JOBS(W, true) {
     const uint32_t i = _base + threadIdx.x;
-    const bool active = i < _n;
     Emit e = emit_none();
     SgState s;
-    uint32_t job = 0;
-    if (active) {
+    uint32_t job = JOB_FINAL;
+    if (i < _n) {
         const uint32_t slot = in_slot(W.qin, _qi, i);
         job = W.qin.job[slot];
-        s = sg_unpack(load_ctx<SG_CHUNKS>(W.qin, slot), W.qin.ray[slot], W.qin.ray[(size_t)W.qin.cap + slot]);
-        V3 o, d;
-        get_ray(W.qin, slot, o, d);
-        e = sg_advance(W, job, s, W.qin.res[slot], o, d);
+        if (!(job & JOB_FINAL)) {
+            s = sg_unpack(load_ctx<SG_CHUNKS>(W.qin, slot), W.qin.ray[(size_t)W.qin.cap + slot]);
+            V3 o, d;
+            get_ray(W.qin, slot, o, d);
+            e = sg_advance(W, job, s, W.qin.res[slot], o, d);
+        }
     }
     const uint32_t slot = append(W.qout, e.kind);
-    if (active && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, sg_pack(s));
-        emit_job(W.qout, slot, job, e);
+    if (e.kind != EMIT_NONE) {
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, sg_pack(s));
+        emit_job(W.qout, slot, e.kind == EMIT_FINAL ? job | JOB_FINAL : job, e);
     }
     }
 }
@@ -758,15 +779,16 @@ __global__ __launch_bounds__(WBLOCK) void k_w_suffix_temporal_setup(WaveArgs W) 
     for (uint32_t d = 0; d < 2; d++) {
         Emit e = emit_none();
         ShState s;
+        ShiftOut out;
         const uint32_t job = 2 * p + d;
         if (temporal) {
             const uint32_t back = make_ref(REF_SUFFIX_BACK, p), canon = make_ref(REF_SUFFIX_SCRATCH, p);
-            e = d == 0 ? sh_start_suffix(A.S, W.R, s, back, canon) : sh_start_suffix(A.S, W.R, s, canon, back);
-            if (e.kind == EMIT_NONE) shift_finish(W, job, v3(0.0f), 0.0f);
+            e = d == 0 ? sh_start_suffix(A.S, W.R, s, back, canon, out) : sh_start_suffix(A.S, W.R, s, canon, back, out);
+            if (e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
         }
         const uint32_t slot = append(W.qout, e.kind);
         if (temporal && e.kind != EMIT_NONE) {
-            store_ctx(W.qout, slot, sh_pack(s));
+            if (keeps_context(e.kind)) store_ctx(W.qout, slot, sh_pack(s));
             emit_job(W.qout, slot, job, e);
         }
     }
@@ -1023,21 +1045,22 @@ __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     const bool want = p < A.P && ((W.validMask[p] >> i) & 1u);
     Emit e = emit_none();
     ShState s;
+    ShiftOut out;
     const uint32_t job = ((uint32_t)p * k + i) * 2 + d;
     if (want) {
         const uint32_t n = A.neighIdx[(size_t)p * k + i];
         const uint32_t neigh = make_ref(REF_SUFFIX_FRONT, n);
         if (W.gIdx == 0) {
             const uint32_t canon = make_ref(REF_SUFFIX_SCRATCH, p);
-            e = d == 0 ? sh_start_suffix(A.S, W.R, s, neigh, canon) : sh_start_suffix(A.S, W.R, s, canon, neigh);
+            e = d == 0 ? sh_start_suffix(A.S, W.R, s, neigh, canon, out) : sh_start_suffix(A.S, W.R, s, canon, neigh, out);
         } else {
-            e = sh_start_suffix(A.S, W.R, s, neigh, make_ref(REF_PACKED_TRACED, p));
+            e = sh_start_suffix(A.S, W.R, s, neigh, make_ref(REF_PACKED_TRACED, p), out);
         }
-        if (e.kind == EMIT_NONE) shift_finish(W, job, v3(0.0f), 0.0f);
+        if (e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
     }
     const uint32_t slot = append(W.qout, e.kind);
     if (want && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, sh_pack(s));
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, sh_pack(s));
         emit_job(W.qout, slot, job, e);
     }
 }
@@ -1190,7 +1213,7 @@ __device__ __forceinline__ Emit fg_advance(const WaveArgs& W, uint32_t job, FgSt
 }
 
 __global__ __launch_bounds__(WBLOCK) void k_w_fg_step(WaveArgs W) {
-    CX_FOR_JOBS(W) {
+    CX_FOR_JOBS(W, false) {
     const uint32_t i = _base + threadIdx.x;
     const bool active = i < _n;
     Emit e = emit_none();
@@ -1206,7 +1229,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_fg_step(WaveArgs W) {
     }
     const uint32_t slot = append(W.qout, e.kind);
     if (active && e.kind != EMIT_NONE) {
-        store_ctx(W.qout, slot, fg_pack(s));
+        if (keeps_context(e.kind)) store_ctx(W.qout, slot, fg_pack(s));
         emit_job(W.qout, slot, job, e);
     }
     }
@@ -1216,11 +1239,13 @@ __global__ __launch_bounds__(WBLOCK) void k_w_fg_step(WaveArgs W) {
 // Tail: a machine's last rounds in one launch
 // ======================================================================================
 
+// is_final: whether a queued shadow ray of the machine is a final one.
 template <int M>
 struct Mach;
 template <>
 struct Mach<WK_PG_STEP> {
     using S = PgState;
+    __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, uint32_t slot) { return pg_load(W.qin, slot, W.A.lp); }
     __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
         return pg_advance(W, job, s, r, o, d);
@@ -1229,6 +1254,7 @@ struct Mach<WK_PG_STEP> {
 template <>
 struct Mach<WK_CP_STEP> {
     using S = CpState;
+    __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, uint32_t slot) { return cp_load(W.qin, slot); }
     __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
         return cp_advance(W, job, s, r, o, d);
@@ -1237,8 +1263,9 @@ struct Mach<WK_CP_STEP> {
 template <>
 struct Mach<WK_SG_STEP> {
     using S = SgState;
+    __device__ static bool is_final(uint32_t job) { return (job & JOB_FINAL) != 0; }
     __device__ static S load(const WaveArgs& W, uint32_t slot) {
-        return sg_unpack(load_ctx<SG_CHUNKS>(W.qin, slot), W.qin.ray[slot], W.qin.ray[(size_t)W.qin.cap + slot]);
+        return sg_unpack(load_ctx<SG_CHUNKS>(W.qin, slot), W.qin.ray[(size_t)W.qin.cap + slot]);
     }
     __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
         return sg_advance(W, job, s, r, o, d);
@@ -1247,6 +1274,7 @@ struct Mach<WK_SG_STEP> {
 template <>
 struct Mach<WK_SH_STEP> {
     using S = ShState;
+    __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, uint32_t slot) { return sh_unpack(load_ctx<SH_CHUNKS>(W.qin, slot)); }
     __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
         return sh_advance(W, job, s, r, o, d);
@@ -1255,6 +1283,7 @@ struct Mach<WK_SH_STEP> {
 template <>
 struct Mach<WK_FG_STEP> {
     using S = FgState;
+    __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, uint32_t slot) { return fg_unpack(load_ctx<FG_CHUNKS>(W.qin, slot)); }
     __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
         return fg_advance(W, job, s, r, o, d);
@@ -1269,25 +1298,26 @@ struct Mach<WK_FG_STEP> {
 // rounds cost nothing.  maxSteps is the machine's remaining round bound; a job still running
 // after it raises the queue's overflow flag (bit 1).
 template <int M, int WIDTH>
-__global__ __launch_bounds__(WBLOCK) void k_w_tail(WaveArgs W, uint32_t maxSteps, int pass) {
+__global__ __launch_bounds__(WBLOCK) void k_w_tail(WaveArgs W, uint32_t maxSteps, int pass, FinalArgs F) {
     __shared__ int s_st[SHORT_STACK * WBLOCK];
     int ovf[STACK_OVF<SHORT_STACK>];
     TravStack<SHORT_STACK, WBLOCK> st{s_st + threadIdx.x, ovf};
     const DScene& S = W.A.S;
     uint32_t nClosest = 0, nShadow = 0;
-    CX_FOR_JOBS(W) {
+    CX_FOR_JOBS(W, true) {
     const uint32_t i = _base + threadIdx.x;
     if (i < _n) {
         const uint32_t slot = in_slot(W.qin, _qi, i);
-        const uint32_t job = W.qin.job[slot];
-        typename Mach<M>::S s = Mach<M>::load(W, slot);
+        const uint32_t queued = W.qin.job[slot], job = M == WK_SG_STEP ? queued & ~JOB_FINAL : queued;
         const float4 a = W.qin.ray[slot], b = W.qin.ray[(size_t)W.qin.cap + slot];
         Emit e;
-        e.kind = i < _nc ? EMIT_CLOSEST : EMIT_SHADOW;
+        e.kind = i < _nc ? EMIT_CLOSEST : (Mach<M>::is_final(queued) ? EMIT_FINAL : EMIT_SHADOW);
         e.o = V3{a.x, a.y, a.z};
         e.tmin = a.w;
         e.d = V3{b.x, b.y, b.z};
         e.tmax = b.w;
+        typename Mach<M>::S s;
+        if (keeps_context(e.kind)) s = Mach<M>::load(W, slot);
         for (uint32_t k = 0; k < maxSteps && e.kind != EMIT_NONE; k++) {
             Hit h;
             uint4 r;
@@ -1301,7 +1331,12 @@ __global__ __launch_bounds__(WBLOCK) void k_w_tail(WaveArgs W, uint32_t maxSteps
                 r = uint4{occ ? 1u : 0u, 0u, 0u, 0u};
                 nShadow++;
             }
-            e = Mach<M>::advance(W, job, s, r, e.o, e.d);
+            if (e.kind == EMIT_FINAL) {
+                (void)final_answer(F, M == WK_SG_STEP ? job | JOB_FINAL : job, r.x != 0);
+                e = emit_none();
+            } else {
+                e = Mach<M>::advance(W, job, s, r, e.o, e.d);
+            }
         }
         if (e.kind != EMIT_NONE) atomicOr(W.qin.overflow, 2u);
     }
@@ -1378,24 +1413,56 @@ hipError_t wave_zero_counts(uint32_t* c, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t wave_trace(const DScene& S, const Queue& qin, const Queue& qout, unsigned long long* counters,
+// Where the final shadow rays of a machine leave their answers.
+static FinalArgs final_args(int step, const WaveArgs& W) {
+    FinalArgs F{};
+    switch (step) {
+        case WK_PG_STEP:
+            F.mode = FINAL_PREFIX;
+            F.records = W.prefixScratch;
+            break;
+        case WK_SG_STEP:
+            F.mode = FINAL_SUFFIX;
+            F.records = W.suffixScratch;
+            break;
+        case WK_SH_STEP:
+            F.mode = FINAL_SHIFT;
+            F.shiftRes = W.shiftRes;
+            break;
+        case WK_CP_STEP:
+            F.mode = FINAL_PATH;
+            F.radiance = W.radScratch;
+            F.out = W.A.out;
+            F.accum = W.A.lp.enableAccum != 0 ? 1u : 0u;
+            F.frameIdx = W.A.lp.frameIdx;
+            F.dyn = W.A.dyn;
+            break;
+        default: F.mode = FINAL_NONE; break;
+    }
+    return F;
+}
+
+hipError_t wave_trace(int step, const WaveArgs& W, const Queue& qin, const Queue& qout, unsigned long long* counters,
                       uint32_t minChunk, hipStream_t s) {
+    const DScene& S = W.A.S;
+    const FinalArgs F = final_args(step, W);
     const dim3 b(WBLOCK);
     const uint32_t mc = std::max(1u, std::min(minChunk, TRACE_CHUNK));
     if (S.width == 4)
-        hipLaunchKernelGGL(k_q_trace<4>, range_grid(qin, k_q_trace<4>), b, 0, s, S, qin, qout, counters, mc);
+        hipLaunchKernelGGL(k_q_trace<4>, range_grid(qin, k_q_trace<4>), b, 0, s, S, qin, qout, counters, mc, F);
     else if (S.width == 8)
-        hipLaunchKernelGGL(k_q_trace<8>, range_grid(qin, k_q_trace<8>), b, 0, s, S, qin, qout, counters, mc);
-    else hipLaunchKernelGGL(k_q_trace<2>, range_grid(qin, k_q_trace<2>), b, 0, s, S, qin, qout, counters, mc);
+        hipLaunchKernelGGL(k_q_trace<8>, range_grid(qin, k_q_trace<8>), b, 0, s, S, qin, qout, counters, mc, F);
+    else hipLaunchKernelGGL(k_q_trace<2>, range_grid(qin, k_q_trace<2>), b, 0, s, S, qin, qout, counters, mc, F);
     return hipGetLastError();
 }
 
 template <int M>
 static hipError_t tail_launch_w(const WaveArgs& W, uint32_t maxSteps, int pass, hipStream_t s) {
     const dim3 g = stride_grid(W.qin), b(WBLOCK);
-    if (W.A.S.width == 4) hipLaunchKernelGGL((k_w_tail<M, 4>), g, b, 0, s, W, maxSteps, pass);
-    else if (W.A.S.width == 8) hipLaunchKernelGGL((k_w_tail<M, 8>), g, b, 0, s, W, maxSteps, pass);
-    else hipLaunchKernelGGL((k_w_tail<M, 2>), g, b, 0, s, W, maxSteps, pass);
+    const FinalArgs F = final_args(M, W);
+    if (W.A.S.width == 4) hipLaunchKernelGGL((k_w_tail<M, 4>), g, b, 0, s, W, maxSteps, pass, F);
+    else if (W.A.S.width == 8) hipLaunchKernelGGL((k_w_tail<M, 8>), g, b, 0, s, W, maxSteps, pass, F);
+    else hipLaunchKernelGGL((k_w_tail<M, 2>), g, b, 0, s, W, maxSteps, pass, F);
     return hipGetLastError();
 }
 

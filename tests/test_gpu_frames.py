@@ -155,3 +155,36 @@ def test_frames_match_oracle(case, exec_mode, orc, cx_runtime, cx_ctx):
             assert (hist[1:] > 0).all(), hist
         if "full_k" in c:
             assert hist[k] >= c["full_k"], hist
+
+
+@pytest.mark.parametrize("rounds", [0, 1, 2, 6])
+@pytest.mark.parametrize("mode", ["path_tracer", "restir_pt_cornell", "conditional_restir"])
+def test_final_shadow_rays_in_queue_and_tail_match_megakernel(mode, rounds, cx_runtime, cx_ctx):
+    """A walk or shift whose last ray is a shadow ray stores its result ahead of the ray, and the
+    kernel that answers the ray takes it back if it is occluded: in the traversal of a queue, or in
+    the tail after `rounds` rounds (0: no tail), with accumulation, eagerly and replayed from a
+    frame graph.  Every frame equals the one-kernel-per-pass mode, which traces first, bit for
+    bit, and so do the reservoirs."""
+    W, H = 40, 24
+    sc = tent_grid_scene()
+    gs = cx_runtime.Scene(cx_ctx, sc)
+    p = abi.workload_params(mode, W, H, gs.size)
+    p.enableAccum = 0 if mode == "conditional_restir" else 1
+    cam = scenes.orbit_camera(sc, W, H)
+    cd = abi.CameraData.from_dict(cam.data())
+    rens = [cx_runtime.Renderer(W, H, cx_ctx, cam, gs, params=p, seed=9) for _ in range(3)]
+    rens[0].set_exec_mode("megakernel")
+    for ren in rens[1:]:
+        ren.set_wave_rounds(rounds)
+    rens[2].set_graph_mode(True)
+    for f in range(4):
+        imgs = [ren.launch_frame(cd, f == 0).numpy() for ren in rens]
+        for img in imgs[1:]:
+            assert np.array_equal(imgs[0].view(np.uint32), img.view(np.uint32)), f
+    if mode != "path_tracer":
+        ref = rens[0].prefix(rens[0].state().frontBufferIdx)
+        for ren in rens[1:]:
+            got = ren.prefix(ren.state().frontBufferIdx)
+            for k in ref:
+                assert np.array_equal(ref[k].view(np.uint32), got[k].view(np.uint32)), k
+    assert all(ren.stats().queueOverflow == 0 for ren in rens[1:])
