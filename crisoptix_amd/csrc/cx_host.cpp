@@ -79,7 +79,8 @@ struct cx_renderer {
         uint32_t* job[2] = {nullptr, nullptr};
         float4* ray[2] = {nullptr, nullptr};
         uint4* res[2] = {nullptr, nullptr};
-        uint32_t* count = nullptr;   // [2][2] closest / shadow count of each queue
+        uint32_t* count = nullptr;   // [MACHINE_SETS][MACHINE_WORDS] counters of the machines, overflow flag
+        uint32_t set = MACHINE_SETS; // the next machine's counters (MACHINE_SETS: clear all first)
         float4* shiftRes = nullptr;
         size_t jobCap = 0;           // jobs a queue holds
         size_t ctxWords = 0;         // 16-byte context words a queue holds
@@ -113,7 +114,7 @@ struct cx_renderer {
     // 8192 / 16384 -> 9.53 / 8.59-8.62 / 8.45 / 8.47 ms; a machine of fewer jobs launches fewer.
     uint32_t gridLimit = 8192;
     // Set by cx_batch_frame while it enqueues this renderer's frame beside other views: the
-    // traversal then keeps whole 32-ray chunks (wave_trace minChunk); results are unchanged.
+    // traversal then keeps whole 32-ray chunks (wave_trace); results are unchanged.
     bool concurrent = false;
     uint32_t waveRounds = CX_WAVE_ROUNDS_DEFAULT;   // rounds before the tail kernel, every machine (0: all; default per machine)
     uint64_t allocEpoch = 0;     // bumped whenever a buffer a frame uses is reallocated
@@ -324,8 +325,8 @@ size_t shift_jobs(const cx_renderer* r, const cx_launch_params& lp) {
     return (size_t)2 * slots * r->P;
 }
 
-// Two queues' stripe counters, then the shared overflow flag.
-constexpr size_t COUNT_WORDS = 2 * QSTRIPES * QCOUNT_STRIDE + 16;
+// The counters of MACHINE_SETS machines, then the shared overflow flag.
+constexpr size_t COUNT_WORDS = (size_t)MACHINE_SETS * MACHINE_WORDS + 16;
 
 int ensure_wave(cx_renderer* r, const cx_launch_params& lp) {
     auto& w = r->wave;
@@ -409,8 +410,9 @@ Queue queue_view(const cx_renderer* r, int side, uint32_t jobs) {
     q.job = r->wave.job[side];
     q.ray = r->wave.ray[side];
     q.res = r->wave.res[side];
-    q.count = r->wave.count + (size_t)side * QSTRIPES * QCOUNT_STRIDE;
-    q.overflow = r->wave.count + (size_t)2 * QSTRIPES * QCOUNT_STRIDE;
+    uint32_t* const set = r->wave.count + (size_t)r->wave.set * MACHINE_WORDS;
+    q.count = set + (size_t)side * QSTRIPES * QCOUNT_STRIDE;
+    q.overflow = r->wave.count + (size_t)MACHINE_SETS * MACHINE_WORDS;
     q.jobs = jobs;
     q.maxBlocks = r->gridLimit;
     q.stripeCap = queue_stripe_cap(jobs, r->P, r->gridLimit);
@@ -462,10 +464,6 @@ WaveArgs make_wave_args(const cx_renderer* r, const FrameArgs& A) {
     return W;
 }
 
-// Runs one machine: `setup` (one thread per pixel) appends the first rays to queue 0, then
-// `rounds` rounds of traversal + step.  Every job finishes within `rounds` rounds (the bounds
-// below are the longest chains of trace calls of each machine), and a round whose queue is
-// empty costs two near-empty launches.
 // Records one event of the traversal timing pairs (grows the pool outside any capture).
 void trace_rec(cx_renderer* r, hipStream_t s) {
     if (!r->timing) return;
@@ -480,40 +478,68 @@ void trace_rec(cx_renderer* r, hipStream_t s) {
     (void)hipEventRecord(r->traceEv[r->traceEvUsed++], s);
 }
 
-// Wavefront rounds before the tail kernel, per machine: 3 for suffix walks, 2 for the others.
-// Measured on the 1080p Conditional ReSTIR frame (tent of traced lights, 14.6 rays/px): every
-// machine 1 (suffix walks) or 2 (the others) / 2 / 3 / 4 / 6 rounds, or all rounds as traversal
-// + step (0) -> 29.28 / 28.77 / 28.91 / 29.15 / 29.82 / 29.88 ms per frame; then, with the
-// range-per-wavefront traversal, suffix walks 3 / 4 / 5 rounds against 2 -> 25.43 / 25.69 / 25.98
-// against 25.77 ms, shifts 1 or 3 and prefix walks 1 or 3 against 2 no better.  The tail traces
-// in place at 3 waves per SIMD, so long suffix walks are cheaper in the queue rounds.
-uint32_t default_wave_rounds(int machine) { return machine == WK_SG_STEP ? 3u : 2u; }
+// Rounds of traversal and step before the tail kernel, at most; a round that finds no more than
+// tailJobs jobs left skips itself and those after it (WaveArgs::skip).  tailJobs is what the
+// machine's tail holds on the device at once, four lanes a job: up to there every job follows its
+// own chain of rays without waiting for the slowest ray of each round, above it the queue's 7
+// waves per SIMD beat the tail's 2 to 4.
+//  * An image of at most tailJobs pixels goes to the tail at once: 160x90 Conditional ReSTIR 1.42 ms
+//    against 1.96 with rounds, 320x200 2.19 against 2.76, 64x64 path tracer 285 us against 410; at
+//    more pixels than that, 400x300 ReSTIR PT 1.00 ms against 1.04 with one round, 512x512 gradient
+//    step 1.69 against 1.47.
+//  * Suffix walks at most 3 rounds, prefix walks and suffix shifts 2 (1080p Conditional ReSTIR:
+//    suffix walks 3 / 4 / 5 against 2 -> 25.43 / 25.69 / 25.98 against 25.77 ms before the tail
+//    took four lanes a job; one shift round less, 14.55 against 13.83 ms after).
+//  * Complete paths, whose context is 2 chunks, 6 rounds: 720p 1.51 ms against 1.79 (2), 1.57 (4)
+//    and 1.57 (9).
+//  * Prefix shifts, most of which are one shadow ray, go to the tail at once up to 768 k pixels:
+//    256x256 ReSTIR PT 352 us against 391 with 2 rounds, 700x500 1.67 ms against 1.77, 900x600
+//    1.28 against 1.35, but 1920x1080 6.52 against 6.02.
+static constexpr uint32_t PREFIX_SHIFT_TAIL_PIXELS = 768u << 10;
 
+uint32_t default_wave_rounds(int machine, int pass, uint32_t P, uint32_t tailJobs) {
+    if (P <= tailJobs) return 0u;
+    const bool prefixShift = pass == CX_PASS_PREFIX_GEN_TEMP || pass == CX_PASS_PREFIX_SPATIAL;
+    switch (machine) {
+        case WK_SG_STEP: return 3u;
+        case WK_CP_STEP: return 6u;
+        case WK_SH_STEP: return prefixShift && tailJobs && P <= PREFIX_SHIFT_TAIL_PIXELS ? 0u : 2u;
+        default: return 2u;
+    }
+}
+
+// Runs one machine: `setup` (one thread per pixel) appends the first rays to queue 0, then at most
+// `rounds` rounds of traversal + step, or fewer and the tail.  Every job finishes within `rounds`
+// rounds (the bounds in wave_pass are the longest chains of trace calls of each machine).
 hipError_t run_machine(cx_renderer* r, WaveArgs W, int setup, int step, uint32_t cap, uint32_t rounds,
                        int pass, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    if (r->wave.set >= MACHINE_SETS) {
+        e = launch_zero_words(r->wave.count, MACHINE_SETS * MACHINE_WORDS, s);
+        r->wave.set = 0;
+    }
     W.qin = queue_view(r, 1, cap);
     W.qout = queue_view(r, 0, cap);
     if ((size_t)W.qout.cap > r->wave.jobCap) return hipErrorInvalidValue;   // ensure_wave sized every machine
-    hipError_t e = wave_zero_counts(W.qout.count, s);
     if (e == hipSuccess) e = wave_launch(setup, W, r->P, s);
-    int cur = 0;
-    const uint32_t wr = r->waveRounds != CX_WAVE_ROUNDS_DEFAULT ? r->waveRounds : default_wave_rounds(step);
-    const uint32_t waveRounds = (wr > 0 && wr < rounds) ? wr : rounds;
-    for (uint32_t i = 0; i < waveRounds && e == hipSuccess; i++) {
-        const Queue qin = queue_view(r, cur, cap), qout = queue_view(r, 1 - cur, cap);
+    W.qin = queue_view(r, 0, cap);   // the setup's queue is side 0
+    W.qout = queue_view(r, 1, cap);
+    W.side = r->wave.count + (size_t)r->wave.set * MACHINE_WORDS + 2 * QSTRIPES * QCOUNT_STRIDE;
+    // a setting of 0 runs every round in the queue; a default of 0 starts with the tail
+    const bool set = r->waveRounds != CX_WAVE_ROUNDS_DEFAULT;
+    const uint32_t tailJobs = wave_tail_jobs(step, W.A.S);
+    const uint32_t wr = set ? (r->waveRounds ? r->waveRounds : rounds) : default_wave_rounds(step, pass, r->P, tailJobs);
+    const uint32_t waveRounds = std::min({wr, rounds, MACHINE_ROUNDS - 1});
+    W.skip = set || waveRounds == rounds ? 0u : tailJobs;
+    for (W.round = 0; W.round < waveRounds && e == hipSuccess; W.round++) {
         trace_rec(r, s);
-        e = wave_trace(step, W, qin, qout, W.A.counters + 2 * pass, r->concurrent ? ~0u : 1u, s);
+        e = wave_trace(step, W, W.A.counters + 2 * pass, r->concurrent, s);
         trace_rec(r, s);
-        W.qin = qin;
-        W.qout = qout;
         if (e == hipSuccess) e = wave_launch(step, W, 0, s);
-        cur = 1 - cur;
     }
-    if (e == hipSuccess && waveRounds < rounds) {   // the remaining rounds in one launch
-        W.qin = queue_view(r, cur, cap);
-        W.qout = queue_view(r, 1 - cur, cap);
-        e = wave_tail(step, W, rounds - waveRounds, pass, s);
-    }
+    if (e == hipSuccess && waveRounds < rounds)   // the remaining rounds in one launch
+        e = wave_tail(step, W, rounds, pass, s);
+    r->wave.set++;
     return e;
 }
 
@@ -1306,7 +1332,12 @@ int frame_body(cx_renderer* r, void* stream) {
         d.frameIdx = r->params.frameIdx;
         CX_HIP(r->ctx, launch_next_dyn(r->dyn, r->devRng, d, s));
     }
-    CX_HIP(r->ctx, launch_zero_counters(r->counters, COUNTER_STRIPES * NUM_COUNTERS, s));
+    // one kernel clears the frame's counters and those of its machines
+    const bool wave = r->exec == CX_EXEC_WAVEFRONT;
+    if (wave && (rc = ensure_wave(r, lp))) return rc;
+    CX_HIP(r->ctx, launch_zero_counters(r->counters, COUNTER_STRIPES * NUM_COUNTERS, wave ? r->wave.count : nullptr,
+                                        wave ? MACHINE_SETS * MACHINE_WORDS : 0u, s));
+    if (wave) r->wave.set = 0;
     rec(r, 0, s);
     auto run = [&](cx_pass p) -> int {
         r->passRan[p] = true;
@@ -1603,7 +1634,7 @@ int cx_renderer_get_stats(cx_renderer* r, cx_frame_stats* st) {
     st->numEntries = nv;
     if (r->wave.count) {
         uint32_t ovf = 0;
-        CX_HIP(r->ctx, hipMemcpy(&ovf, r->wave.count + (size_t)2 * QSTRIPES * QCOUNT_STRIDE, 4, hipMemcpyDeviceToHost));
+        CX_HIP(r->ctx, hipMemcpy(&ovf, r->wave.count + (size_t)MACHINE_SETS * MACHINE_WORDS, 4, hipMemcpyDeviceToHost));
         st->queueOverflow = ovf;
     }
     if (r->evValid) {

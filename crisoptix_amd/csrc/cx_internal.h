@@ -14,7 +14,9 @@ namespace cx {
 
 hipError_t launch_pass(int pass, const FrameArgs& A, hipStream_t s);
 hipError_t launch_reset(const FrameArgs& A, hipStream_t s);
-hipError_t launch_zero_counters(unsigned long long* c, uint32_t n, hipStream_t s);
+// words: the wavefront machines' counters, cleared with the frame's counters, or null.
+hipError_t launch_zero_counters(unsigned long long* c, uint32_t n, uint32_t* words, uint32_t numWords, hipStream_t s);
+hipError_t launch_zero_words(uint32_t* words, uint32_t n, hipStream_t s);
 hipError_t launch_set_dyn(FrameDyn* dst, const FrameDyn& d, hipStream_t s);
 hipError_t launch_next_dyn(FrameDyn* dst, uint64_t* state, const FrameDyn& d, hipStream_t s);
 hipError_t launch_set_materials(DMaterial* dst, const float* rows, uint32_t n, hipStream_t s);
@@ -94,12 +96,12 @@ enum WaveKernel {
     WK_SUFFIX_AOS,
 };
 
-hipError_t wave_zero_counts(uint32_t* c, hipStream_t s);
+// Jobs of machine `step` that the tail holds on the device at once, four lanes each (0: a width
+// whose rays take one lane).
+uint32_t wave_tail_jobs(int step, const DScene& S);
 hipError_t wave_tail(int step, const WaveArgs& W, uint32_t maxSteps, int pass, hipStream_t s);
-// minChunk: the fewest rays per traversal chunk (1 for a frame that has the device alone, the
-// largest chunk for one that runs beside others; results are the same either way).
-hipError_t wave_trace(int step, const WaveArgs& W, const Queue& qin, const Queue& qout, unsigned long long* counters,
-                      uint32_t minChunk, hipStream_t s);
+// wholeChunks: a frame that runs beside others (results are the same either way).
+hipError_t wave_trace(int step, const WaveArgs& W, unsigned long long* counters, bool wholeChunks, hipStream_t s);
 hipError_t wave_launch(int kernel, const WaveArgs& W, uint32_t threads, hipStream_t s);
 
 // Most triangles per BVH leaf when cx_scene_desc.bvhMaxLeafSize is 0.  Measured on the

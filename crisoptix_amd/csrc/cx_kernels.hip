@@ -442,9 +442,11 @@ __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
     if (i < n) p[i] = 0u;
 }
 
-__global__ void k_zero_u64(unsigned long long* p, uint32_t n, unsigned long long minInit) {
+__global__ void k_zero_u64(unsigned long long* p, uint32_t n, unsigned long long minInit, uint32_t* words,
+                           uint32_t numWords) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = (i % NUM_COUNTERS == (uint32_t)STAT_MIN) ? minInit : 0ull;
+    if (i < numWords) words[i] = 0u;
 }
 
 // ---- entry sort: least-significant-digit radix sort of the valid entries' Morton keys ----
@@ -964,8 +966,15 @@ hipError_t launch_reset(const FrameArgs& A, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_zero_counters(unsigned long long* c, uint32_t n, hipStream_t s) {
-    hipLaunchKernelGGL(k_zero_u64, dim3((n + 255) / 256), dim3(256), 0, s, c, n, 0xFFFFFFFFull);
+hipError_t launch_zero_counters(unsigned long long* c, uint32_t n, uint32_t* words, uint32_t numWords,
+                                hipStream_t s) {
+    const uint32_t m = std::max(n, numWords);
+    hipLaunchKernelGGL(k_zero_u64, dim3((m + 255) / 256), dim3(256), 0, s, c, n, 0xFFFFFFFFull, words, numWords);
+    return hipGetLastError();
+}
+
+hipError_t launch_zero_words(uint32_t* words, uint32_t n, hipStream_t s) {
+    hipLaunchKernelGGL(k_zero_u32, dim3((n + 255) / 256), dim3(256), 0, s, words, n);
     return hipGetLastError();
 }
 

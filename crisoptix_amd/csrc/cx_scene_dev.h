@@ -568,6 +568,112 @@ CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& st, bool any) {
     return false;
 }
 
+// ---- four lanes per ray ----
+//
+// Where there are fewer rays than lanes, a ray's time is its chain of steps: a fetch, then the
+// step's instructions one after another.  Four neighbouring lanes (a quad) then share one 4-wide
+// ray: each tests one child box of a node, or one triangle of a leaf, so a node step is about 60
+// instructions instead of 110 and its fetch 7 loads of one float per lane from one 128-byte node.
+// The quad's state is the same in its four lanes, and they stay together.  The nodes are visited
+// nearest child first as above (ties and the last two bits of a distance aside), so the answers
+// are the same.
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_swap(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xF, 0xF, true);
+}
+static constexpr int QUAD_1 = 0xB1, QUAD_2 = 0x4E, QUAD_3 = 0x1B;   // the lane 1, 2 or 3 away (xor) in the quad
+
+__device__ __forceinline__ uint32_t quad_or(uint32_t x) {
+    x |= quad_swap<QUAD_1>(x);
+    return x | quad_swap<QUAD_2>(x);
+}
+
+// The lesser of this lane's and the other lane's hit by (t, primitive), u and v with it.
+template <int CTRL>
+__device__ __forceinline__ void quad_best(Hit& h) {
+    Hit o;
+    o.t = __builtin_bit_cast(float, quad_swap<CTRL>(__builtin_bit_cast(uint32_t, h.t)));
+    o.u = __builtin_bit_cast(float, quad_swap<CTRL>(__builtin_bit_cast(uint32_t, h.u)));
+    o.v = __builtin_bit_cast(float, quad_swap<CTRL>(__builtin_bit_cast(uint32_t, h.v)));
+    o.prim = quad_swap<CTRL>(h.prim);
+    if (o.t < h.t || (o.t == h.t && o.prim < h.prim)) h = o;
+}
+
+// Traces one ray per quad to its end; `col` is the quad's stack column in LDS (STACK_DEPTH entries,
+// `stride` apart).  The whole quad calls it with the same ray.  Closest hit in best (prim
+// INVALID_PRIM: a miss), occlusion as best.prim != INVALID_PRIM.
+__device__ __forceinline__ void quad_trace(const DScene& S, V3 o, V3 d, float tmin, float tmax, bool any, Hit& best,
+                                           int* col, int stride) {
+    best = Hit{INVALID_PRIM, tmax, 0.0f, 0.0f};
+    if (S.numTris == 0) return;
+    const RayPre rp = ray_pre(d);
+    const RaySlab r = slab_init(o, d);
+    const uint32_t j = threadIdx.x & 3u;
+    const uint32_t ax = 4u * j + ((__builtin_bit_cast(uint32_t, r.inv.x) >> 27) & 16u);
+    const uint32_t ay = 4u * j + ((__builtin_bit_cast(uint32_t, r.inv.y) >> 27) & 16u) + 32u;
+    const uint32_t az = 4u * j + ((__builtin_bit_cast(uint32_t, r.inv.z) >> 27) & 16u) + 64u;
+    const char* const nodes = (const char*)S.wnodes;
+    int ref = S.wroot, sp = 0;
+    while (true) {
+        const int top = col[(sp > 0 ? sp - 1 : 0) * stride];
+        if (ref >= 0) {
+            const uint32_t off = (uint32_t)ref * 128u;
+            const float nx = *(const float*)(nodes + (off | ax)), fx = *(const float*)(nodes + ((off | ax) ^ 16u));
+            const float ny = *(const float*)(nodes + (off | ay)), fy = *(const float*)(nodes + ((off | ay) ^ 16u));
+            const float nz = *(const float*)(nodes + (off | az)), fz = *(const float*)(nodes + ((off | az) ^ 16u));
+            const int child = *(const int*)(nodes + (off | (96u + 4u * j)));
+            bool h;
+            const float t = slab_box(nx, fx, ny, fy, nz, fz, r, tmin, best.t, h);
+            h = h && child != WIDE_EMPTY;
+            // distance with the lane in its last two bits, as a signed number; misses above all
+            const int miss = 0x7fffffff;
+            const int k = h ? (int)((__builtin_bit_cast(uint32_t, t) & ~3u) | j) : miss;
+            const int k1 = (int)quad_swap<QUAD_1>((uint32_t)k), k2 = (int)quad_swap<QUAD_2>((uint32_t)k),
+                      k3 = (int)quad_swap<QUAD_3>((uint32_t)k);
+            const int first = min(min(k, k1), min(k2, k3));
+            if (first != miss) {
+                const int nearer = (k1 < k ? 1 : 0) + (k2 < k ? 1 : 0) + (k3 < k ? 1 : 0);
+                const int more = (k != miss ? 1 : 0) + (k1 != miss ? 1 : 0) + (k2 != miss ? 1 : 0) +
+                                 (k3 != miss ? 1 : 0) - 1;   // entries to push
+                if (h && nearer > 0) col[(sp + more - nearer) * stride] = child;
+                __builtin_amdgcn_wave_barrier();   // the quad's other lanes read the entries
+                sp += more;
+                ref = (int)quad_or(k == first ? (uint32_t)child : 0u);
+                continue;
+            }
+        } else {
+            const uint32_t code = ~(uint32_t)ref;
+            const uint32_t slot0 = code >> 4, cnt = code & 15u;
+            for (uint32_t b = 0; b < cnt; b += 4u) {
+                Hit h = Hit{INVALID_PRIM, INFINITY, 0.0f, 0.0f};
+                bool ok = false;
+                if (b + j < cnt) {
+                    const f32x4* tv = (const f32x4*)S.tris + 3 * (size_t)(slot0 + b + j);
+                    const f32x4 q0 = tv[0], q1 = tv[1], q2 = tv[2];
+                    float t, u, v;
+                    if (!(bits_of(q1[3]) & (any ? 2u : 1u)) &&
+                        tri_hit(o, rp, V3{q0[0], q0[1], q0[2]}, V3{q1[0], q1[1], q1[2]}, V3{q2[0], q2[1], q2[2]}, tmin,
+                                best.t, t, u, v)) {
+                        ok = true;
+                        h = Hit{bits_of(q0[3]), t, u, v};
+                    }
+                }
+                if (!quad_or(ok ? 1u : 0u)) continue;
+                if (any) {
+                    best.prim = 0u;
+                    return;
+                }
+                quad_best<QUAD_1>(h);
+                quad_best<QUAD_2>(h);
+                if (h.t < best.t || (h.t == best.t && h.prim < best.prim)) best = h;
+            }
+        }
+        if (sp == 0) return;
+        --sp;
+        ref = top;
+    }
+}
+
 template <bool ANY, int WIDTH, typename Stack>
 CX_HD bool trav_step(const DScene& S, TravRay& r, Stack& st) {
     return trav_step_rt<WIDTH>(S, r, st, ANY);

@@ -35,6 +35,14 @@ static constexpr uint32_t JOB_FINAL = 0x80000000u;
 static constexpr uint32_t QSTRIPES = 64;       // one per lane of the wavefront that scans them
 static constexpr uint32_t QCOUNT_STRIDE = 16;  // words between stripes' counters (64 bytes)
 
+// Counter words of one machine: the stripe counts of its two queues and, per round, which of them
+// holds the jobs.  A frame's machines use one
+// set after another, so that one kernel at the start of the frame clears them all (a kernel per
+// machine took 5 us each, 8 of them in a Conditional ReSTIR frame).
+static constexpr uint32_t MACHINE_ROUNDS = 272;   // rounds of the longest walk and one more (maxPathLen <= 255)
+static constexpr uint32_t MACHINE_WORDS = 2 * QSTRIPES * QCOUNT_STRIDE + MACHINE_ROUNDS;
+static constexpr uint32_t MACHINE_SETS = 16;
+
 struct Queue {
     uint4* ctx;         // [chunks][cap]
     uint32_t* job;      // [cap]
@@ -819,13 +827,16 @@ struct FinalArgs {
     const FrameDyn* dyn;      // frame index of a graph replay, or null
 };
 
-// Everything a wavefront kernel reads or writes.  qin is the queue whose rays were just
-// answered, qout the queue the kernel appends to; both share one allocation per side and are
-// viewed with the capacity and chunk count of the machine in flight.
+// Everything a wavefront kernel reads or writes.  qin and qout are the machine's two queues; both
+// share one allocation per side and are viewed with the capacity and chunk count of the machine in
+// flight.  A setup kernel appends to qout; in the rounds, side[round] says which queue holds the
+// jobs (0: qin), and a round of at most `skip` jobs is left to the tail.
 struct WaveArgs {
     FrameArgs A;
     RecordSet R;
     Queue qin, qout;
+    uint32_t* side;
+    uint32_t round, skip;
     uint4* prefixScratch;   // [PREFIX_CHUNKS][P] canonical prefix of the pass
     uint4* suffixScratch;   // [SUFFIX_CHUNKS][P] canonical suffix of the pass
     uint4* packedScratch;   // [P][2] last vertex of a final-gather prefix (Packed)

@@ -188,3 +188,31 @@ def test_final_shadow_rays_in_queue_and_tail_match_megakernel(mode, rounds, cx_r
             for k in ref:
                 assert np.array_equal(ref[k].view(np.uint32), got[k].view(np.uint32)), k
     assert all(ren.stats().queueOverflow == 0 for ren in rens[1:])
+
+
+@pytest.mark.parametrize("width", [2, 4, 8])
+@pytest.mark.parametrize("queue_grid", [1, 3, 8192])
+@pytest.mark.parametrize("mode", ["path_tracer", "conditional_restir"])
+def test_queue_paths_match_megakernel(mode, queue_grid, width, cx_runtime, cx_ctx):
+    """The traversal of a queue takes one lane per ray when there are more rays than its grid holds
+    at four lanes each, or when the tree is not 4-wide; the tail likewise.  A grid of one or three
+    blocks over a small image takes the long-queue path, the default grid the four-lane one; both
+    with every round in the queue and with the default rounds.  All equal the one-kernel-per-pass
+    mode bit for bit."""
+    W, H = 61, 37
+    sc = tent_grid_scene()
+    gs = cx_runtime.Scene(cx_ctx, sc, width=width)
+    assert gs.info.bvhWidth == width
+    p = abi.workload_params(mode, W, H, gs.size)
+    cam = scenes.orbit_camera(sc, W, H)
+    cd = abi.CameraData.from_dict(cam.data())
+    rens = [cx_runtime.Renderer(W, H, cx_ctx, cam, gs, params=p, seed=31) for _ in range(3)]
+    rens[0].set_exec_mode("megakernel")
+    for ren in rens[1:]:
+        ren.set_queue_grid(queue_grid)
+    rens[1].set_wave_rounds(0)
+    for f in range(2):
+        imgs = [ren.launch_frame(cd, f == 0).numpy() for ren in rens]
+        for img in imgs[1:]:
+            assert np.array_equal(imgs[0].view(np.uint32), img.view(np.uint32)), f
+    assert all(ren.stats().queueOverflow == 0 for ren in rens[1:])
