@@ -1032,13 +1032,13 @@ int cx_bvh_host_trace(const cx_scene_desc* d, const float* rays, uint32_t n, int
 int cx_trace_closest(cx_ctx* ctx, const cx_scene* s, const float* rays, uint32_t n, uint32_t* prim, float* t,
                      float* u, float* v, void* stream) {
     if (!ctx || !s || (n && (!rays || !prim || !t || !u || !v))) return set_err(ctx, CX_ERR_INVALID_ARG, "null argument");
-    CX_HIP(ctx, launch_trace(s->d, rays, n, 0, prim, t, u, v, nullptr, (hipStream_t)stream));
+    CX_HIP(ctx, launch_trace(s->d, rays, n, 0, prim, t, u, v, (hipStream_t)stream));
     return CX_OK;
 }
 
 int cx_trace_occluded(cx_ctx* ctx, const cx_scene* s, const float* rays, uint32_t n, uint32_t* occ, void* stream) {
     if (!ctx || !s || (n && (!rays || !occ))) return set_err(ctx, CX_ERR_INVALID_ARG, "null argument");
-    CX_HIP(ctx, launch_trace(s->d, rays, n, 1, nullptr, nullptr, nullptr, nullptr, occ, (hipStream_t)stream));
+    CX_HIP(ctx, launch_trace(s->d, rays, n, 1, occ, nullptr, nullptr, nullptr, (hipStream_t)stream));
     return CX_OK;
 }
 

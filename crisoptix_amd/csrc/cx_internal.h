@@ -48,8 +48,9 @@ hipError_t noalloc_setup(int device);
 void ctx_set_error(cx_ctx* ctx, const char* msg);
 int ctx_device(const cx_ctx* ctx);
 
-hipError_t launch_trace(const DScene& S, const float* rays, uint32_t n, int anyHit, uint32_t* prim, float* t,
-                        float* u, float* v, uint32_t* occ, hipStream_t s);
+// Rays [n][8] answered into prim, t, u, v (closest hit) or prim alone (occlusion flags).
+hipError_t launch_trace(const DScene& S, const float* rays, uint32_t n, int anyHit, uint32_t* prim, float* t, float* u,
+                        float* v, hipStream_t s);
 
 // Path-replay adjoint (cx_adjoint.hip).  Gradients accumulate into the double arrays.
 struct AdjArgs {

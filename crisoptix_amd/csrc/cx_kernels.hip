@@ -916,29 +916,6 @@ __global__ void k_reset_state(FrameArgs A) {
     A.neighCount[p] = 0;
 }
 
-// ------------------------------------------------------------------------------------------
-// Standalone traversal (cx_trace_closest / cx_trace_occluded)
-// ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void k_trace(DScene S, const float* rays, uint32_t n, int anyHit,
-                                                 uint32_t* prim, float* t, float* u, float* v, uint32_t* occ) {
-    __shared__ int s_stack[STACK_DEPTH * BLOCK];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float* r = rays + 8 * (size_t)i;
-    Hit h;
-    const V3 o = V3{r[0], r[1], r[2]}, d = V3{r[3], r[4], r[5]};
-    if (anyHit) {
-        occ[i] = traverse<true>(S, o, d, r[6], r[7], h, s_stack + threadIdx.x) ? 1u : 0u;
-    } else {
-        traverse<false>(S, o, d, r[6], r[7], h, s_stack + threadIdx.x);
-        const bool hit = h.prim != INVALID_PRIM;
-        prim[i] = h.prim;
-        t[i] = hit ? h.t : 0.0f;
-        u[i] = hit ? h.u : 0.0f;
-        v[i] = hit ? h.v : 0.0f;
-    }
-}
-
 // ==========================================================================================
 // Host launchers
 // ==========================================================================================
@@ -1098,14 +1075,6 @@ hipError_t launch_entries_query(const EntryTree& T, const float* q, uint32_t nq,
     const dim3 grid((nq + BLOCK - 1) / BLOCK);
     if (k <= 8) hipLaunchKernelGGL(k_entries_query<8>, grid, dim3(BLOCK), 0, s, T, q, nq, k, idx, dist, count);
     else hipLaunchKernelGGL(k_entries_query<32>, grid, dim3(BLOCK), 0, s, T, q, nq, k, idx, dist, count);
-    return hipGetLastError();
-}
-
-hipError_t launch_trace(const DScene& S, const float* rays, uint32_t n, int anyHit, uint32_t* prim, float* t,
-                        float* u, float* v, uint32_t* occ, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_trace, dim3((n + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, s, S, rays, n, anyHit, prim, t, u, v,
-                       occ);
     return hipGetLastError();
 }
 

@@ -104,7 +104,7 @@ __device__ __forceinline__ ChunkRange chunk_range(uint32_t base, uint32_t n, uin
     const uint32_t share = n / (waves * 4u);
     c.base = base;
     c.lc = max(share < 1u ? 0u : min(31u - (uint32_t)__clz((int)share), TRACE_CHUNK_LOG2), minLog2);
-    const uint32_t nch = (n + (1u << c.lc) - 1u) >> c.lc;
+    const uint32_t nch = (n >> c.lc) + ((n & ((1u << c.lc) - 1u)) ? 1u : 0u);
     c.cnt = 0;
     if (w < nch) {
         const uint32_t mine = (nch - 1 - w) / waves + 1;
@@ -119,15 +119,62 @@ __device__ __forceinline__ uint32_t chunk_ray(const ChunkRange& c, uint32_t v, u
     return c.base + ((w + (v >> c.lc) * waves) << c.lc) + (v & ((1u << c.lc) - 1u));
 }
 
+// Where the traversal's rays come from and its answers go.  fetch: ray i as {origin, tmin},
+// {direction, tmax} and the place of its answer; store: the answer of a closest-hit ray or, any, of
+// a shadow ray.
+struct QueueRays {
+    const Queue& q;
+    const QIndex& qi;
+    const FinalArgs& F;
+    __device__ __forceinline__ uint32_t fetch(uint32_t i, float4& a, float4& b) const {
+        const uint32_t slot = in_slot(q, qi, i);
+        a = q.ray[slot];
+        b = q.ray[(size_t)q.cap + slot];
+        return slot;
+    }
+    __device__ __forceinline__ void store(uint32_t slot, bool any, const Hit& h) const {
+        const bool hit = h.prim != INVALID_PRIM;
+        if (!any || !final_answer(F, q.job[slot], hit))
+            q.res[slot] = any ? uint4{hit ? 1u : 0u, 0u, 0u, 0u}
+                              : uint4{h.prim, fb(hit ? h.t : 0.0f), fb(hit ? h.u : 0.0f), fb(hit ? h.v : 0.0f)};
+    }
+};
+
+// Rays of cx_trace_closest and cx_trace_occluded: [n][8] floats, at the caller's address, so the
+// 16-byte loads assume no more than a float's alignment.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+struct ArrayRays {
+    const float* rays;
+    uint32_t* prim;   // occlusion: the flags
+    float *t, *u, *v;
+    __device__ __forceinline__ uint32_t fetch(uint32_t i, float4& a, float4& b) const {
+        const f32x4u x = *(const f32x4u*)(rays + 8 * (size_t)i), y = *(const f32x4u*)(rays + 8 * (size_t)i + 4);
+        a = float4{x[0], x[1], x[2], y[2]};
+        b = float4{x[3], y[0], y[1], y[3]};
+        return i;
+    }
+    __device__ __forceinline__ void store(uint32_t i, bool any, const Hit& h) const {
+        const bool hit = h.prim != INVALID_PRIM;
+        if (any) {
+            prim[i] = hit ? 1u : 0u;
+            return;
+        }
+        prim[i] = h.prim;
+        t[i] = hit ? h.t : 0.0f;
+        u[i] = hit ? h.u : 0.0f;
+        v[i] = hit ? h.v : 0.0f;
+    }
+};
+
 // The wavefront's closest-hit chunks and then its shadow chunks as one sequence, so a lane whose
 // closest-hit ray is answered takes a shadow ray at the next refill instead of idling until its
 // wavefront has finished every closest-hit ray.  A lane's ray kind is a runtime flag: the two
 // kinds step through the same code, which differs only in the leaf's early exit and the result
 // written.
-template <int WIDTH, typename Stack>
-__device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, const QIndex& qi, uint32_t nc,
-                                             uint32_t ns, uint32_t w, uint32_t waves, uint32_t minLog2,
-                                             const FinalArgs& F, Stack& st) {
+template <int WIDTH, typename Rays, typename Stack>
+__device__ __forceinline__ void trace_chunks(const DScene& S, const Rays& rays, uint32_t nc, uint32_t ns, uint32_t w,
+                                             uint32_t waves, uint32_t minLog2, Stack& st) {
     const ChunkRange cc = chunk_range(0u, nc, w, waves, minLog2), cs = chunk_range(nc, ns, w, waves, minLog2);
     const uint32_t cnt = cc.cnt + cs.cnt;
     uint32_t cursor = 0;   // wavefront-uniform, counts this wavefront's rays
@@ -145,8 +192,8 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, 
                     if (v < cnt) {
                         any = v >= cc.cnt;
                         const uint32_t i = any ? chunk_ray(cs, v - cc.cnt, w, waves) : chunk_ray(cc, v, w, waves);
-                        slot = in_slot(qin, qi, i);
-                        const float4 a = qin.ray[slot], b = qin.ray[(size_t)qin.cap + slot];
+                        float4 a, b;
+                        slot = rays.fetch(i, a, b);
                         trav_init<WIDTH>(S, r, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w);
                         has = true;
                     }
@@ -159,11 +206,7 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Queue& qin, 
             continue;
         }
         if (trav_step_rt<WIDTH>(S, r, st, any)) {
-            const Hit& h = r.best;
-            const bool hit = h.prim != INVALID_PRIM;
-            if (!any || !final_answer(F, qin.job[slot], hit))
-                qin.res[slot] = any ? uint4{hit ? 1u : 0u, 0u, 0u, 0u}
-                                    : uint4{h.prim, fb(hit ? h.t : 0.0f), fb(hit ? h.u : 0.0f), fb(hit ? h.v : 0.0f)};
+            rays.store(slot, any, r.best);
             has = false;
         }
     }
@@ -177,23 +220,19 @@ static constexpr uint32_t QUAD_RAYS = 32;
 // Four lanes per ray (quad_trace): the queues of small images and of a machine's last rounds.  The
 // rays are spread over all wavefronts, so that as few as possible share a wavefront and wait for
 // each other's fetches.
-__device__ __forceinline__ void trace_quads(const DScene& S, const Queue& qin, const QIndex& qi, uint32_t nc,
-                                            uint32_t n, uint32_t w, uint32_t waves, const FinalArgs& F, int* lds) {
+template <typename Rays>
+__device__ __forceinline__ void trace_quads(const DScene& S, const Rays& rays, uint32_t nc, uint32_t n, uint32_t w,
+                                            uint32_t waves, int* lds) {
     const uint32_t per = (n + waves - 1) / waves, q = (threadIdx.x & 63u) >> 2;   // rays per wavefront
     for (uint32_t k = q; k < per; k += 16u) {
         const uint32_t i = w * per + k;
         if (i >= n) break;
         const bool any = i >= nc;
-        const uint32_t slot = in_slot(qin, qi, i);
-        const float4 a = qin.ray[slot], b = qin.ray[(size_t)qin.cap + slot];
+        float4 a, b;
+        const uint32_t slot = rays.fetch(i, a, b);
         Hit h;
         quad_trace(S, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w, any, h, lds + (threadIdx.x >> 2), WBLOCK / 4);
-        if ((threadIdx.x & 3u) == 0u) {
-            const bool hit = h.prim != INVALID_PRIM;
-            if (!any || !final_answer(F, qin.job[slot], hit))
-                qin.res[slot] = any ? uint4{hit ? 1u : 0u, 0u, 0u, 0u}
-                                    : uint4{h.prim, fb(hit ? h.t : 0.0f), fb(hit ? h.u : 0.0f), fb(hit ? h.v : 0.0f)};
-        }
+        if ((threadIdx.x & 3u) == 0u) rays.store(slot, any, h);
     }
 }
 
@@ -231,15 +270,57 @@ __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH ==
         }
     }
     const uint32_t waves = gridDim.x * (WBLOCK / 64), w = blockIdx.x * (WBLOCK / 64) + (threadIdx.x >> 6);
+    const QueueRays rays{qin, qi, F};
     if constexpr (WIDTH == 4) {
         if (nc + ns <= waves * QUAD_RAYS) {
-            trace_quads(S, qin, qi, nc, nc + ns, w, waves, F, s_st);
+            trace_quads(S, rays, nc, nc + ns, w, waves, s_st);
             return;
         }
     }
     int ovf[STACK_OVF<SHORT_STACK>];
     TravStack<SHORT_STACK, WBLOCK> st{s_st + threadIdx.x, ovf};
-    trace_chunks<WIDTH>(S, qin, qi, nc, ns, w, waves, minLog2, F, st);
+    trace_chunks<WIDTH>(S, rays, nc, ns, w, waves, minLog2, st);
+}
+
+// ---- traversal of a ray array (cx_trace_closest / cx_trace_occluded) ----
+//
+// Latency and VALU bound: a ray's chain of fetches and box tests.  With one thread per ray and all
+// widths in one kernel (136 registers, 32 KiB of stacks per block: 3 wavefronts per SIMD), each
+// wavefront waited for its slowest ray.  The frame's loop (rays refilled, 7 wavefronts at width 4)
+// takes 2 M closest-hit and occlusion rays on 1.06 M triangles from 1878 to 840 us; four lanes per
+// ray take 4096 rays on the Cornell box from 56 to 23 us.
+
+template <int WIDTH>
+__global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH == 8 ? 1 : (WIDTH == 4 ? 7 : 5), 8))) void k_trace_lanes(
+    DScene S, ArrayRays rays, uint32_t n, int any) {
+    __shared__ int s_st[SHORT_STACK * WBLOCK];
+    int ovf[STACK_OVF<SHORT_STACK>];
+    TravStack<SHORT_STACK, WBLOCK> st{s_st + threadIdx.x, ovf};
+    const uint32_t waves = gridDim.x * (WBLOCK / 64), w = blockIdx.x * (WBLOCK / 64) + (threadIdx.x >> 6);
+    trace_chunks<WIDTH>(S, rays, any ? 0u : n, any ? n : 0u, w, waves, 0u, st);
+}
+
+// One thread per ray, its whole stack in LDS: the rays that fit on the device at once, at widths 2
+// and 8 (trace_lanes_launch).
+template <int WIDTH, bool ANY>
+__global__ __launch_bounds__(WBLOCK) void k_trace_few(DScene S, ArrayRays rays, uint32_t n) {
+    static_assert(WBLOCK == TRACE_BLOCK, "the stack's column stride");
+    __shared__ int s_st[STACK_DEPTH * WBLOCK];
+    const uint32_t i = blockIdx.x * WBLOCK + threadIdx.x;
+    if (i >= n) return;
+    TravStack<STACK_DEPTH, WBLOCK> st{s_st + threadIdx.x, nullptr};
+    float4 a, b;
+    rays.fetch(i, a, b);
+    Hit h;
+    const bool hit = traverse_w<ANY, WIDTH>(S, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w, h, st);
+    if (ANY) h.prim = hit ? 0u : INVALID_PRIM;
+    rays.store(i, ANY, h);
+}
+
+__global__ __launch_bounds__(WBLOCK) void k_trace_quads(DScene S, ArrayRays rays, uint32_t n, int any) {
+    __shared__ int s_st[STACK_DEPTH * WBLOCK / 4];
+    const uint32_t waves = gridDim.x * (WBLOCK / 64), w = blockIdx.x * (WBLOCK / 64) + (threadIdx.x >> 6);
+    trace_quads(S, rays, any ? 0u : n, n, w, waves, s_st);
 }
 
 // Grid-stride loop over the jobs of qin whose bound is uniform per block, so every lane of a
@@ -1484,6 +1565,51 @@ static dim3 quad_grid(const Queue& q) {
 template <typename K>
 static dim3 range_grid(const Queue& q, K kernel) {
     return dim3(std::min(quad_grid(q).x, resident_blocks(kernel)));
+}
+
+// While all rays fit on the device there is nothing to refill, and the refill loop's own
+// instructions are on each ray's chain: width 8 on 271 k triangles takes 119 us (k_trace_few) and
+// 143 us (k_trace_lanes) for 1000 rays, 163 and 205 us for 100 k, 247 and 239 us for 200 k (164 k
+// fit).  The steps of width 2 are shorter and the loop's share of them larger: 100 k rays on 1.06 M
+// triangles take 276 and 388 us, 400 k on the Cornell box 145 and 162 us, 1 M 987 and 712 us on
+// 271 k triangles, so there the line is four times what fits.
+template <int WIDTH>
+static hipError_t trace_lanes_launch(const DScene& S, const ArrayRays& rays, uint32_t n, int any, hipStream_t s) {
+    if constexpr (WIDTH != 4) {
+        if (n <= (uint64_t)(WIDTH == 2 ? 4 : 1) * WBLOCK * resident_blocks(k_trace_few<WIDTH, false>)) {
+            const dim3 grid((n + WBLOCK - 1) / WBLOCK);
+            if (any) hipLaunchKernelGGL((k_trace_few<WIDTH, true>), grid, dim3(WBLOCK), 0, s, S, rays, n);
+            else hipLaunchKernelGGL((k_trace_few<WIDTH, false>), grid, dim3(WBLOCK), 0, s, S, rays, n);
+            return hipGetLastError();
+        }
+    }
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(((uint64_t)n + WBLOCK - 1) / WBLOCK,
+                                                         resident_blocks(k_trace_lanes<WIDTH>));
+    hipLaunchKernelGGL(k_trace_lanes<WIDTH>, dim3(blocks), dim3(WBLOCK), 0, s, S, rays, n, any);
+    return hipGetLastError();
+}
+
+hipError_t launch_trace(const DScene& S, const float* rays, uint32_t n, int anyHit, uint32_t* prim, float* t, float* u,
+                        float* v, hipStream_t s) {
+    if (n == 0) return hipSuccess;
+    const ArrayRays R{rays, prim, t, u, v};
+    // Width 4, four lanes per ray: up to one ray per quad of the resident wavefronts (16 each, 115 k
+    // rays), two per wavefront while there are few.  90 k rays take 46 us by quads and 49 us by
+    // lanes on the Cornell box, 145 and 224 us on 1.06 M triangles; 120 k take 67 and 49 us, 193 and
+    // 216 us, and 300 k the same on both.
+    constexpr uint32_t FEW_RAYS = 2, MOST_RAYS = 16;   // per wavefront
+    if (S.width == 4) {
+        const uint32_t blocks = resident_blocks(k_trace_quads), waves = blocks * (WBLOCK / 64);
+        if (n <= (uint64_t)waves * MOST_RAYS) {
+            constexpr uint32_t few = FEW_RAYS * (WBLOCK / 64);
+            const uint64_t want = ((uint64_t)n + few - 1) / few;
+            hipLaunchKernelGGL(k_trace_quads, dim3((uint32_t)std::min<uint64_t>(want, blocks)), dim3(WBLOCK), 0, s, S, R,
+                               n, anyHit);
+            return hipGetLastError();
+        }
+        return trace_lanes_launch<4>(S, R, n, anyHit, s);
+    }
+    return S.width == 8 ? trace_lanes_launch<8>(S, R, n, anyHit, s) : trace_lanes_launch<2>(S, R, n, anyHit, s);
 }
 
 // Where the final shadow rays of a machine leave their answers.

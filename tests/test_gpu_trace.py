@@ -205,3 +205,40 @@ def test_device_build_random_soups(seed, orc, cx_runtime, cx_ctx):
     for width in (2, 4, 8):
         gscene = cx_runtime.Scene(cx_ctx, sc, width=width, builder="device")
         _check_against_oracle(sc, gscene, oscene, rays, srays)
+
+
+@pytest.mark.parametrize("width", [2, 4, 8])
+def test_ray_counts_and_alignment(width, orc, cx_runtime, cx_ctx):
+    """Every split of the rays over the device gives the oracle's bits: counts at the edges of a
+    wavefront and a block, of one ray per quad, of the device's capacity (width 8: 164 k rays,
+    width 2: four times that) and beyond, with the rays at addresses that are aligned to 16 bytes
+    and to 4 bytes only."""
+    from crisoptix_amd.runtime import DeviceArray, lib, synchronize
+    sc = small_grid_scene()
+    gscene = cx_runtime.Scene(cx_ctx, sc, width=width)
+    assert gscene.info.bvhWidth == width
+    part = np.concatenate([random_rays(sc, 9000, seed=91), shadow_rays(sc, 2000, seed=92)])
+    part[5, 3:6] = 0.0        # no direction
+    part[6, 0] = np.nan
+    part[7, 3:5] = 0.0        # along an axis
+    part[8, 6] = -5.0         # from behind the origin
+    part[9, 6:8] = np.nan
+    part[10, 7] = -1.0        # an empty interval
+    part[11, 7] = np.inf
+    oscene = orc.OracleScene(sc)
+    ref, occ = oscene.trace_closest(part), oscene.trace_occluded(part)
+    most = 700_001
+    rays = np.resize(part, (most, 8))
+    for shift in (0, 1, 3):
+        dev = DeviceArray.from_numpy(np.concatenate([np.zeros(shift, np.float32), rays.ravel()]))
+        for n in (1, 2, 63, 65, 129, 4096, 114_688, 114_689, 163_841, most):
+            outs = [DeviceArray((n,), dt) for dt in (np.uint32, np.float32, np.float32, np.float32)]
+            flags = DeviceArray((n,), np.uint32)
+            cx_ctx.check(lib().cx_trace_closest(cx_ctx.h, gscene.h, dev.ptr + 4 * shift, n, *[o.ptr for o in outs], None),
+                         "cx_trace_closest")
+            cx_ctx.check(lib().cx_trace_occluded(cx_ctx.h, gscene.h, dev.ptr + 4 * shift, n, flags.ptr, None),
+                         "cx_trace_occluded")
+            synchronize()
+            for x, y in zip(ref, outs):
+                assert np.array_equal(np.resize(bits(x), n), bits(y.numpy())), (n, shift)
+            assert np.array_equal(np.resize(occ, n), flags.numpy()), (n, shift)
