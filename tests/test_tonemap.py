@@ -57,3 +57,25 @@ def test_gpu_tonemap_bit_exact(orc, cx_runtime, cx_ctx):
     d = cx_runtime.DeviceArray.from_numpy(c)
     got = cx_runtime.tonemap(cx_ctx, d)
     assert np.array_equal(got, orc.tonemap(c))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 1023, 1024, 1025, 300_001])
+def test_gpu_tonemap_sizes_and_alignment(n, shift, orc, cx_runtime, cx_ctx):
+    """Output words cut at either end (the bytes beyond them stay as they are), input and output at
+    any alignment that their types allow, values on both sides of every step of the bytes."""
+    from crisoptix_amd.runtime import DeviceArray, lib, synchronize
+    steps = (((np.arange(1, 256) / 255.0 + 0.055) / 1.055) ** 2.4).astype(np.float32)
+    ulps = steps.view(np.int32)[:, None] + np.arange(-40, 41, dtype=np.int32)
+    special = np.array([0.0, -0.0, -1.0, np.nan, np.inf, -np.inf, 1.0, 1.001, 0.0031308, 3e37, 1e-45, 3.4e38, 12.0],
+                       np.float32)
+    c = np.resize(np.concatenate([special, ulps.view(np.float32).ravel(),
+                                  np.random.default_rng(5).random(9000, np.float32) * 1.1]), n)
+    hdr = DeviceArray.from_numpy(np.concatenate([np.zeros(shift, np.float32), c]))
+    ldr = DeviceArray.from_numpy(np.full(n + 16, 0xA5, np.uint8))
+    cx_ctx.check(lib().cx_tonemap(cx_ctx.h, hdr.ptr + 4 * shift, ldr.ptr + 4 + shift, n, None), "cx_tonemap")
+    synchronize()
+    got = ldr.numpy()
+    assert np.array_equal(got[4 + shift:4 + shift + n], orc.tonemap(c))
+    assert np.all(got[:4 + shift] == 0xA5) and np.all(got[4 + shift + n:] == 0xA5)
