@@ -634,33 +634,55 @@ __device__ __forceinline__ void grow_box(float4& lo, float4& hi, float4 l2, floa
     hi = float4{fmaxf(hi.x, h2.x), fmaxf(hi.y, h2.y), fmaxf(hi.z, h2.z), 0.0f};
 }
 
-// Levels of the range tree over the valid entries.
-__global__ void k_seg_prep(EntryTree T) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *T.segLevels = entry_seg_levels(*T.numValid);
-}
+// Range tree over the sorted entries, SEG_UP levels per launch: the block's SEG_BLOCK nodes of one
+// level are reduced upwards in LDS.  Bound by its launches: 547 k entries take 18 levels, 3 launches
+// (one per level took 77 us).
+static constexpr uint32_t SEG_BLOCK = 256;
+static constexpr uint32_t SEG_UP = 8;
+static_assert(SEG_BLOCK == 1u << SEG_UP, "a block ends in one node");
 
-// Range-tree leaf j: sorted entries [8j, 8j + 8) that are valid (an empty leaf keeps an empty box).
-__global__ void k_seg_leaves(EntryTree T, uint32_t leavesCap) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t leaves = 1u << *T.segLevels;
-    if (j >= leavesCap || j >= leaves) return;
-    const uint32_t n = *T.numValid;
+// below = 0: the leaves, leaf j holding the sorted entries [8j, 8j + 8) that are valid (an empty leaf
+// keeps an empty box), and the SEG_UP levels above them; below > 0: the SEG_UP levels above the
+// level that lies `below` levels over the leaves.
+__global__ __launch_bounds__(SEG_BLOCK) void k_seg_levels(EntryTree T, uint32_t below) {
+    __shared__ float4 s_lo[SEG_BLOCK], s_hi[SEG_BLOCK];
+    const uint32_t n = *T.numValid, levels = entry_seg_levels(n);
+    if (below == 0u && blockIdx.x == 0u && threadIdx.x == 0u) *T.segLevels = levels;
+    if (below > levels) return;
+    uint32_t level = levels - below;
+    const uint32_t first = blockIdx.x * SEG_BLOCK;
+    if (first >= (1u << level)) return;   // the whole block
+    uint32_t here = min(SEG_BLOCK, 1u << level);   // the block's nodes of this level
+    const uint32_t t = threadIdx.x;
     float4 lo = float4{INFINITY, INFINITY, INFINITY, -INFINITY}, hi = float4{-INFINITY, -INFINITY, -INFINITY, 0.0f};
-    const uint32_t b = j * ENTRY_SEG_LEAF, e = min(b + ENTRY_SEG_LEAF, n);
-    for (uint32_t i = b; i < e; i++) grow_entry(lo, hi, T.entrySorted[i]);
-    T.segLo[leaves - 1u + j] = lo;
-    T.segHi[leaves - 1u + j] = hi;
-}
-
-// Range-tree nodes of level l (heap indices [2^l - 1, 2^(l+1) - 1)) above the leaf level.
-__global__ void k_seg_level(EntryTree T, uint32_t level, uint32_t count) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= count || level >= *T.segLevels) return;
-    const uint32_t node = (1u << level) - 1u + j;
-    float4 lo = T.segLo[2 * node + 1], hi = T.segHi[2 * node + 1];
-    grow_box(lo, hi, T.segLo[2 * node + 2], T.segHi[2 * node + 2]);
-    T.segLo[node] = lo;
-    T.segHi[node] = hi;
+    if (t < here) {
+        const uint32_t node = (1u << level) - 1u + first + t;
+        if (below == 0u) {
+            const uint32_t b = min((first + t) * ENTRY_SEG_LEAF, n), e = min(b + ENTRY_SEG_LEAF, n);
+            for (uint32_t i = b; i < e; i++) grow_entry(lo, hi, T.entrySorted[i]);
+            T.segLo[node] = lo;
+            T.segHi[node] = hi;
+        } else {
+            lo = T.segLo[node];
+            hi = T.segHi[node];
+        }
+    }
+    for (uint32_t up = 1; up <= SEG_UP && level > 0u; up++) {
+        s_lo[t] = lo;
+        s_hi[t] = hi;
+        __syncthreads();
+        here >>= 1;
+        level--;
+        if (t < here) {
+            lo = s_lo[2 * t];
+            hi = s_hi[2 * t];
+            grow_box(lo, hi, s_lo[2 * t + 1], s_hi[2 * t + 1]);
+            const uint32_t node = (1u << level) - 1u + (first >> up) + t;
+            T.segLo[node] = lo;
+            T.segHi[node] = hi;
+        }
+        __syncthreads();
+    }
 }
 
 // Bounds (and largest radius) of the sorted entries [a, b], b >= a: short ranges are scanned;
@@ -732,21 +754,31 @@ __global__ void k_lbvh_nodes(EntryTree T) {
     nd[3] = float4{hi1.x, hi1.y, hi1.z, __int_as_float(refR)};
 }
 
+// One thread per query.  Bound by the latency of the walk's dependent fetches, so by the wavefronts
+// in flight: ENTRY_QUERY_SHORT deferred siblings per thread in LDS (8 KiB per block) leave room for
+// seven per SIMD; with the whole stack there (32 KiB) it was two to three.  547 k queries in random
+// order among 736 k entries, k = 8: 963 us before, 540 us now (of them 130 us by the limits, keys and
+// fetches of entries_query; without those, k = 31 takes 808 instead of 381 us for 7800 queries).
+static constexpr int ENTRY_QUERY_SHORT = 8;
+
 template <int KR>
-__global__ __launch_bounds__(BLOCK) void k_entries_query(EntryTree T, const float* q, uint32_t nq, uint32_t k,
-                                                        uint32_t* idx, float* dist, uint32_t* count) {
-    __shared__ int s_stack[STACK_DEPTH * BLOCK];
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(KR <= 8 ? 7 : 1, 8))) void k_entries_query(
+    EntryTree T, const float* q, uint32_t nq, uint32_t k, uint32_t* idx, float* dist, uint32_t* count) {
+    __shared__ int s_stack[2 * ENTRY_QUERY_SHORT * BLOCK];
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nq) return;
-    for (uint32_t i = 0; i < k; i++) {
-        idx[(size_t)j * k + i] = 0xFFFFFFFFu;
-        dist[(size_t)j * k + i] = 0.0f;
-    }
-    QueryStack<STACK_DEPTH / 2> st;
+    QueryStack<ENTRY_QUERY_SHORT> st;
     st.lds = s_stack + threadIdx.x;
     st.stride = BLOCK;
-    count[j] = entries_query<KR>(T, V3{q[3 * j], q[3 * j + 1], q[3 * j + 2]}, k, st, idx + (size_t)j * k,
-                                 dist + (size_t)j * k);
+    uint32_t* const jIdx = idx + (size_t)j * k;
+    float* const jDist = dist + (size_t)j * k;
+    const uint32_t found = entries_query<KR>(T, V3{q[3 * (size_t)j], q[3 * (size_t)j + 1], q[3 * (size_t)j + 2]}, k, st,
+                                             jIdx, jDist);
+    for (uint32_t i = found; i < k; i++) {
+        jIdx[i] = 0xFFFFFFFFu;
+        jDist[i] = 0.0f;
+    }
+    count[j] = found;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1048,8 +1080,7 @@ hipError_t launch_key_sort(uint32_t* keys, uint32_t* vals, uint32_t* keysAlt, ui
 }
 
 // Sorts the valid entries by Morton key and builds the LBVH over them: the sorted slots, the
-// range tree (one launch per level; levels above the valid entries' tree return at once), then
-// every internal node at once.  Grids cover the capacity n; kernels read the valid count on the
+// range tree, then every internal node at once.  Grids cover the capacity n; kernels read the valid count on the
 // device.
 hipError_t launch_tree_build(const EntryBuild& E, const EntryTree& T, uint32_t n, void* temp, size_t tempBytes,
                              hipStream_t s) {
@@ -1058,12 +1089,10 @@ hipError_t launch_tree_build(const EntryBuild& E, const EntryTree& T, uint32_t n
     if (e != hipSuccess) return e;
     const dim3 g((n + 255) / 256), b(256);
     hipLaunchKernelGGL(k_lbvh_slots, g, b, 0, s, T, E.vals, E.pos);
-    hipLaunchKernelGGL(k_seg_prep, dim3(1), dim3(64), 0, s, T);
-    const uint32_t leavesCap = 1u << T.segLevelsCap;
-    hipLaunchKernelGGL(k_seg_leaves, dim3((leavesCap + 255) / 256), b, 0, s, T, leavesCap);
-    for (int l = (int)T.segLevelsCap - 1; l >= 0; l--) {
-        const uint32_t cnt = 1u << l;
-        hipLaunchKernelGGL(k_seg_level, dim3((cnt + 255) / 256), b, 0, s, T, (uint32_t)l, cnt);
+    // grids for the capacity's levels; the valid entries' tree has no more
+    for (uint32_t below = 0; below == 0u || below < T.segLevelsCap; below += SEG_UP) {
+        const uint32_t nodes = 1u << (T.segLevelsCap - below);
+        hipLaunchKernelGGL(k_seg_levels, dim3((nodes + SEG_BLOCK - 1) / SEG_BLOCK), dim3(SEG_BLOCK), 0, s, T, below);
     }
     hipLaunchKernelGGL(k_lbvh_nodes, g, b, 0, s, T);
     return hipGetLastError();

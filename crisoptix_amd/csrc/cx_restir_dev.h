@@ -613,52 +613,49 @@ __device__ __forceinline__ bool trace_prefix_fg(const FrameArgs& A, TraceCtx& tc
 // ---- neighbour search over the entry tree ----
 
 // Neighbour query under C2: every entry with |q - pos| <= r is a candidate; the k smallest
-// (distance, index) are kept in ascending order.  Up to KR candidates live in registers.
+// (distance, index) are kept in ascending order, in registers (k <= KR), as the bits of the distance
+// above the index: as doubles, such keys of distances >= 0 compare by distance, then index, and an
+// insertion is one maximum and one minimum per slot (five instructions as separate arrays with a
+// tie test).  The KR - k slots in front hold a key below all others, so the k-th smallest is always
+// in the last slot.
 template <int KR>
 struct TopK {
-    float d[KR];
-    uint32_t i[KR];
+    double key[KR];
     uint32_t count;
-    __device__ __forceinline__ void init() {
+    __device__ __forceinline__ void init(uint32_t k) {
 #pragma unroll
-        for (int j = 0; j < KR; j++) {
-            d[j] = INFINITY;
-            i[j] = 0xFFFFFFFFu;
-        }
+        for (int j = 0; j < KR; j++) key[j] = (uint32_t)j + k < (uint32_t)KR ? -1.0 : hit_key(INFINITY, -1);
         count = 0;
     }
-    __device__ __forceinline__ static bool less(float da, uint32_t ia, float db, uint32_t ib) {
-        return da < db || (da == db && ia < ib);
-    }
-    // Sorted insertion; a candidate not smaller than the k-th entry changes nothing.
+    // A candidate not smaller than the k-th entry changes nothing.
     __device__ __forceinline__ void insert(float cd, uint32_t ci, uint32_t k) {
+        const double c = hit_key(cd, (int)ci);
 #pragma unroll
-        for (int j = KR - 1; j >= 0; j--) {
-            if ((uint32_t)j >= k) continue;
-            if (less(cd, ci, d[j], i[j])) {
-                if (j > 0 && less(cd, ci, d[j - 1], i[j - 1])) {
-                    d[j] = d[j - 1];
-                    i[j] = i[j - 1];
-                } else {
-                    d[j] = cd;
-                    i[j] = ci;
-                }
-            }
-        }
+        for (int j = KR - 1; j > 0; j--) key[j] = key_min(key_max(c, key[j - 1]), key[j]);
+        key[0] = key_min(c, key[0]);
         if (count < k) count++;
+    }
+    // The k-th smallest distance, infinite while fewer are held.
+    __device__ __forceinline__ float kth() const {
+        return __builtin_bit_cast(float, __builtin_bit_cast(u32x2, key[KR - 1]).y);
     }
 };
 
-// Lower bound of distance(q, p) over the positions p inside [lo, hi]: per axis the gap to the
-// box (0 inside), squared and summed in the order length() uses.  Float subtraction, squaring,
-// addition and sqrt are monotone, and the bounds are exact entry coordinates, so the bound never
-// exceeds the float distance the leaf test computes for any entry of the node.
-__device__ __forceinline__ float box_distance(V3 q, float4 lo, float4 hi) {
+// Lower bound of the squared distance of q to the positions p inside [lo, hi]: per axis the gap to
+// the box (0 inside), squared and summed in the order distance() uses.  Float subtraction,
+// squaring and addition are monotone, and the bounds are exact entry coordinates, so the bound
+// never exceeds the sum under distance()'s root for any entry of the node.
+__device__ __forceinline__ float box_distance2(V3 q, float4 lo, float4 hi) {
     const float dx = q.x < lo.x ? lo.x - q.x : (q.x > hi.x ? q.x - hi.x : 0.0f);
     const float dy = q.y < lo.y ? lo.y - q.y : (q.y > hi.y ? q.y - hi.y : 0.0f);
     const float dz = q.z < lo.z ? lo.z - q.z : (q.z > hi.z ? q.z - hi.z : 0.0f);
-    return sqrtf(dx * dx + dy * dy + dz * dz);
+    return dx * dx + dy * dy + dz * dz;
 }
+
+// A number that no squared distance whose rounded root is at most d exceeds: the root, the square
+// and the sum of roundings are within 2^-22 of d^2, or within the smallest normal number where
+// d^2 underflows.  Infinite for a d whose square overflows, NaN for NaN.
+__device__ __forceinline__ float square_limit(float d) { return d * d * 1.000001f + 2e-38f; }
 
 // Deferred siblings of the entry query: (child reference, its distance bound).  The first SHORT
 // entries live in a per-thread LDS column (two ints per entry, lds[(2 i) * stride] and
@@ -692,27 +689,38 @@ struct QueryStack {
 // of its positions is within the largest radius of its entries (only then can one of them have
 // |q - p| <= r) and, once k candidates are held, within the k-th distance (an entry farther than
 // that cannot enter the set; one at exactly that distance can, through the index tie-break).
+// Both tests compare squares against limits rounded up (square_limit), so they keep every child
+// and entry that the distances would; an entry that passes is tested by its distance.
 // The nearer child (by that bound) is visited first, the other deferred with its bound and
 // dropped when it is popped if the k-th distance found since has passed it.  The set found is
 // the same as with an exhaustive visit of all candidates.
 template <int KR, typename Stack>
 __device__ __forceinline__ uint32_t entries_query(const EntryTree& T, V3 q, uint32_t k, Stack& st, uint32_t* outIdx,
                                                   float* outDist) {
-    TopK<KR> top;
-    top.init();
     const uint32_t n = *T.numValid;
     if (k == 0 || n == 0 || isnan(q.x) || isnan(q.y) || isnan(q.z)) return 0;
-    float kth = INFINITY;   // k-th smallest distance once k candidates are held
+    TopK<KR> top;
+    top.init(k);
+    float kth2 = INFINITY;   // square_limit of the k-th smallest distance
+    // four entries are fetched at a time (the last one again beyond the end), so a leaf is two waits
     auto scan = [&](uint32_t first, uint32_t cnt) {
-        for (uint32_t s = first; s < first + cnt; s++) {
-            const float4 ep = T.entrySorted[s];
-            const float dd = distance(q, V3{ep.x, ep.y, ep.z});
-            if (!(dd <= ep.w) || dd > kth) continue;   // a NaN distance or radius is no candidate
-            top.insert(dd, T.entryPixel[s], k);
-            if (top.count == k) {
+        const uint32_t end = first + cnt, last = end - 1u;
+        for (uint32_t s = first; s < end; s += 4u) {
+            float4 ep[4];
+            uint32_t pixel[4];
 #pragma unroll
-                for (int m = 0; m < KR; m++)
-                    if ((uint32_t)m + 1u == k) kth = top.d[m];
+            for (uint32_t j = 0; j < 4u; j++) {
+                ep[j] = T.entrySorted[min(s + j, last)];
+                pixel[j] = T.entryPixel[min(s + j, last)];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; j++) {
+                const V3 w = V3{ep[j].x, ep[j].y, ep[j].z} - q;
+                if (s + j >= end || dot(w, w) > fminf(square_limit(ep[j].w), kth2)) continue;
+                const float dd = distance(q, V3{ep[j].x, ep[j].y, ep[j].z});
+                if (!(dd <= ep[j].w) || dd > top.kth()) continue;   // a NaN distance or radius is no candidate
+                top.insert(dd, pixel[j], k);
+                kth2 = square_limit(top.kth());
             }
         }
     };
@@ -725,8 +733,8 @@ __device__ __forceinline__ uint32_t entries_query(const EntryTree& T, V3 q, uint
             if (ref >= 0) {
                 const float4* nd = T.nodes + 4 * (size_t)ref;
                 const float4 lo0 = nd[0], hi0 = nd[1], lo1 = nd[2], hi1 = nd[3];
-                const float b0 = box_distance(q, lo0, hi0), b1 = box_distance(q, lo1, hi1);
-                const bool ok0 = b0 <= lo0.w && b0 <= kth, ok1 = b1 <= lo1.w && b1 <= kth;
+                const float b0 = box_distance2(q, lo0, hi0), b1 = box_distance2(q, lo1, hi1);
+                const bool ok0 = b0 <= square_limit(lo0.w) && b0 <= kth2, ok1 = b1 <= square_limit(lo1.w) && b1 <= kth2;
                 const int r0 = __float_as_int(hi0.w), r1 = __float_as_int(hi1.w);
                 if (ok0 && ok1) {
                     const bool near0 = b0 <= b1;
@@ -748,16 +756,18 @@ __device__ __forceinline__ uint32_t entries_query(const EntryTree& T, V3 q, uint
                 --sp;
                 float b;
                 st.get(sp, ref, b);
-                found = b <= kth;
+                found = b <= kth2;
             }
             if (!found) break;
         }
     }
 #pragma unroll
     for (int j = 0; j < KR; j++) {
-        if ((uint32_t)j < top.count) {
-            outIdx[j] = top.i[j];
-            outDist[j] = top.d[j];
+        const uint32_t m = (uint32_t)j - (KR - k);   // beyond count in the slots in front
+        if (m < top.count) {
+            const u32x2 b = __builtin_bit_cast(u32x2, top.key[j]);
+            outIdx[m] = b.x;
+            outDist[m] = __builtin_bit_cast(float, (uint32_t)b.y);
         }
     }
     return top.count;

@@ -312,21 +312,31 @@ CX_HD bool key_miss(double k) {
     return b.y == 0x7f800000u;
 }
 
-CX_HD void key_cswap(double& a, double& b) {
+// The instructions themselves on the device: fmin and fmax would quiet their operands first.
+CX_HD double key_min(double a, double b) {
 #ifdef __HIP_DEVICE_COMPILE__
-    // the instructions themselves: fmin and fmax would quiet their operands first
-    double lo, hi;
-    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
-    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return b < a ? b : a;
+#endif
+}
+
+CX_HD double key_max(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return b < a ? a : b;
+#endif
+}
+
+CX_HD void key_cswap(double& a, double& b) {
+    const double lo = key_min(a, b), hi = key_max(a, b);
     a = lo;
     b = hi;
-#else
-    if (b < a) {
-        const double t = a;
-        a = b;
-        b = t;
-    }
-#endif
 }
 
 // One wide node (2 N float4 per node, the 8th of each group of 4 children unused): test the N

@@ -1140,7 +1140,7 @@ __device__ __forceinline__ uint32_t gather_total(const WaveArgs& W) { return *W.
 // more waves per SIMD; its deferred siblings take GATHER_QUERY_SHORT stack entries of LDS per
 // thread (dynamic shared memory, gather_query_lds bytes).
 template <int KR>
-__global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(KR <= 8 ? 8 : 1, 8))) void k_w_gather_query(
+__global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(KR <= 8 ? 7 : 1, 8))) void k_w_gather_query(
     WaveArgs W) {
     extern __shared__ int s_st[];
     const FrameArgs& A = W.A;

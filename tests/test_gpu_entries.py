@@ -59,3 +59,42 @@ def test_empty_and_all_invalid(cx_runtime, cx_ctx):
     E.build(pos, np.ones(10, np.float32), np.zeros(10, np.uint8), np.zeros(3), np.ones(3))
     _, _, c = E.query(np.zeros((5, 3), np.float32), 4)
     assert (c == 0).all()
+
+
+@pytest.mark.parametrize("n", [1, 8, 9, 17, 2048, 2049, 4097, 300_000])
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 31])
+def test_sizes_ties_and_extremes(n, k, orc, cx_runtime, cx_ctx):
+    """Entry counts at the edges of a leaf, of the range tree's levels per launch (2048 entries are
+    256 groups) and of the kernel's k; ties (equal positions, queries on entries: distance zero),
+    distances whose squares underflow, infinite, zero, negative and NaN radii, non-finite queries.
+    Slots beyond a query's count hold the index 0xFFFFFFFF and the distance 0."""
+    pos, radius, _, q = make_entries(max(n, 64), seed=n + k)
+    pos, radius, q = pos[:n], radius[:n], np.resize(q, (256, 3))
+    rng = np.random.default_rng(n * 100 + k)
+    same = rng.integers(0, n, n // 4)
+    pos[rng.integers(0, n, n // 4)] = pos[same]                          # ties by index
+    near = rng.integers(0, n, n // 8)
+    pos[near] = (rng.choice([0.0, 1e-20, 3e-23, 1e-30, 1e-38], (len(near), 3))).astype(np.float32)
+    radius[rng.integers(0, n, n // 10)] = np.inf
+    radius[rng.integers(0, n, n // 10)] = 0.0
+    radius[rng.integers(0, n, n // 10)] = 1e-22
+    radius[rng.integers(0, n, n // 20)] = -1.0
+    radius[rng.integers(0, n, n // 20)] = np.nan
+    q[:64] = pos[rng.integers(0, n, 64)]
+    q[64:96] = rng.choice([0.0, 1e-20, 2e-23, 1e-38], (32, 3))
+    q[96:104] = np.array([1e30, -1e25, 1e19])
+    q[104] = np.inf
+    q[105] = np.nan
+    valid = np.ones(n, np.uint8)
+    # a NaN radius or query is no candidate on the device; the oracle is asked without them
+    io, do, co = orc.entries_query(pos, np.nan_to_num(radius, nan=0.0, posinf=np.inf),
+                                   (~np.isnan(radius)).astype(np.uint8), np.nan_to_num(q, posinf=np.inf), k, brute=True)
+    co[np.isnan(q).any(1)] = 0
+    E = cx_runtime.Entries(cx_ctx, n)
+    E.build(pos, radius, valid, pos.min(0), pos.max(0))
+    ig, dg, cg = E.query(q, k)
+    assert np.array_equal(co, cg), np.nonzero(co != cg)
+    held = np.arange(k)[None, :] < co[:, None]
+    assert np.array_equal(io[held], ig[held])
+    assert np.array_equal(do[held].view(np.uint32), dg[held].view(np.uint32))
+    assert np.all(ig[~held] == 0xFFFFFFFF) and np.all(dg[~held].view(np.uint32) == 0)
