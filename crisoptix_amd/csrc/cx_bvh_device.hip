@@ -22,7 +22,7 @@
 //     cost(node) = min(area * triangles  [if triangles <= maxLeaf], 2 * area + cost(l) + cost(r)),
 //     the host build's traversal-to-intersection cost ratio of 2;
 //   * the top-down pass (triangle slots, kept inner nodes, depths) runs one launch per
-//     iteration in reverse creation order, with no inter-thread synchronisation inside a kernel.
+//     iteration in reverse creation order, the iterations of few nodes in one block.
 // Every step is deterministic (scans, no ordering by atomics).  Child boxes are padded outward by
 // |coord| * 2^-15 when the node arrays are written, as in the host build.
 #include <algorithm>
@@ -249,21 +249,70 @@ __global__ __launch_bounds__(BB) void k_ploc_init(const uint32_t* vals, const fl
     clusters[s] = s;
 }
 
-// nn[i] = the position j != i within PLOC_RADIUS whose merged box with i has the smallest
-// area, ties to the smaller (|i - j|, min(i, j) odd, min(i, j)); i itself when there is none.
 // Device state of the clustering: the current cluster count, the inner nodes made so far, the
 // iterations run, and a flag for an iteration that merged nothing.
 struct PlocState {
     uint32_t m, nodeCount, iters, stalled;
 };
 
+// The position j != i within PLOC_RADIUS whose merged box with i has the smallest area, ties to the
+// smaller (|i - j|, min(i, j) odd, min(i, j)); i itself when there is none.  The boxes lie in LDS,
+// cluster i's at index `at` of size entries; L neighbouring lanes (sub = 0 .. L - 1) take every L-th
+// distance each and agree on the result.  A lane meets its pairs in the order of the tie rule, so
+// a strict comparison keeps the first of equals (and the first pair if all areas are infinite).
+__device__ __forceinline__ int ploc_nearest(const float4* s_lo, const float4* s_hi, int at, int size, int i, int m,
+                                            int sub, int L) {
+    const float4 lo = s_lo[at], hi = s_hi[at];
+    float best = INFINITY;
+    int bestJ = i;
+    auto take = [&](int j) {
+        const int k = min(max(at + j - i, 0), size - 1);
+        const float a = box_area(min4(lo, s_lo[k]), max4(hi, s_hi[k]));
+        if (j >= 0 && j < m && (a < best || (a == best && bestJ == i))) {
+            best = a;
+            bestJ = j;
+        }
+    };
+    for (int d = 1 + sub; d <= PLOC_RADIUS; d += L) {
+        // the pairs' lower positions are i - d and i: the even one first, then the lower
+        const int first = ((i - d) & 1) && !(i & 1) ? d : -d;
+        take(i + first);
+        take(i - first);
+    }
+    auto key = [&](int j) -> unsigned long long {
+        const uint32_t l = (uint32_t)min(i, j);
+        return j == i ? ~0ull
+                      : ((unsigned long long)(uint32_t)abs(j - i) << 33) | ((unsigned long long)(l & 1u) << 32) | l;
+    };
+    for (int off = 1; off < L; off <<= 1) {
+        const float ob = __shfl_xor(best, off, 64);
+        const int oj = __shfl_xor(bestJ, off, 64);
+        if (ob < best || (ob == best && key(oj) < key(bestJ))) {
+            best = ob;
+            bestJ = oj;
+        }
+    }
+    return bestJ;
+}
+
+// Clusters that one block takes to the root (k_ploc_tail); the kernels of a whole iteration leave
+// such a state alone.
+constexpr uint32_t PLOC_TAIL = 1024;
+
+// nn[i] of every cluster, L lanes per cluster.  Bound by its 128 box areas per cluster, read from
+// LDS (1.06 M clusters: 200 us): one lane per cluster while the clusters fill the device, eight below
+// PLOC_LANES_MAX, where one lane's chain of 128 was the time (33 us per iteration, 10 us now).
+constexpr uint32_t PLOC_LANES_MAX = 1u << 18;
+
+template <int L>
 __global__ __launch_bounds__(BB) void k_ploc_nn(const uint32_t* clusters, const PlocState* st, const float4* nlo,
                                                 const float4* nhi, uint32_t* nn) {
+    constexpr int C = BB / L;   // clusters per block
     const uint32_t m = st->m;
-    if (m <= 1 || blockIdx.x * BB >= m) return;   // finished, or a block past the clusters
-    constexpr int W = BB + 2 * PLOC_RADIUS;
+    if (m <= PLOC_TAIL || blockIdx.x * C >= m) return;   // left to the tail, or a block past the clusters
+    constexpr int W = C + 2 * PLOC_RADIUS;
     __shared__ float4 s_lo[W], s_hi[W];
-    const int base = (int)(blockIdx.x * BB) - PLOC_RADIUS;
+    const int base = (int)(blockIdx.x * C) - PLOC_RADIUS;
     for (int k = threadIdx.x; k < W; k += BB) {
         const int j = base + k;
         if (j >= 0 && j < (int)m) {
@@ -273,34 +322,18 @@ __global__ __launch_bounds__(BB) void k_ploc_nn(const uint32_t* clusters, const 
         }
     }
     __syncthreads();
-    const int i = (int)(blockIdx.x * BB + threadIdx.x);
-    if (i >= (int)m) return;
-    const float4 lo = s_lo[threadIdx.x + PLOC_RADIUS], hi = s_hi[threadIdx.x + PLOC_RADIUS];
-    float best = INFINITY;
-    unsigned long long bestKey = ~0ull;
-    int bestJ = i;
-    for (int d = -PLOC_RADIUS; d <= PLOC_RADIUS; d++) {
-        const int j = i + d;
-        if (d == 0 || j < 0 || j >= (int)m) continue;
-        const int k = threadIdx.x + PLOC_RADIUS + d;
-        const float a = box_area(min4(lo, s_lo[k]), max4(hi, s_hi[k]));
-        const uint32_t lo = (uint32_t)min(i, j);
-        const unsigned long long key = ((unsigned long long)(uint32_t)abs(d) << 33) |
-                                       ((unsigned long long)(lo & 1u) << 32) | (unsigned long long)lo;
-        if (a < best || (a == best && key < bestKey)) {
-            best = a;
-            bestKey = key;
-            bestJ = j;
-        }
-    }
-    nn[i] = (uint32_t)bestJ;
+    const int c = (int)threadIdx.x / L, sub = (int)threadIdx.x % L;
+    const int i = (int)(blockIdx.x * C) + c;
+    if (i >= (int)m) return;   // all lanes of the cluster
+    const int j = ploc_nearest(s_lo, s_hi, c + PLOC_RADIUS, W, i, (int)m, sub, L);
+    if (sub == 0) nn[i] = (uint32_t)j;
 }
 
 // flags[i] = (cluster i survives, cluster i creates a node): mutual nearest neighbours merge
 // at the lower position.
 __global__ __launch_bounds__(BB) void k_ploc_flags(const uint32_t* nn, const PlocState* st, uint2* flags) {
     const uint32_t m = st->m, i = tid();
-    if (m <= 1 || i >= m) return;
+    if (m <= PLOC_TAIL || i >= m) return;
     const uint32_t j = nn[i];
     const bool mutual = j != i && nn[j] == i;
     flags[i] = make_uint2(mutual && i > j ? 0u : 1u, mutual && i < j ? 1u : 0u);
@@ -312,7 +345,7 @@ __global__ __launch_bounds__(BB) void k_ploc_merge(const uint32_t* cin, uint32_t
                                                    uint32_t maxLeaf, float4* nlo, float4* nhi, uint2* kids,
                                                    uint32_t* cnt, float* cost, uint32_t* leafOK) {
     const uint32_t m = st->m, nodeBase = st->nodeCount, i = tid();
-    if (m <= 1 || i >= m) return;
+    if (m <= PLOC_TAIL || i >= m) return;
     const uint32_t j = nn[i];
     const bool mutual = j != i && nn[j] == i;
     if (mutual && i > j) return;   // merged into the node its partner creates
@@ -339,10 +372,10 @@ __global__ __launch_bounds__(BB) void k_ploc_merge(const uint32_t* cin, uint32_t
 }
 
 // Ends an iteration: the scan's totals give the surviving clusters and the new nodes; the node
-// count after it goes to iterEnd[iteration].  No-op once one cluster is left or after a stall.
+// count after it goes to iterEnd[iteration].  No-op once the tail's count is reached or after a stall.
 __global__ void k_ploc_advance(PlocState* st, const uint2* total, uint32_t* iterEnd, uint32_t iterCap) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    if (st->m <= 1 || st->stalled) return;
+    if (st->m <= PLOC_TAIL || st->stalled) return;
     const uint2 t = *total;
     if (t.y == 0 || t.x + t.y != st->m || st->iters >= iterCap) {
         st->stalled = 1u;
@@ -354,6 +387,118 @@ __global__ void k_ploc_advance(PlocState* st, const uint2* total, uint32_t* iter
     st->iters += 1u;
 }
 
+// The last iterations in one block, from PLOC_TAIL clusters or fewer to the root: the clusters stay
+// in LDS, and the threads that the clusters leave free share the search (up to 16 lanes per
+// cluster).  Latency bound: half of an 1.06 M-triangle scene's 76 iterations ran here on a few
+// blocks, seven launches each (75 us per iteration, 11 us
+// now).  The clusters are in cA after an even
+// number of iterations, in cB after an odd one.  Every iteration merges or ends the loop.
+__global__ __launch_bounds__(PLOC_TAIL) void k_ploc_tail(PlocState* st, const uint32_t* cA, const uint32_t* cB,
+                                                         uint32_t n, uint32_t maxLeaf, float4* nlo, float4* nhi,
+                                                         uint2* kids, uint32_t* cnt, float* cost, uint32_t* leafOK,
+                                                         uint32_t* iterEnd, uint32_t iterCap) {
+    __shared__ float4 s_lo[PLOC_TAIL], s_hi[PLOC_TAIL];
+    __shared__ uint32_t s_id[PLOC_TAIL], s_cnt[PLOC_TAIL], s_nn[PLOC_TAIL];
+    __shared__ float s_cost[PLOC_TAIL];
+    __shared__ uint32_t s_w[PLOC_TAIL / 64];
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    uint32_t m = st->m, nodeCount = st->nodeCount, iters = st->iters;
+    bool stalled = st->stalled != 0u;
+    if (m <= 1u || m > PLOC_TAIL || stalled) return;
+    if (t < m) {
+        const uint32_t c = (iters & 1u) ? cB[t] : cA[t];
+        s_id[t] = c;
+        s_lo[t] = nlo[c];
+        s_hi[t] = nhi[c];
+        s_cnt[t] = cnt[c];
+        s_cost[t] = cost[c];
+    }
+    __syncthreads();   // also: every thread has read the state that the end writes
+    while (m > 1u) {
+        const uint32_t lanesLog2 = min(31u - (uint32_t)__clz((int)(PLOC_TAIL / m)), 4u);
+        const uint32_t i = t >> lanesLog2, sub = t & ((1u << lanesLog2) - 1u);
+        if (i < m) {
+            const int j = ploc_nearest(s_lo, s_hi, (int)i, (int)m, (int)i, (int)m, (int)sub, 1 << lanesLog2);
+            if (sub == 0u) s_nn[i] = (uint32_t)j;
+        }
+        __syncthreads();
+        // as k_ploc_flags, the pair packed: survivors below, new nodes above bit 16
+        bool alive = false, makes = false;
+        uint32_t j = 0u;
+        if (t < m) {
+            j = s_nn[t];
+            const bool mutual = j != t && s_nn[j] == t;
+            alive = !mutual || t < j;
+            makes = mutual && t < j;
+        }
+        const uint32_t v = (alive ? 1u : 0u) | (makes ? 1u << 16 : 0u);
+        uint32_t x = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t y = __shfl_up(x, off, 64);
+            if (lane >= (uint32_t)off) x += y;
+        }
+        if (lane == 63u) s_w[t >> 6] = x;
+        __syncthreads();
+        uint32_t before = 0u, total = 0u;
+        for (uint32_t k = 0; k < PLOC_TAIL / 64u; k++) {
+            const uint32_t c = s_w[k];
+            if (k < t >> 6) before += c;
+            total += c;
+        }
+        const uint32_t ex = before + x - v;
+        uint32_t id = 0u, c = 0u;
+        float4 lo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), hi = lo;
+        float best = 0.0f;
+        if (alive) {
+            id = s_id[t];
+            c = s_cnt[t];
+            lo = s_lo[t];
+            hi = s_hi[t];
+            best = s_cost[t];
+        }
+        if (makes) {
+            const uint32_t a = id, b = s_id[j];
+            id = n + nodeCount + (ex >> 16);
+            lo = min4(lo, s_lo[j]);
+            hi = max4(hi, s_hi[j]);
+            c += s_cnt[j];
+            const float A = box_area(lo, hi);
+            const float split = 2.0f * A + best + s_cost[j];
+            const float leafC = A * (float)c;
+            const bool ok = c <= maxLeaf && leafC <= split;
+            best = ok ? leafC : split;
+            nlo[id] = lo;
+            nhi[id] = hi;
+            kids[id - n] = make_uint2(a, b);
+            cnt[id] = c;
+            cost[id] = best;
+            leafOK[id] = ok ? 1u : 0u;
+        }
+        __syncthreads();   // every thread has read the clusters
+        if (alive) {
+            const uint32_t at = ex & 0xffffu;
+            s_id[at] = id;
+            s_cnt[at] = c;
+            s_lo[at] = lo;
+            s_hi[at] = hi;
+            s_cost[at] = best;
+        }
+        const uint32_t left = total & 0xffffu, made = total >> 16;   // the same in every thread
+        if (made == 0u || left + made != m || iters >= iterCap) {
+            stalled = true;
+            break;
+        }
+        nodeCount += made;
+        m = left;
+        if (t == 0u) iterEnd[iters] = nodeCount;
+        iters++;
+        __syncthreads();
+    }
+    if (t == 0u) *st = PlocState{m, nodeCount, iters, stalled ? 1u : 0u};
+}
+
+constexpr uint32_t TAIL_THREADS = 1024;
+
 // ---- top-down: triangle slots (off = position of the subtree's first triangle), node states ----
 
 __global__ void k_td_root(uint32_t root, const uint32_t* leafOK, uint32_t* state, uint32_t* off, uint32_t* depth) {
@@ -363,12 +508,10 @@ __global__ void k_td_root(uint32_t root, const uint32_t* leafOK, uint32_t* state
     depth[root] = 0u;
 }
 
-// Inner nodes n + [lo, hi): their states were set by their parents (created later).
-__global__ __launch_bounds__(BB) void k_td(uint32_t n, uint32_t lo, uint32_t hi, const uint2* kids,
-                                           const uint32_t* cnt, const uint32_t* leafOK, uint32_t* state,
-                                           uint32_t* off, uint32_t* depth, uint32_t* bad) {
-    const uint32_t k = lo + tid();
-    if (k >= hi) return;
+// Inner node n + k: its state was set by its parent (created later).
+__device__ __forceinline__ void td_node(uint32_t n, uint32_t k, const uint2* kids, const uint32_t* cnt,
+                                        const uint32_t* leafOK, uint32_t* state, uint32_t* off, uint32_t* depth,
+                                        uint32_t* bad) {
     const uint32_t X = n + k;
     const uint2 ch = kids[k];
     if (ch.x >= X || ch.y >= X) {   // a child is always created before its parent
@@ -386,6 +529,28 @@ __global__ __launch_bounds__(BB) void k_td(uint32_t n, uint32_t lo, uint32_t hi,
     } else {
         state[ch.x] = NODE_BELOW;
         state[ch.y] = NODE_BELOW;
+    }
+}
+
+// The inner nodes n + [lo, hi) of one clustering iteration.
+__global__ __launch_bounds__(BB) void k_td(uint32_t n, uint32_t lo, uint32_t hi, const uint2* kids,
+                                           const uint32_t* cnt, const uint32_t* leafOK, uint32_t* state,
+                                           uint32_t* off, uint32_t* depth, uint32_t* bad) {
+    const uint32_t k = lo + tid();
+    if (k < hi) td_node(n, k, kids, cnt, leafOK, state, off, depth, bad);
+}
+
+// The iterations [first, iters), last first, in one block: ranges of few nodes, whose launches were
+// their time (iters_in_block).  A node's parent lies in a later iteration, behind a barrier.
+__global__ __launch_bounds__(TAIL_THREADS) void k_td_tail(uint32_t n, uint32_t first, uint32_t iters,
+                                                          const uint32_t* iterEnd, const uint2* kids,
+                                                          const uint32_t* cnt, const uint32_t* leafOK, uint32_t* state,
+                                                          uint32_t* off, uint32_t* depth, uint32_t* bad) {
+    for (uint32_t it = iters; it-- > first;) {
+        const uint32_t lo = it ? iterEnd[it - 1] : 0u, hi = iterEnd[it];
+        for (uint32_t k = lo + threadIdx.x; k < hi; k += TAIL_THREADS)
+            td_node(n, k, kids, cnt, leafOK, state, off, depth, bad);
+        __syncthreads();
     }
 }
 
@@ -508,14 +673,12 @@ struct WideDP {
     uint8_t* split;
 };
 
-// Tables of the kept binary nodes made in one clustering iteration (ids n + [lo, hi)); their kept
-// children were made in earlier iterations, so their tables are complete.
+// Table of inner node n + k if it is kept; its kept children were made in earlier iterations, so
+// their tables are complete.
 template <int N>
-__global__ __launch_bounds__(BB) void k_wide_dp(uint32_t n, uint32_t lo, uint32_t hi, const uint32_t* state,
-                                                const uint2* index, const float4* nodes, uint32_t numNodes,
-                                                WideDP dp, uint32_t* bad) {
-    const uint32_t k = lo + tid();
-    if (k >= hi || state[n + k] != NODE_KEPT) return;
+__device__ __forceinline__ void wide_dp_node(uint32_t n, uint32_t k, const uint32_t* state, const uint2* index,
+                                             const float4* nodes, uint32_t numNodes, const WideDP& dp, uint32_t* bad) {
+    if (state[n + k] != NODE_KEPT) return;
     const uint32_t b = index[k].x;
     if (b >= numNodes) {
         atomicOr(bad, 64u);
@@ -562,6 +725,29 @@ __global__ __launch_bounds__(BB) void k_wide_dp(uint32_t n, uint32_t lo, uint32_
             dp.cost[base + i] = dp.cost[base + i - 1];
             dp.use[base + i] = dp.use[base + i - 1];
         }
+    }
+}
+
+// Tables of the inner nodes n + [lo, hi) of one clustering iteration.
+template <int N>
+__global__ __launch_bounds__(BB) void k_wide_dp(uint32_t n, uint32_t lo, uint32_t hi, const uint32_t* state,
+                                                const uint2* index, const float4* nodes, uint32_t numNodes,
+                                                WideDP dp, uint32_t* bad) {
+    const uint32_t k = lo + tid();
+    if (k < hi) wide_dp_node<N>(n, k, state, index, nodes, numNodes, dp, bad);
+}
+
+// The iterations [first, iters) in order, in one block (as k_td_tail).
+template <int N>
+__global__ __launch_bounds__(TAIL_THREADS) void k_wide_dp_tail(uint32_t n, uint32_t first, uint32_t iters,
+                                                               const uint32_t* iterEnd, const uint32_t* state,
+                                                               const uint2* index, const float4* nodes,
+                                                               uint32_t numNodes, WideDP dp, uint32_t* bad) {
+    for (uint32_t it = first; it < iters; it++) {
+        const uint32_t lo = it ? iterEnd[it - 1] : 0u, hi = iterEnd[it];
+        for (uint32_t k = lo + threadIdx.x; k < hi; k += TAIL_THREADS)
+            wide_dp_node<N>(n, k, state, index, nodes, numNodes, dp, bad);
+        __syncthreads();
     }
 }
 
@@ -778,6 +964,16 @@ struct Scan {
 
 inline dim3 blocks(uint32_t n) { return dim3((std::max(n, 1u) + BB - 1) / BB); }
 
+// The first of the last clustering iterations that made at most TAIL_THREADS nodes each: their
+// nodes are walked by one block (k_td_tail, k_wide_dp_tail), one iteration per barrier, instead of
+// by a launch each (1.06 M triangles: 76 launches and 0.7 ms for either walk, 29 launches and 0.25 and
+// 0.41 ms now).
+uint32_t iters_in_block(const std::vector<uint32_t>& iterEnd) {
+    uint32_t it = (uint32_t)iterEnd.size();
+    while (it > 0 && iterEnd[it - 1] - (it > 1 ? iterEnd[it - 2] : 0u) <= TAIL_THREADS) it--;
+    return it;
+}
+
 }  // namespace
 
 bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask, uint32_t n, uint32_t maxLeaf,
@@ -873,7 +1069,8 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
                        B.cost, B.leafOK, B.cA);
     // Clustering.  The cluster count lives on the device (PlocState); the host enqueues
     // PLOC_BATCH iterations at a time, sized for the last count it read (an upper bound: the
-    // count only falls), and reads the state back once per batch.
+    // count only falls), then the tail, which runs once the count is small enough, and reads the
+    // state back once per batch.
     const Scan scan{B.tileSums, B.total};
     const PlocState st0{n, 0u, 0u, 0u};
     e = hipMemcpyAsync(B.ploc, &st0, sizeof(st0), hipMemcpyHostToDevice, s);
@@ -881,10 +1078,13 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
     PlocState st = st0;
     uint32_t* cin = B.cA;
     uint32_t* cout = B.cB;
-    constexpr int PLOC_BATCH = 16;
+    constexpr int PLOC_BATCH = 8;
     while (st.m > 1) {
-        for (int it = 0; it < PLOC_BATCH && e == hipSuccess; it++) {
-            hipLaunchKernelGGL(k_ploc_nn, blocks(st.m), dim3(BB), 0, s, cin, B.ploc, B.nlo, B.nhi, B.nn);
+        for (int it = 0; it < PLOC_BATCH && st.m > PLOC_TAIL && e == hipSuccess; it++) {
+            if (st.m > PLOC_LANES_MAX)
+                hipLaunchKernelGGL(k_ploc_nn<1>, blocks(st.m), dim3(BB), 0, s, cin, B.ploc, B.nlo, B.nhi, B.nn);
+            else
+                hipLaunchKernelGGL(k_ploc_nn<8>, blocks(8 * st.m), dim3(BB), 0, s, cin, B.ploc, B.nlo, B.nhi, B.nn);
             hipLaunchKernelGGL(k_ploc_flags, blocks(st.m), dim3(BB), 0, s, B.nn, B.ploc, B.flags);
             e = scan.run(B.flags, st.m, s, &B.ploc->m);
             hipLaunchKernelGGL(k_ploc_merge, blocks(st.m), dim3(BB), 0, s, cin, cout, B.nn, B.flags, B.ploc, n, maxLeaf,
@@ -892,6 +1092,8 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
             hipLaunchKernelGGL(k_ploc_advance, dim3(1), dim3(64), 0, s, B.ploc, B.total, B.iterEnd, n);
             std::swap(cin, cout);
         }
+        hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(PLOC_TAIL), 0, s, B.ploc, B.cA, B.cB, n, maxLeaf, B.nlo, B.nhi,
+                           B.kids, B.cnt, B.cost, B.leafOK, B.iterEnd, n);
         if (e == hipSuccess) e = hipMemcpy(&st, B.ploc, sizeof(st), hipMemcpyDeviceToHost);
         if (e != hipSuccess) return fail(e, "clustering");
         if (st.stalled) {
@@ -907,7 +1109,11 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
     const uint32_t root = n == 1 ? 0u : n + inner - 1;   // the last node created
     // top-down: slots, states, depths
     hipLaunchKernelGGL(k_td_root, dim3(1), dim3(64), 0, s, root, B.leafOK, B.state, B.off, B.depth);
-    for (size_t it = iterEnd.size(); it-- > 0;) {
+    const uint32_t inBlock = iters_in_block(iterEnd), iters = (uint32_t)iterEnd.size();
+    if (inBlock < iters)
+        hipLaunchKernelGGL(k_td_tail, dim3(1), dim3(TAIL_THREADS), 0, s, n, inBlock, iters, B.iterEnd, B.kids, B.cnt,
+                           B.leafOK, B.state, B.off, B.depth, B.scalars + 2);
+    for (uint32_t it = inBlock; it-- > 0;) {
         const uint32_t lo = it ? iterEnd[it - 1] : 0u, hi = iterEnd[it];
         hipLaunchKernelGGL(k_td, blocks(hi - lo), dim3(BB), 0, s, n, lo, hi, B.kids, B.cnt, B.leafOK, B.state, B.off,
                            B.depth, B.scalars + 2);
@@ -983,7 +1189,7 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
             return fail(e, "allocation of the wide nodes failed");
         }
         // the tables, one clustering iteration at a time (B.flags still holds the kept ranks)
-        for (size_t it = 0; it < iterEnd.size(); it++) {
+        for (uint32_t it = 0; it < inBlock; it++) {
             const uint32_t lo = it ? iterEnd[it - 1] : 0u, hi = iterEnd[it];
             if (wantWidth == 4)
                 hipLaunchKernelGGL(k_wide_dp<4>, blocks(hi - lo), dim3(BB), 0, s, n, lo, hi, B.state, B.flags, out.nodes,
@@ -991,6 +1197,14 @@ bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask
             else
                 hipLaunchKernelGGL(k_wide_dp<8>, blocks(hi - lo), dim3(BB), 0, s, n, lo, hi, B.state, B.flags, out.nodes,
                                    numNodes, dp, bad);
+        }
+        if (inBlock < iters) {
+            if (wantWidth == 4)
+                hipLaunchKernelGGL(k_wide_dp_tail<4>, dim3(1), dim3(TAIL_THREADS), 0, s, n, inBlock, iters, B.iterEnd,
+                                   B.state, B.flags, out.nodes, numNodes, dp, bad);
+            else
+                hipLaunchKernelGGL(k_wide_dp_tail<8>, dim3(1), dim3(TAIL_THREADS), 0, s, n, inBlock, iters, B.iterEnd,
+                                   B.state, B.flags, out.nodes, numNodes, dp, bad);
         }
         // one level of wide nodes per round; the least-area tables first, the greedy rule if
         // their tree's stack bound does not fit

@@ -242,3 +242,19 @@ def test_ray_counts_and_alignment(width, orc, cx_runtime, cx_ctx):
             for x, y in zip(ref, outs):
                 assert np.array_equal(np.resize(bits(x), n), bits(y.numpy())), (n, shift)
             assert np.array_equal(np.resize(occ, n), flags.numpy()), (n, shift)
+
+
+@pytest.mark.parametrize("k", [1023, 1024, 1025, 1100, 2304])
+def test_device_build_at_the_tail_of_the_clustering(k, orc, cx_runtime, cx_ctx):
+    """Triangle counts around the one that a single block clusters to the root (1024), and coincident
+    and zero-area triangles among them (areas that tie): the answers stay the oracle's."""
+    sc = _subset(scenes.cornell_box(1, 8), k)
+    sc.indices[k // 2:k // 2 + 40] = sc.indices[3]        # coincident
+    sc.indices[k // 3:k // 3 + 40, 1] = sc.indices[k // 3:k // 3 + 40, 0]   # zero area
+    rays = np.concatenate([random_rays(sc, 4000, seed=93), centroid_rays(sc, seed=94)])
+    srays = shadow_rays(sc, 4000, seed=95)
+    oscene = orc.OracleScene(sc)
+    for width in (2, 4, 8):
+        gscene = cx_runtime.Scene(cx_ctx, sc, width=width, builder="device")
+        assert gscene.info.bvhBuilder == 1
+        _check_against_oracle(sc, gscene, oscene, rays, srays)
