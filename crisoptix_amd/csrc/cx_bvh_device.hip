@@ -147,6 +147,65 @@ __global__ __launch_bounds__(BB) void k_scan_apply(uint2* a, uint32_t n, const u
     }
 }
 
+// ---- geometry check and vertex bounds ----
+
+// Memory bound (16 bytes per triangle and 12 per vertex, read once).  On the host the same loops took
+// 2 ms of a 1.06 M-triangle scene's build (10.7 to 8.8 ms with the first query); the kernel takes
+// 19 us.
+constexpr uint32_t CHECK_BLOCKS = 512;
+
+struct GeometryPart {
+    float mn[3], mx[3];   // of the block's vertices and the origin
+    uint32_t bad;         // an index, a material id or a position out of range
+    uint32_t pad;
+};
+
+__global__ __launch_bounds__(BB) void k_check_geometry(const float* pos, uint32_t numVertices, const uint32_t* idx,
+                                                       const uint32_t* triMat, uint32_t numTriangles,
+                                                       uint32_t numMaterials, GeometryPart* parts) {
+    __shared__ float s_mn[BB / 64][3], s_mx[BB / 64][3];
+    __shared__ uint32_t s_bad[BB / 64];
+    const uint32_t stride = gridDim.x * BB;
+    bool bad = false;
+    for (size_t t = tid(); t < numTriangles; t += stride)
+        bad |= triMat[t] >= numMaterials || idx[3 * t] >= numVertices || idx[3 * t + 1] >= numVertices ||
+               idx[3 * t + 2] >= numVertices;
+    float mn[3] = {0.0f, 0.0f, 0.0f}, mx[3] = {0.0f, 0.0f, 0.0f};
+    for (size_t v = tid(); v < numVertices; v += stride)
+        for (int a = 0; a < 3; a++) {
+            const float c = pos[3 * v + a];
+            bad |= !(fabsf(c) < INFINITY);
+            mn[a] = c < mn[a] ? c : mn[a];
+            mx[a] = mx[a] < c ? c : mx[a];
+        }
+    for (int off = 32; off > 0; off >>= 1)
+        for (int a = 0; a < 3; a++) {
+            const float l = __shfl_xor(mn[a], off, 64), h = __shfl_xor(mx[a], off, 64);
+            mn[a] = l < mn[a] ? l : mn[a];
+            mx[a] = mx[a] < h ? h : mx[a];
+        }
+    const uint32_t w = threadIdx.x >> 6;
+    const bool any = __ballot(bad) != 0ull;
+    if ((threadIdx.x & 63u) == 0u) {
+        for (int a = 0; a < 3; a++) {
+            s_mn[w][a] = mn[a];
+            s_mx[w][a] = mx[a];
+        }
+        s_bad[w] = any ? 1u : 0u;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0u) return;
+    GeometryPart p{{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, 0u, 0u};
+    for (uint32_t k = 0; k < BB / 64; k++) {
+        for (int a = 0; a < 3; a++) {
+            p.mn[a] = s_mn[k][a] < p.mn[a] ? s_mn[k][a] : p.mn[a];
+            p.mx[a] = p.mx[a] < s_mx[k][a] ? s_mx[k][a] : p.mx[a];
+        }
+        p.bad |= s_bad[k];
+    }
+    parts[blockIdx.x] = p;
+}
+
 // ---- triangle boxes, centroid bounds, Morton keys ----
 
 __global__ __launch_bounds__(BB) void k_tri_boxes(const float* pos, const uint32_t* idx, uint32_t n, float4* triLo,
@@ -975,6 +1034,31 @@ uint32_t iters_in_block(const std::vector<uint32_t>& iterEnd) {
 }
 
 }  // namespace
+
+hipError_t check_geometry_device(const float* pos, uint32_t numVertices, const uint32_t* idx, const uint32_t* triMat,
+                                 uint32_t numTriangles, uint32_t numMaterials, bool& ok, float (&mn)[3],
+                                 float (&mx)[3]) {
+    GeometryPart* parts = nullptr;
+    hipError_t e = hipMalloc((void**)&parts, CHECK_BLOCKS * sizeof(GeometryPart));
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_check_geometry, dim3(CHECK_BLOCKS), dim3(BB), 0, nullptr, pos, numVertices, idx, triMat,
+                       numTriangles, numMaterials, parts);
+    e = hipGetLastError();
+    GeometryPart host[CHECK_BLOCKS];
+    if (e == hipSuccess) e = hipMemcpy(host, parts, sizeof(host), hipMemcpyDeviceToHost);
+    (void)hipFree(parts);
+    if (e != hipSuccess) return e;
+    ok = true;
+    for (int a = 0; a < 3; a++) mn[a] = mx[a] = 0.0f;
+    for (const GeometryPart& p : host) {
+        ok = ok && p.bad == 0u;
+        for (int a = 0; a < 3; a++) {
+            mn[a] = std::min(mn[a], p.mn[a]);
+            mx[a] = std::max(mx[a], p.mx[a]);
+        }
+    }
+    return hipSuccess;
+}
 
 bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask, uint32_t n, uint32_t maxLeaf,
                       int wantWidth, DeviceBvh& out, std::vector<void*>& allocs, std::string& err, hipError_t& herr) {

@@ -686,28 +686,39 @@ int cx_scene_build(cx_ctx* ctx, const cx_scene_desc* d, cx_scene** out) {
     if (d->numEmitters == 0 || !d->emitterFaces || !d->emitterFaceOffset || !d->emitterColor)
         return set_err(ctx, CX_ERR_INVALID_ARG, "at least one emitter is required (sample_emitter.h:5-6)");
     if (d->numMaterials == 0 || !d->materials) return set_err(ctx, CX_ERR_INVALID_ARG, "no materials");
-    for (uint32_t t = 0; t < d->numTriangles; t++) {
-        if (d->triMaterial[t] >= d->numMaterials) return set_err(ctx, CX_ERR_INVALID_ARG, "material id out of range");
-        for (int k = 0; k < 3; k++)
-            if (d->indices[3 * (size_t)t + k] >= d->numVertices)
-                return set_err(ctx, CX_ERR_INVALID_ARG, "vertex index out of range");
-    }
+    // For the device builder the uploaded arrays are checked on the device; these loops then only
+    // name the error, ahead of any found after them.
+    const bool onDevice = d->bvhBuilder == CX_BVH_BUILD_DEVICE;
+    auto index_error = [&]() -> const char* {
+        for (uint32_t t = 0; t < d->numTriangles; t++) {
+            if (d->triMaterial[t] >= d->numMaterials) return "material id out of range";
+            for (int k = 0; k < 3; k++)
+                if (d->indices[3 * (size_t)t + k] >= d->numVertices) return "vertex index out of range";
+        }
+        return nullptr;
+    };
+    if (!onDevice)
+        if (const char* m = index_error()) return set_err(ctx, CX_ERR_INVALID_ARG, m);
+    auto refuse = [&](const char* msg) {
+        const char* first = onDevice ? index_error() : nullptr;
+        return set_err(ctx, CX_ERR_INVALID_ARG, first ? first : msg);
+    };
     const uint32_t numFaces = d->emitterFaceOffset[d->numEmitters];
     for (uint32_t e = 0; e < d->numEmitters; e++)
         if (d->emitterFaceOffset[e + 1] <= d->emitterFaceOffset[e])
-            return set_err(ctx, CX_ERR_INVALID_ARG, "every emitter needs at least one face");
+            return refuse("every emitter needs at least one face");
     // Textures: the sampler's wrap arithmetic needs 1 <= size <= 65536 per axis, and texel
     // offsets are 32-bit.
-    if (d->numTextures && !d->textures) return set_err(ctx, CX_ERR_INVALID_ARG, "missing texture array");
+    if (d->numTextures && !d->textures) return refuse("missing texture array");
     std::vector<uint4> texInfo(d->numTextures);
     uint64_t numTexels = 0;
     for (uint32_t t = 0; t < d->numTextures; t++) {
         const cx_texture& tx = d->textures[t];
         if (!tx.rgba || tx.width == 0 || tx.height == 0 || tx.width > 65536u || tx.height > 65536u)
-            return set_err(ctx, CX_ERR_INVALID_ARG, "texture size must be 1..65536 per axis with data");
+            return refuse("texture size must be 1..65536 per axis with data");
         texInfo[t] = make_uint4((uint32_t)numTexels, tx.width, tx.height, 0u);
         numTexels += (uint64_t)tx.width * tx.height;
-        if (numTexels >= (1ull << 32)) return set_err(ctx, CX_ERR_INVALID_ARG, "more than 2^32 texels");
+        if (numTexels >= (1ull << 32)) return refuse("more than 2^32 texels");
     }
     std::vector<int4> matTex(d->numMaterials, make_int4(-1, -1, -1, 0));
     if (d->materialTex)
@@ -716,20 +727,23 @@ int cx_scene_build(cx_ctx* ctx, const cx_scene_desc* d, cx_scene** out) {
             const int32_t ids[3] = {mt.diffTex, mt.specTex, mt.roughTex};
             for (int k = 0; k < 3; k++)
                 if (ids[k] < -1 || (ids[k] >= 0 && (uint32_t)ids[k] >= d->numTextures))
-                    return set_err(ctx, CX_ERR_INVALID_ARG, "material texture index out of range");
+                    return refuse("material texture index out of range");
             if (mt.specTexUsage > CX_SPEC_TEX_OCC_ROUGH_METAL)
-                return set_err(ctx, CX_ERR_INVALID_ARG, "unknown specTexUsage");
+                return refuse("unknown specTexUsage");
             matTex[m] = make_int4(mt.diffTex, mt.specTex, mt.roughTex, (int32_t)mt.specTexUsage);
         }
     const uint32_t wantWidth = d->bvhWidth ? d->bvhWidth : 4u;
     if (wantWidth != 2 && wantWidth != 4 && wantWidth != 8)
-        return set_err(ctx, CX_ERR_INVALID_ARG, "bvhWidth must be 0, 2, 4 or 8");
+        return refuse("bvhWidth must be 0, 2, 4 or 8");
     if (d->bvhBuilder != CX_BVH_BUILD_HOST && d->bvhBuilder != CX_BVH_BUILD_DEVICE)
-        return set_err(ctx, CX_ERR_INVALID_ARG, "unknown bvhBuilder");
-    const bool onDevice = d->bvhBuilder == CX_BVH_BUILD_DEVICE;
+        return refuse("unknown bvhBuilder");
     // Both builders compare box areas and centroids: they need finite coordinates.
-    for (size_t i = 0; i < 3 * (size_t)d->numVertices; i++)
-        if (!std::isfinite(d->positions[i])) return set_err(ctx, CX_ERR_INVALID_ARG, "non-finite vertex position");
+    auto positions_finite = [&]() {
+        for (size_t i = 0; i < 3 * (size_t)d->numVertices; i++)
+            if (!std::isfinite(d->positions[i])) return false;
+        return true;
+    };
+    if (!onDevice && !positions_finite()) return refuse("non-finite vertex position");
     const uint32_t maxLeaf = d->bvhMaxLeafSize ? d->bvhMaxLeafSize : DEFAULT_MAX_LEAF;
     const auto tBuild = std::chrono::steady_clock::now();
     BvhHost bvh;
@@ -800,7 +814,17 @@ int cx_scene_build(cx_ctx* ctx, const cx_scene_desc* d, cx_scene** out) {
         return hip_err(ctx, e, "scene upload");
     }
     uint32_t builderUsed = d->bvhBuilder;
+    float mn[3] = {0.0f, 0.0f, 0.0f}, mx[3] = {0.0f, 0.0f, 0.0f};
     if (onDevice) {
+        bool ok = false;
+        const hipError_t ce = check_geometry_device(s->d.pos, d->numVertices, s->d.idx, s->d.triMat, d->numTriangles,
+                                                    d->numMaterials, ok, mn, mx);
+        if (ce != hipSuccess || !ok) {
+            free_all(s->allocs);
+            delete s;
+            if (ce != hipSuccess) return hip_err(ctx, ce, "geometry check");
+            return refuse("non-finite vertex position");
+        }
         DeviceBvh db;
         hipError_t he = hipSuccess;
         std::vector<void*> bvhAllocs;
@@ -867,8 +891,7 @@ int cx_scene_build(cx_ctx* ctx, const cx_scene_desc* d, cx_scene** out) {
     s->d.wroot = wroot;
     s->d.width = width;
     // Scene::GetSceneSize (src/Scene.cpp:48-71): bbox of all vertices and the origin.
-    float mn[3] = {0.0f, 0.0f, 0.0f}, mx[3] = {0.0f, 0.0f, 0.0f};
-    for (uint32_t v = 0; v < d->numVertices; v++)
+    for (uint32_t v = 0; v < d->numVertices && !onDevice; v++)
         for (int a = 0; a < 3; a++) {
             const float c = d->positions[3 * (size_t)v + a];
             mn[a] = (c < mn[a]) ? c : mn[a];

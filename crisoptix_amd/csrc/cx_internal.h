@@ -141,6 +141,10 @@ struct DeviceBvh {
     uint32_t width = 2, maxDepth = 0, stackBound = 0;
     bool tooDeep = false;        // the binary tree is deeper than the traversal stack
 };
+// ok: indices and material ids in range, positions finite; mn, mx: bounds of the vertices and the origin.
+hipError_t check_geometry_device(const float* pos, uint32_t numVertices, const uint32_t* idx, const uint32_t* triMat,
+                                 uint32_t numTriangles, uint32_t numMaterials, bool& ok, float (&mn)[3],
+                                 float (&mx)[3]);
 // mask: CX_VIS_* bits per triangle in device memory, or null.
 bool build_bvh_device(const float* pos, const uint32_t* idx, const uint8_t* mask, uint32_t numTris, uint32_t maxLeaf,
                       int wantWidth, DeviceBvh& out, std::vector<void*>& allocs, std::string& err, hipError_t& herr);

@@ -258,3 +258,26 @@ def test_device_build_at_the_tail_of_the_clustering(k, orc, cx_runtime, cx_ctx):
         gscene = cx_runtime.Scene(cx_ctx, sc, width=width, builder="device")
         assert gscene.info.bvhBuilder == 1
         _check_against_oracle(sc, gscene, oscene, rays, srays)
+
+
+@pytest.mark.parametrize("fault,message", [("index", "vertex index out of range"), ("material", "material id out of range"),
+                                           ("nan", "non-finite vertex position"), ("inf", "non-finite vertex position"),
+                                           ("index and width", "vertex index out of range")])
+@pytest.mark.parametrize("builder", ["host", "device"])
+def test_faulty_geometry_is_refused(fault, message, builder, cx_runtime, cx_ctx):
+    """One wrong element at the end of an array is refused by name with either builder (the device
+    builder checks the uploaded arrays on the device, before anything reads through them), and the
+    same bounds and scene size are reported for the sound scene."""
+    sc = small_grid_scene()
+    a, b = (cx_runtime.Scene(cx_ctx, sc, builder=k).info for k in ("host", builder))
+    assert a.sceneSize == b.sceneSize and list(a.boundsMin) == list(b.boundsMin) and list(a.boundsMax) == list(b.boundsMax)
+    import copy
+    bad = copy.deepcopy(sc)
+    if "index" in fault:
+        bad.indices[-1, 2] = len(bad.positions)
+    if fault == "material":
+        bad.tri_material[-1] = 10**6
+    if fault in ("nan", "inf"):
+        bad.positions[-1, 1] = np.nan if fault == "nan" else -np.inf
+    with pytest.raises(Exception, match=message):
+        cx_runtime.Scene(cx_ctx, bad, width=3 if "width" in fault else 4, builder=builder)
