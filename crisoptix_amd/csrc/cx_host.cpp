@@ -491,18 +491,22 @@ void trace_rec(cx_renderer* r, hipStream_t s) {
 //    suffix walks 3 / 4 / 5 against 2 -> 25.43 / 25.69 / 25.98 against 25.77 ms before the tail
 //    took four lanes a job; one shift round less, 14.55 against 13.83 ms after).
 //  * Complete paths, whose context is 2 chunks, 6 rounds: 720p 1.51 ms against 1.79 (2), 1.57 (4)
-//    and 1.57 (9).
+//    and 1.57 (9).  At widths 2 and 8, whose tail takes one lane per job and rounds never skip
+//    (tailJobs 0), 2 and above 512 k pixels 3: 600x400 at width 2 on 1.06 M triangles 1.30 ms (2), 1.44
+//    (3) and 1.59 (6), 1280x720 2.32, 2.01 and 2.34; at width 8 on 271 k triangles 0.90, 1.02 and 1.07,
+//    and 1.76, 1.45 and 1.58.
 //  * Prefix shifts, most of which are one shadow ray, go to the tail at once up to 768 k pixels:
 //    256x256 ReSTIR PT 352 us against 391 with 2 rounds, 700x500 1.67 ms against 1.77, 900x600
 //    1.28 against 1.35, but 1920x1080 6.52 against 6.02.
 static constexpr uint32_t PREFIX_SHIFT_TAIL_PIXELS = 768u << 10;
+static constexpr uint32_t CP_THREE_ROUNDS_PIXELS = 512u << 10;
 
 uint32_t default_wave_rounds(int machine, int pass, uint32_t P, uint32_t tailJobs) {
     if (P <= tailJobs) return 0u;
     const bool prefixShift = pass == CX_PASS_PREFIX_GEN_TEMP || pass == CX_PASS_PREFIX_SPATIAL;
     switch (machine) {
         case WK_SG_STEP: return 3u;
-        case WK_CP_STEP: return 6u;
+        case WK_CP_STEP: return tailJobs ? 6u : (P > CP_THREE_ROUNDS_PIXELS ? 3u : 2u);
         case WK_SH_STEP: return prefixShift && tailJobs && P <= PREFIX_SHIFT_TAIL_PIXELS ? 0u : 2u;
         default: return 2u;
     }
