@@ -110,17 +110,14 @@ hipError_t wave_launch(int kernel, const WaveArgs& W, uint32_t threads, hipStrea
 // 8 triangles trace a frame's rays in 5.13-5.18 / 4.87-4.88 / 5.03-5.05 / 5.15 ms.
 static constexpr uint32_t DEFAULT_MAX_LEAF = 2;
 
-// Host BVH build output (binary SAH BVH in the node format of cx_scene_dev.h).
-// Zero float4 after the last triangle slot of every triangle array the traversal reads.
-static constexpr size_t TRI_PAD = 4;
-
 // Most bytes of a wide node array: the traversal addresses its nodes by 32-bit byte offsets.  A
 // larger one (more than 33 M 4-wide nodes) is replaced by the binary tree.
 static constexpr uint64_t WIDE_BYTES_MAX = uint64_t(1) << 32;
 
+// Host BVH build output (binary SAH BVH in the node format of cx_scene_dev.h).
 struct BvhHost {
     std::vector<float4> nodes;   // 4 per inner node
-    std::vector<float4> tris;    // 3 per triangle slot, then TRI_PAD zero float4 (none without triangles)
+    std::vector<float4> tris;    // 3 per triangle slot
     int32_t root = 0;
     uint32_t maxDepth = 0;
 };
