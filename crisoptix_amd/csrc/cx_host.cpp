@@ -80,7 +80,7 @@ struct cx_renderer {
         float4* ray[2] = {nullptr, nullptr};
         uint4* res[2] = {nullptr, nullptr};
         uint32_t* count = nullptr;   // [MACHINE_SETS][MACHINE_WORDS] counters of the machines, overflow flag
-        uint32_t set = MACHINE_SETS; // the next machine's counters (MACHINE_SETS: clear all first)
+        uint32_t set = 0;            // the next machine's counters (run_machine)
         float4* shiftRes = nullptr;
         size_t jobCap = 0;           // jobs a queue holds
         size_t ctxWords = 0;         // 16-byte context words a queue holds
@@ -138,6 +138,7 @@ struct cx_renderer {
     hipStream_t side = nullptr;       // non-blocking, default priority
     hipEvent_t evFork = nullptr, evQuery = nullptr;
     hipStream_t fgSide = nullptr;     // set while frame_body launches the final gather
+    bool inFrame = false;             // set while frame_body launches the passes
     // The caller's stream is recording a graph (hipStreamIsCapturing): the frame forks no side
     // stream and nothing may allocate, create streams or events, or synchronise.
     bool callerCapture = false;
@@ -515,12 +516,20 @@ uint32_t default_wave_rounds(int machine, int pass, uint32_t P, uint32_t tailJob
 // Runs one machine: `setup` (one thread per pixel) appends the first rays to queue 0, then at most
 // `rounds` rounds of traversal + step, or fewer and the tail.  Every job finishes within `rounds`
 // rounds (the bounds in wave_pass are the longest chains of trace calls of each machine).
+//
+// The machine's counters are clear when it starts because of a clear on the same stream in the same
+// unit of work, never because of what the host remembers: a caller may record a frame or a pass
+// and replay it, which the host does not see.  A frame clears all sets at its start and its
+// machines take one after another; a machine of a lone pass clears its own (the first) set.
 hipError_t run_machine(cx_renderer* r, WaveArgs W, int setup, int step, uint32_t cap, uint32_t rounds,
                        int pass, hipStream_t s) {
     hipError_t e = hipSuccess;
-    if (r->wave.set >= MACHINE_SETS) {
-        e = launch_zero_words(r->wave.count, MACHINE_SETS * MACHINE_WORDS, s);
+    if (!r->inFrame) {
         r->wave.set = 0;
+        e = launch_zero_words(r->wave.count, MACHINE_WORDS, s);
+    } else if (r->wave.set >= MACHINE_SETS) {   // a frame of many machines: all sets again
+        r->wave.set = 0;
+        e = launch_zero_words(r->wave.count, MACHINE_SETS * MACHINE_WORDS, s);
     }
     W.qin = queue_view(r, 1, cap);
     W.qout = queue_view(r, 0, cap);
@@ -1364,7 +1373,12 @@ int frame_body(cx_renderer* r, void* stream) {
     if (wave && (rc = ensure_wave(r, lp))) return rc;
     CX_HIP(r->ctx, launch_zero_counters(r->counters, COUNTER_STRIPES * NUM_COUNTERS, wave ? r->wave.count : nullptr,
                                         wave ? MACHINE_SETS * MACHINE_WORDS : 0u, s));
-    if (wave) r->wave.set = 0;
+    r->wave.set = 0;
+    struct InFrame {
+        bool& b;
+        explicit InFrame(bool& x) : b(x) { b = true; }
+        ~InFrame() { b = false; }
+    } inFrame(r->inFrame);
     rec(r, 0, s);
     auto run = [&](cx_pass p) -> int {
         r->passRan[p] = true;

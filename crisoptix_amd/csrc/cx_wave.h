@@ -36,9 +36,9 @@ static constexpr uint32_t QSTRIPES = 64;       // one per lane of the wavefront 
 static constexpr uint32_t QCOUNT_STRIDE = 16;  // words between stripes' counters (64 bytes)
 
 // Counter words of one machine: the stripe counts of its two queues and, per round, which of them
-// holds the jobs.  A frame's machines use one
-// set after another, so that one kernel at the start of the frame clears them all (a kernel per
-// machine took 5 us each, 8 of them in a Conditional ReSTIR frame).
+// holds the jobs.  A frame's machines use one set after another, so that one kernel at the start of
+// the frame clears them all (a kernel per machine took 5 us each, 8 of them in a Conditional ReSTIR
+// frame); the machines of a pass launched by itself clear the first set each.
 static constexpr uint32_t MACHINE_ROUNDS = 272;   // rounds of the longest walk and one more (maxPathLen <= 255)
 static constexpr uint32_t MACHINE_WORDS = 2 * QSTRIPES * QCOUNT_STRIDE + MACHINE_ROUNDS;
 static constexpr uint32_t MACHINE_SETS = 16;
