@@ -420,11 +420,13 @@ __global__ __launch_bounds__(WBLOCK) void k_w_prefix_init(WaveArgs W) {
 }
 
 // The step of each machine on the answer r to a job's last ray (origin o, direction d): the
-// reference's logic up to the job's next trace call or its end, where it stores the result.
+// reference's logic up to the job's next trace call or its end, where it stores the result if
+// `store` (false for the lanes that take a job's steps beside the one that stores).
 // Shared by the step kernels and the tail kernel.
-__device__ __forceinline__ Emit pg_advance(const WaveArgs& W, uint32_t job, PgState& s, uint4 r, V3 o, V3 d) {
+__device__ __forceinline__ Emit pg_advance(const WaveArgs& W, uint32_t job, PgState& s, uint4 r, V3 o, V3 d,
+                                         bool store) {
     const Emit e = pg_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d));
-    if (e.kind != EMIT_CLOSEST) pg_finish(W, job, s);
+    if (store && e.kind != EMIT_CLOSEST) pg_finish(W, job, s);
     return e;
 }
 
@@ -441,7 +443,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_pg_step(WaveArgs W) {
         s = pg_load(QI, slot, W.A.lp);
         V3 o, d;
         get_ray(QI, slot, o, d);
-        e = pg_advance(W, job, s, QI.res[slot], o, d);
+        e = pg_advance(W, job, s, QI.res[slot], o, d, true);
     }
     const uint32_t slot = append(QO, e.kind);
     if (active && e.kind != EMIT_NONE) {
@@ -451,9 +453,10 @@ __global__ __launch_bounds__(WBLOCK) void k_w_pg_step(WaveArgs W) {
     }
 }
 
-__device__ __forceinline__ Emit cp_advance(const WaveArgs& W, uint32_t job, CpState& s, uint4 r, V3 o, V3 d) {
+__device__ __forceinline__ Emit cp_advance(const WaveArgs& W, uint32_t job, CpState& s, uint4 r, V3 o, V3 d,
+                                         bool store) {
     const Emit e = cp_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d));
-    cp_finish(W, job, s, e.kind);
+    if (store) cp_finish(W, job, s, e.kind);
     return e;
 }
 
@@ -470,7 +473,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_cp_step(WaveArgs W) {
         s = cp_load(QI, slot);
         V3 o, d;
         get_ray(QI, slot, o, d);
-        e = cp_advance(W, job, s, QI.res[slot], o, d);
+        e = cp_advance(W, job, s, QI.res[slot], o, d, true);
     }
     const uint32_t slot = append(QO, e.kind);
     if (active && e.kind != EMIT_NONE) {
@@ -520,10 +523,11 @@ __global__ __launch_bounds__(WBLOCK) void k_w_prefix_temporal_setup(WaveArgs W) 
     }
 }
 
-__device__ __forceinline__ Emit sh_advance(const WaveArgs& W, uint32_t job, ShState& s, uint4 r, V3 o, V3 d) {
+__device__ __forceinline__ Emit sh_advance(const WaveArgs& W, uint32_t job, ShState& s, uint4 r, V3 o, V3 d,
+                                         bool store) {
     ShiftOut out;
     const Emit e = sh_on_hit(W.A.S, W.R, s, inter_from_hit(W.A.S, r, d), out);
-    if (e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
+    if (store && e.kind != EMIT_CLOSEST) shift_finish(W, job, out);
     return e;
 }
 
@@ -540,7 +544,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_sh_step(WaveArgs W) {
         s = sh_unpack(load_ctx<SH_CHUNKS>(QI, slot));
         V3 o, d;
         get_ray(QI, slot, o, d);
-        e = sh_advance(W, job, s, QI.res[slot], o, d);
+        e = sh_advance(W, job, s, QI.res[slot], o, d, true);
     }
     const uint32_t slot = append(QO, e.kind);
     if (active && e.kind != EMIT_NONE) {
@@ -864,12 +868,13 @@ __global__ __launch_bounds__(WBLOCK) void k_w_suffix_init(WaveArgs W, int gather
     }
 }
 
-__device__ __forceinline__ Emit sg_advance(const WaveArgs& W, uint32_t job, SgState& s, uint4 r, V3 o, V3 d) {
+__device__ __forceinline__ Emit sg_advance(const WaveArgs& W, uint32_t job, SgState& s, uint4 r, V3 o, V3 d,
+                                         bool store) {
     Emit e;
     if (s.state == SG_TRACE) e = sg_on_hit(W.A.S, W.A.lp, s, inter_from_hit(W.A.S, r, d), o);
     else if (s.state == SG_NEE) e = sg_on_shadow(s, r.x != 0, o);
     else e = sg_on_recon(s, inter_from_hit(W.A.S, r, d));
-    if (!keeps_context(e.kind)) sg_finish_store(W, job, s);
+    if (store && !keeps_context(e.kind)) sg_finish_store(W, job, s);
     return e;
 }
 
@@ -886,7 +891,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_sg_step(WaveArgs W) {
             s = sg_unpack(load_ctx<SG_CHUNKS>(QI, slot), QI.ray[(size_t)QI.cap + slot]);
             V3 o, d;
             get_ray(QI, slot, o, d);
-            e = sg_advance(W, job, s, QI.res[slot], o, d);
+            e = sg_advance(W, job, s, QI.res[slot], o, d, true);
         }
     }
     const uint32_t slot = append(QO, e.kind);
@@ -1323,10 +1328,11 @@ __global__ __launch_bounds__(WBLOCK) void k_w_fg_init(WaveArgs W) {
     }
 }
 
-__device__ __forceinline__ Emit fg_advance(const WaveArgs& W, uint32_t job, FgState& s, uint4 r, V3 o, V3 d) {
+__device__ __forceinline__ Emit fg_advance(const WaveArgs& W, uint32_t job, FgState& s, uint4 r, V3 o, V3 d,
+                                         bool store) {
     const Inter it = inter_from_hit(W.A.S, r, d);
     if (!it.valid) {
-        fg_finish(W, job, s, false, packed_invalid());
+        if (store) fg_finish(W, job, s, false, packed_invalid());
         return emit_none();
     }
     Rng rng;
@@ -1334,7 +1340,7 @@ __device__ __forceinline__ Emit fg_advance(const WaveArgs& W, uint32_t job, FgSt
     const BrdfSample bs = ggx_sample(W.A.S, it, rng);
     s.rng = rng.s;
     if (bs.pdf <= 0.0f) {
-        fg_finish(W, job, s, false, it.pack());
+        if (store) fg_finish(W, job, s, false, it.pack());
         return emit_none();
     }
     s.thr = s.thr * bs.brdf;
@@ -1342,7 +1348,7 @@ __device__ __forceinline__ Emit fg_advance(const WaveArgs& W, uint32_t job, FgSt
     s.idx++;
     s.dir = bs.outDir;
     if (s.idx < (uint32_t)W.A.lp.prefixLen) return emit_closest(it.pos, bs.outDir);
-    fg_finish(W, job, s, true, it.pack());
+    if (store) fg_finish(W, job, s, true, it.pack());
     return emit_none();
 }
 
@@ -1359,7 +1365,7 @@ __global__ __launch_bounds__(WBLOCK) void k_w_fg_step(WaveArgs W) {
         s = fg_unpack(load_ctx<FG_CHUNKS>(QI, slot));
         V3 o, d;
         get_ray(QI, slot, o, d);
-        e = fg_advance(W, job, s, QI.res[slot], o, d);
+        e = fg_advance(W, job, s, QI.res[slot], o, d, true);
     }
     const uint32_t slot = append(QO, e.kind);
     if (active && e.kind != EMIT_NONE) {
@@ -1381,8 +1387,8 @@ struct Mach<WK_PG_STEP> {
     using S = PgState;
     __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, const Queue& q, uint32_t slot) { return pg_load(q, slot, W.A.lp); }
-    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
-        return pg_advance(W, job, s, r, o, d);
+    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d, bool store) {
+        return pg_advance(W, job, s, r, o, d, store);
     }
 };
 template <>
@@ -1390,8 +1396,8 @@ struct Mach<WK_CP_STEP> {
     using S = CpState;
     __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, const Queue& q, uint32_t slot) { return cp_load(q, slot); }
-    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
-        return cp_advance(W, job, s, r, o, d);
+    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d, bool store) {
+        return cp_advance(W, job, s, r, o, d, store);
     }
 };
 template <>
@@ -1401,8 +1407,8 @@ struct Mach<WK_SG_STEP> {
     __device__ static S load(const WaveArgs& W, const Queue& q, uint32_t slot) {
         return sg_unpack(load_ctx<SG_CHUNKS>(q, slot), q.ray[(size_t)q.cap + slot]);
     }
-    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
-        return sg_advance(W, job, s, r, o, d);
+    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d, bool store) {
+        return sg_advance(W, job, s, r, o, d, store);
     }
 };
 template <>
@@ -1410,8 +1416,8 @@ struct Mach<WK_SH_STEP> {
     using S = ShState;
     __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, const Queue& q, uint32_t slot) { return sh_unpack(load_ctx<SH_CHUNKS>(q, slot)); }
-    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
-        return sh_advance(W, job, s, r, o, d);
+    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d, bool store) {
+        return sh_advance(W, job, s, r, o, d, store);
     }
 };
 template <>
@@ -1419,8 +1425,8 @@ struct Mach<WK_FG_STEP> {
     using S = FgState;
     __device__ static bool is_final(uint32_t job) { return true; }
     __device__ static S load(const WaveArgs& W, const Queue& q, uint32_t slot) { return fg_unpack(load_ctx<FG_CHUNKS>(q, slot)); }
-    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d) {
-        return fg_advance(W, job, s, r, o, d);
+    __device__ static Emit advance(const WaveArgs& W, uint32_t job, S& s, uint4 r, V3 o, V3 d, bool store) {
+        return fg_advance(W, job, s, r, o, d, store);
     }
 };
 
@@ -1432,7 +1438,8 @@ struct Mach<WK_FG_STEP> {
 // rounds cost nothing.  maxSteps is the machine's remaining round bound; a job still running
 // after it raises the queue's overflow flag (bit 1).
 // With at most TAIL_QUADS jobs a 4-wide ray is traced by four lanes (quad_trace): the job's steps
-// are then taken by all four with the same values, its first lane alone counting the rays and
+// are then taken by all four with the same values, its first lane alone storing the result (an
+// accumulated pixel and the pixel flags are read, changed and written), counting the rays and
 // answering the final one.
 // (160x90 frame 2.41 -> 1.96 ms, 256x256 ReSTIR PT 0.43 -> 0.40, 512x512 gradient step 1.72 -> 1.57,
 // 1080p frame 14.28 -> 13.88; a limit of 16 k jobs leaves the middle two as they were, one of 256 k
@@ -1476,7 +1483,7 @@ __device__ __forceinline__ void tail_job(const WaveArgs& W, const Queue& q, cons
             if (first) (void)final_answer(F, M == WK_SG_STEP ? job | JOB_FINAL : job, hit);
             e = emit_none();
         } else {
-            e = Mach<M>::advance(W, job, s, r, e.o, e.d);
+            e = Mach<M>::advance(W, job, s, r, e.o, e.d, first);
         }
     }
     if (e.kind != EMIT_NONE) atomicOr(q.overflow, 2u);
