@@ -646,7 +646,11 @@ __device__ __forceinline__ void quad_trace(const DScene& S, V3 o, V3 d, float tm
                 const int more = (k != miss ? 1 : 0) + (k1 != miss ? 1 : 0) + (k2 != miss ? 1 : 0) +
                                  (k3 != miss ? 1 : 0) - 1;   // entries to push
                 if (h && nearer > 0) col[(sp + more - nearer) * stride] = child;
-                __builtin_amdgcn_wave_barrier();   // the quad's other lanes read the entries
+                // the quad's other lanes read the entries: LDS answers a wavefront in order, so this
+                // only keeps the compiler from moving those reads ahead of the writes
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 sp += more;
                 ref = (int)quad_or(k == first ? (uint32_t)child : 0u);
                 continue;
