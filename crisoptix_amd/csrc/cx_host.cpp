@@ -550,8 +550,11 @@ hipError_t run_machine(cx_renderer* r, WaveArgs W, int setup, int step, uint32_t
         trace_rec(r, s);
         if (e == hipSuccess) e = wave_launch(step, W, 0, s);
     }
-    if (e == hipSuccess && waveRounds < rounds)   // the remaining rounds in one launch
-        e = wave_tail(step, W, rounds, pass, s);
+    // The remaining rounds in one launch.  Its bound on a job's steps is what the rounds have left of
+    // the machine's; where rounds may skip themselves the host cannot tell how many ran, and the
+    // bound is the machine's own.
+    if (e == hipSuccess && waveRounds < rounds)
+        e = wave_tail(step, W, W.skip ? rounds : rounds - waveRounds, pass, s);
     r->wave.set++;
     return e;
 }

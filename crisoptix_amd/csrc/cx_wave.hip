@@ -1435,8 +1435,10 @@ struct Mach<WK_FG_STEP> {
 // rays in place until it ends, instead of one traversal launch and one step launch per round.
 // For a machine's last rounds, whose queues are short: every job then follows its own chain of
 // rays, without waiting each round for the slowest ray of the whole queue, and the near-empty
-// rounds cost nothing.  maxSteps is the machine's remaining round bound; a job still running
-// after it raises the queue's overflow flag (bit 1).
+// rounds cost nothing.  maxSteps is at least the machine's remaining round bound and at most the
+// whole (run_machine); a job still running after it raises the queue's overflow flag (bit 1).  The
+// remaining bound itself, counted on the device where rounds skip themselves, took 15 of 1370 us of a
+// 160x90 frame.
 // With at most TAIL_QUADS jobs a 4-wide ray is traced by four lanes (quad_trace): the job's steps
 // are then taken by all four with the same values, its first lane alone storing the result (an
 // accumulated pixel and the pixel flags are read, changed and written), counting the rays and

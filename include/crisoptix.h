@@ -252,7 +252,7 @@ typedef struct cx_frame_stats {
     /* Nonzero if the wavefront queues ever failed since the renderer was created: bit 0, an
        append found its queue stripe full (the queues are sized so that it cannot; a diagnostic of
        that sizing); bit 1, a tail kernel ended a job that was still running at its step bound
-       (the bound is the longest trace chain of the machine, so it cannot either).  A frame with
+       (the bound is at least what is left of the machine's longest trace chain, so it cannot either).  A frame with
        either bit set has dropped work; bench.py refuses its numbers. */
     uint32_t queueOverflow;
     /* Rays traced in place by the tail kernels (cx_renderer_set_wave_rounds), included in the

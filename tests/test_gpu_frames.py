@@ -190,6 +190,38 @@ def test_final_shadow_rays_in_queue_and_tail_match_megakernel(mode, rounds, cx_r
     assert all(ren.stats().queueOverflow == 0 for ren in rens[1:])
 
 
+# Pixels: above the most jobs that a tail holds at four lanes each (65536); above them and the most
+# possible jobs (two per pixel and neighbour) of a prefix shift that goes to the tail at once.
+@pytest.mark.parametrize("W,H", [(401, 301), (1501, 1063)])
+@pytest.mark.parametrize("mode", ["path_tracer", "restir_pt_cornell", "conditional_restir"])
+def test_rounds_that_leave_the_rest_to_the_tail_match_megakernel(mode, W, H, cx_runtime, cx_ctx):
+    """At the default rounds an image of more pixels than the tail holds starts with queue rounds, and
+    the round that finds few enough jobs left, known on the device only, hands them to the tail: with
+    accumulation, on a closed scene (long paths, whose jobs thin out over the rounds), every frame and
+    the reservoirs equal the one-kernel-per-pass mode bit for bit."""
+    print(f"rounds and tail {mode} {W}x{H}", flush=True)
+    sc = scenes.cornell_box(1, 8)
+    gs = cx_runtime.Scene(cx_ctx, sc)
+    assert gs.info.bvhWidth == 4
+    p = abi.workload_params(mode, W, H, gs.size)
+    p.enableAccum = 0 if mode == "conditional_restir" else 1
+    cam = scenes.cornell_camera(W, H)
+    cd = abi.CameraData.from_dict(cam.data())
+    ref, ren = (cx_runtime.Renderer(W, H, cx_ctx, cam, gs, params=p, seed=15) for _ in range(2))
+    ref.set_exec_mode("megakernel")
+    for f in range(3):
+        a, b = (r.launch_frame(cd, f == 0).numpy() for r in (ref, ren))
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f
+    st = ren.stats()
+    assert st.queueOverflow == 0
+    assert 0 < st.tailClosestRays + st.tailShadowRays < st.closestRays + st.shadowRays
+    if mode != "path_tracer":
+        front = ref.state().frontBufferIdx
+        x, y = ref.prefix(front), ren.prefix(front)
+        for k in x:
+            assert np.array_equal(x[k].view(np.uint32), y[k].view(np.uint32)), k
+
+
 @pytest.mark.parametrize("width", [2, 4, 8])
 @pytest.mark.parametrize("queue_grid", [1, 3, 8192])
 @pytest.mark.parametrize("mode", ["path_tracer", "conditional_restir"])
