@@ -487,7 +487,10 @@ void trace_rec(cx_renderer* r, hipStream_t s) {
 //  * An image of at most tailJobs pixels goes to the tail at once: 160x90 Conditional ReSTIR 1.42 ms
 //    against 1.96 with rounds, 320x200 2.19 against 2.76, 64x64 path tracer 285 us against 410; at
 //    more pixels than that, 400x300 ReSTIR PT 1.00 ms against 1.04 with one round, 512x512 gradient
-//    step 1.69 against 1.47.
+//    step 1.69 against 1.47.  By pixels also for the suffix shifts, which have up to 2 (gatherM - 1)
+//    jobs a pixel: at most 65536 jobs at once instead, else two rounds, takes 160x90 with gatherM 2,
+//    9, 17, 32 from 1.27, 1.38, 1.58, 1.70 ms to 1.27, 1.45, 1.54, 1.75, 240x180 from 1.50, 1.77,
+//    1.88, 2.14 to 1.55, 1.84, 1.99, 2.19 (96 k triangles; the same picture on 1.06 M).
 //  * Suffix walks at most 3 rounds, prefix walks and suffix shifts 2 (1080p Conditional ReSTIR:
 //    suffix walks 3 / 4 / 5 against 2 -> 25.43 / 25.69 / 25.98 against 25.77 ms before the tail
 //    took four lanes a job; one shift round less, 14.55 against 13.83 ms after).
@@ -496,19 +499,28 @@ void trace_rec(cx_renderer* r, hipStream_t s) {
 //    (tailJobs 0), 2 and above 512 k pixels 3: 600x400 at width 2 on 1.06 M triangles 1.30 ms (2), 1.44
 //    (3) and 1.59 (6), 1280x720 2.32, 2.01 and 2.34; at width 8 on 271 k triangles 0.90, 1.02 and 1.07,
 //    and 1.76, 1.45 and 1.58.
-//  * Prefix shifts, most of which are one shadow ray, go to the tail at once up to 768 k pixels:
-//    256x256 ReSTIR PT 352 us against 391 with 2 rounds, 700x500 1.67 ms against 1.77, 900x600
-//    1.28 against 1.35, but 1920x1080 6.52 against 6.02.
-static constexpr uint32_t PREFIX_SHIFT_TAIL_PIXELS = 768u << 10;
+//  * Prefix shifts, most of which are one shadow ray, go to the tail at once up to 3.5 M possible
+//    jobs, two per pixel and neighbour.  ReSTIR PT, tail at once against 2 rounds, ms: spatial shifts
+//    on 271 k triangles 400x300 with 6 neighbours (1.4 M jobs) 1.07 and 1.14, 1280x720 with one
+//    (1.8 M) 2.41 and 2.51, 900x600 with 3 (3.2 M) 2.02 and 2.02 (Cornell box 1.27 and 1.29),
+//    640x480 with 6 (3.7 M) 1.75 and 1.72, 900x600 with 10 (10.8 M) 3.31 and 3.02, 1920x1080 with 10
+//    10.9 and 9.5; temporal shifts 1280x720 (1.8 M) 2.41 and 2.48, 1600x900 (2.9 M) 3.53 and 3.53,
+//    1920x1080 (4.1 M) 4.85 and 4.80.
+static constexpr uint64_t PREFIX_SHIFT_TAIL_JOBS = 3500000u;
 static constexpr uint32_t CP_THREE_ROUNDS_PIXELS = 512u << 10;
 
-uint32_t default_wave_rounds(int machine, int pass, uint32_t P, uint32_t tailJobs) {
+uint32_t default_wave_rounds(int machine, int setup, const WaveArgs& W, uint32_t tailJobs) {
+    const uint32_t P = W.A.P;
     if (P <= tailJobs) return 0u;
-    const bool prefixShift = pass == CX_PASS_PREFIX_GEN_TEMP || pass == CX_PASS_PREFIX_SPATIAL;
     switch (machine) {
         case WK_SG_STEP: return 3u;
         case WK_CP_STEP: return tailJobs ? 6u : (P > CP_THREE_ROUNDS_PIXELS ? 3u : 2u);
-        case WK_SH_STEP: return prefixShift && tailJobs && P <= PREFIX_SHIFT_TAIL_PIXELS ? 0u : 2u;
+        case WK_SH_STEP: {
+            const uint64_t jobs = setup == WK_PREFIX_TEMPORAL_SETUP  ? 2ull * P
+                                  : setup == WK_PREFIX_SPATIAL_SETUP ? 2ull * P * W.S
+                                                                     : ~0ull;
+            return tailJobs && jobs <= PREFIX_SHIFT_TAIL_JOBS ? 0u : 2u;
+        }
         default: return 2u;
     }
 }
@@ -541,7 +553,7 @@ hipError_t run_machine(cx_renderer* r, WaveArgs W, int setup, int step, uint32_t
     // a setting of 0 runs every round in the queue; a default of 0 starts with the tail
     const bool set = r->waveRounds != CX_WAVE_ROUNDS_DEFAULT;
     const uint32_t tailJobs = wave_tail_jobs(step, W.A.S);
-    const uint32_t wr = set ? (r->waveRounds ? r->waveRounds : rounds) : default_wave_rounds(step, pass, r->P, tailJobs);
+    const uint32_t wr = set ? (r->waveRounds ? r->waveRounds : rounds) : default_wave_rounds(step, setup, W, tailJobs);
     const uint32_t waveRounds = std::min({wr, rounds, MACHINE_ROUNDS - 1});
     W.skip = set || waveRounds == rounds ? 0u : tailJobs;
     for (W.round = 0; W.round < waveRounds && e == hipSuccess; W.round++) {

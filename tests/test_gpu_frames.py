@@ -192,7 +192,7 @@ def test_final_shadow_rays_in_queue_and_tail_match_megakernel(mode, rounds, cx_r
 
 # Pixels: above the most jobs that a tail holds at four lanes each (65536); above them and the most
 # possible jobs (two per pixel and neighbour) of a prefix shift that goes to the tail at once.
-@pytest.mark.parametrize("W,H", [(401, 301), (1501, 1063)])
+@pytest.mark.parametrize("W,H", [(401, 301), (1701, 1063)])
 @pytest.mark.parametrize("mode", ["path_tracer", "restir_pt_cornell", "conditional_restir"])
 def test_rounds_that_leave_the_rest_to_the_tail_match_megakernel(mode, W, H, cx_runtime, cx_ctx):
     """At the default rounds an image of more pixels than the tail holds starts with queue rounds, and
@@ -220,6 +220,30 @@ def test_rounds_that_leave_the_rest_to_the_tail_match_megakernel(mode, W, H, cx_
         x, y = ref.prefix(front), ren.prefix(front)
         for k in x:
             assert np.array_equal(x[k].view(np.uint32), y[k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("W,H,neighbours,launches", [(500, 400, 10, 4), (500, 400, 3, 2), (1280, 720, 1, 2),
+                                                     (1920, 1080, 1, 6)])
+def test_prefix_shift_rounds_follow_the_jobs(W, H, neighbours, launches, cx_runtime, cx_ctx):
+    """A prefix shift starts with the tail up to 3.5 M possible jobs, two per pixel and neighbour
+    (spatial) or two per pixel (temporal), else it takes two queue rounds, as the prefix walk does:
+    the traversal launches of a ReSTIR PT frame say which.  The image is that of two rounds throughout,
+    bit for bit."""
+    sc = scenes.cornell_box(1, 8)
+    gs = cx_runtime.Scene(cx_ctx, sc)
+    p = abi.workload_params("restir_pt_cornell", W, H, gs.size)
+    p.prefixSpatialCount = neighbours
+    cam = scenes.cornell_camera(W, H)
+    cd = abi.CameraData.from_dict(cam.data())
+    two, ren = (cx_runtime.Renderer(W, H, cx_ctx, cam, gs, params=p, seed=19) for _ in range(2))
+    two.set_wave_rounds(2)
+    ren.enable_timing(True)
+    for f in range(2):
+        a, b = (r.launch_frame(cd, f == 0).numpy() for r in (two, ren))
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f
+    st = ren.stats()
+    assert st.queueOverflow == 0 and two.stats().queueOverflow == 0
+    assert st.traceLaunches == launches
 
 
 @pytest.mark.parametrize("width", [2, 4, 8])
