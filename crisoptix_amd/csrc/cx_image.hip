@@ -49,8 +49,9 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // the c
 
 // Memory bound: 5 bytes per value.  A thread encodes the four values of one aligned 4-byte word of
 // the output (16-byte load, 4-byte store); the words at the ends, where the output does not begin
-// or end on a word, go value by value.  The double power on every value was the cost before: 24.9 M
-// values (4K RGB) took 132 us, 30 us now (4.1 TB/s).
+// or end on a word, go value by value.  The double power on every value was the cost before: a call
+// on 24.9 M values (4K RGB) took 144 us, 35 us now (3.5 TB/s, the launch included; calls queued one
+// behind the other 30 us each).
 __global__ __launch_bounds__(256) void k_tonemap(const float* __restrict__ hdr, uint8_t* __restrict__ ldr, uint32_t n,
                                                  uint32_t shift, uint32_t words) {
     const uint32_t g = blockIdx.x * 256u + threadIdx.x;

@@ -79,3 +79,20 @@ def test_gpu_tonemap_sizes_and_alignment(n, shift, orc, cx_runtime, cx_ctx):
     got = ldr.numpy()
     assert np.array_equal(got[4 + shift:4 + shift + n], orc.tonemap(c))
     assert np.all(got[:4 + shift] == 0xA5) and np.all(got[4 + shift + n:] == 0xA5)
+
+
+@pytest.mark.gpu
+def test_gpu_tonemap_every_float_of_the_curve(orc, cx_runtime, cx_ctx):
+    """Every float that takes the power (0.0031308 to 1.001, beyond which the clamp gives 255), where
+    the kernel estimates the byte and falls back on the double power beside its steps, and every 97th
+    of all floats, NaN payloads and both infinities among them."""
+    from concurrent.futures import ThreadPoolExecutor
+    first, last = (int(np.float32(x).view(np.uint32)) for x in (0.0031308, 1.001))
+    curve = np.arange(first - 64, last + 64, dtype=np.uint32)
+    parts = np.array_split(curve, 8) + np.array_split(np.arange(0, 2**32, 97, dtype=np.uint64).astype(np.uint32), 8)
+    with ThreadPoolExecutor(8) as ex:
+        for i, (part, ref) in enumerate(zip(parts, ex.map(lambda p: orc.tonemap(p.view(np.float32)), parts))):
+            got = cx_runtime.tonemap(cx_ctx, cx_runtime.DeviceArray.from_numpy(part.view(np.float32)))
+            bad = np.flatnonzero(got != ref)
+            print(f"part {i}: {part.size} floats, {bad.size} differ", flush=True)
+            assert bad.size == 0, part[bad[:8]]
