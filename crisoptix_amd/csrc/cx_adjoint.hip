@@ -30,6 +30,7 @@
 namespace cx {
 
 static constexpr int ABLOCK = 128;
+static_assert(ABLOCK == TRACE_BLOCK, "the traversal stack's column stride");
 static constexpr int MAX_FACTORS = 16;
 static constexpr uint32_t NO_EMITTER = 0xFFFFFFFFu;
 
