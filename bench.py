@@ -9,8 +9,9 @@ rays only), max path length 8, camera inside the tent orbiting by 2*pi/64 per fr
 seeded scene data; every frame runs the full pass sequence of Renderer::LaunchFrame.
 
 One step = one frame.  ms_per_step = the median over the timed frames (frames W+1 .. W+K) of
-HIP-event time around one frame; value = counted rays (closest-hit + shadow) of the timed frames
-per second of their summed time.  roofline: the dominant kernel is the ray traversal
+HIP-event time around one frame; value = traced rays (closest-hit + shadow, cx_frame_stats; a
+shadow ray whose answer would change nothing is neither traced nor counted in wavefront mode) of the
+timed frames per second of their summed time.  roofline: the dominant kernel is the ray traversal
 (k_q_trace), timed by HIP events around each of its launches on the frame's stream; its
 algorithmic bytes are 48 B per closest-hit ray (32 B ray + 16 B hit) and 36 B per shadow ray
 (32 B ray + 4 B flag).  The line reports the workload's reuse density (valid suffixes, prefix

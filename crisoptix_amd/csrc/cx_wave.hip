@@ -246,8 +246,8 @@ __device__ __forceinline__ void trace_quads(const DScene& S, const Rays& rays, u
 // children sorted as 64-bit keys, branch-free pushes (trav_step_rt).  About 110 vector
 // instructions for a node and 90 for a triangle against 190 and 110 before (1080p frame 21.8 ->
 // 19.3 ms, the 720p path tracer 2.39 -> 1.87 ms, a 160x90 frame 3.56 -> 3.09 ms).  The 4-wide
-// kernel is held to at least 7 waves per SIMD (72 VGPRs, no spills); the 2-wide kernel keeps at
-// least 5.
+// kernel is held to at least 7 waves per SIMD (71 VGPRs; four that only an answered ray needs are
+// stored ahead of the loop and read back per answer); the 2-wide kernel keeps at least 5.
 template <int WIDTH>
 __global__ __launch_bounds__(WBLOCK) __attribute__((amdgpu_waves_per_eu(WIDTH == 8 ? 1 : (WIDTH == 4 ? 7 : 5), 8))) void k_q_trace(
     DScene S, Queue q0, Queue q1, const uint32_t* side, uint32_t skip, unsigned long long* counters,

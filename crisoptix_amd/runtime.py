@@ -459,7 +459,8 @@ class Renderer:
         lib().cx_renderer_enable_timing(self.h, 1 if on else 0)
 
     def set_exec_mode(self, mode: str):
-        """'wavefront' (default) or 'megakernel'; both give identical results."""
+        """'wavefront' (default) or 'megakernel'; both give identical images and records, the
+        shadow-ray counts of stats() differ (include/crisoptix.h, cx_frame_stats)."""
         self.ctx.check(lib().cx_renderer_set_exec_mode(self.h, abi.EXEC_MODES[mode]), "cx_renderer_set_exec_mode")
 
     def set_queue_grid(self, max_blocks: int):
@@ -474,7 +475,8 @@ class Renderer:
         self.ctx.check(lib().cx_renderer_set_overlap(self.h, 1 if enable else 0), "cx_renderer_set_overlap")
 
     def set_wave_rounds(self, rounds: int):
-        """Trace/step rounds per machine before the in-place tail kernel (0: all rounds)."""
+        """Trace/step rounds per machine before the in-place tail kernel (0: all rounds;
+        abi.CX_WAVE_ROUNDS_DEFAULT: chosen per machine, the initial setting)."""
         self.ctx.check(lib().cx_renderer_set_wave_rounds(self.h, rounds), "cx_renderer_set_wave_rounds")
 
     def set_device_random(self, enable: bool = True, seed: int = 0):

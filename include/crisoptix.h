@@ -196,8 +196,10 @@ typedef struct cx_scene_desc {
     uint32_t numEmitters;
     uint32_t bvhMaxLeafSize;       /* most triangles per leaf, 1..15; 0 = default (2) */
     uint32_t bvhWidth;             /* children per BVH node: 2, 4 or 8; 0 = default (4).  A wide
-                                      BVH whose worst-case traversal stack would not fit falls
-                                      back to 2 (cx_scene_info.bvhWidth reports the width used) */
+                                      BVH whose worst-case traversal stack would not fit, or whose
+                                      nodes would take more than 4 GiB (128 bytes each at width 4,
+                                      256 at 8; of the order of 10^8 triangles), falls back to 2
+                                      (cx_scene_info.bvhWidth reports the width used) */
     const float* uvs;              /* host, [numVertices][2] texture coordinates (Vertex::uv,
                                       src/Model.cpp:79-92), or NULL: all (0, 0) */
     const cx_material_tex* materialTex; /* host, [numMaterials], or NULL: no textures and
@@ -232,7 +234,12 @@ typedef struct cx_scene_info {
                                       the device build, ms */
 } cx_scene_info;
 
-/* Per-pass timing of the last frame, ms (src/Renderer.cpp:396-402), plus ray counts. */
+/* Per-pass timing of the last frame, ms (src/Renderer.cpp:396-402), plus the counts of the rays that
+ * were traced.  Closest-hit counts are the same in either execution mode.  CX_EXEC_WAVEFRONT
+ * evaluates what a path or shift would contribute before its last shadow ray, and neither traces nor
+ * counts the ray if that is nothing whatever the answer (no BSDF density towards the light or across
+ * the reconnection, a contribution of zero), so its shadow-ray counts are smaller than those of
+ * CX_EXEC_MEGAKERNEL, which traces first. */
 typedef struct cx_frame_stats {
     float passMs[CX_PASS_COUNT];
     float totalMs;
@@ -360,8 +367,9 @@ int cx_renderer_begin_frame(cx_renderer* r, const cx_camera* cam, int cameraChan
                             float* d_output);
 int cx_pass_launch(cx_renderer* r, cx_pass pass, const cx_launch_params* params, void* stream);
 /*
- * Execution strategy of the passes; both give identical results.  No counterpart in the
- * reference, whose passes are single OptiX raygen launches.
+ * Execution strategy of the passes; both give identical images, reservoirs and neighbour lists
+ * (their counts of shadow rays differ, cx_frame_stats).  No counterpart in the reference, whose
+ * passes are single OptiX raygen launches.
  *   CX_EXEC_WAVEFRONT (default): path generation and shifts run as state machines whose
  *     rays are answered by separate traversal kernels, several launches per pass, with no
  *     host synchronisation inside a frame.
@@ -393,8 +401,9 @@ int cx_renderer_set_queue_grid(cx_renderer* r, uint32_t maxBlocks);
  * launch and one step launch, then finishes its remaining jobs in one kernel that traces each
  * job's rays in place (the same traversal, so the same answers and ray counts).  `rounds` applies
  * to every machine; 0 runs every round as traversal + step; CX_WAVE_ROUNDS_DEFAULT (the initial
- * setting) chooses per machine by the image's size and ends the rounds once the jobs left fit on
- * the device at once.  Results are identical for every value; a tuning knob
+ * setting) chooses per machine by the image's size and jobs, starts small ones with the in-place
+ * kernel, and ends the rounds once the jobs left fit on the device at once, which a set number of
+ * rounds never does.  Results are identical for every value; a tuning knob
  * (crisoptix_amd/tune.py). */
 #define CX_WAVE_ROUNDS_DEFAULT 0xFFFFFFFFu
 int cx_renderer_set_wave_rounds(cx_renderer* r, uint32_t rounds);
