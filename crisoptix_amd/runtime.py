@@ -460,7 +460,7 @@ class Renderer:
 
     def set_exec_mode(self, mode: str):
         """'wavefront' (default) or 'megakernel'; both give identical images and records, the
-        shadow-ray counts of stats() differ (include/crisoptix.h, cx_frame_stats)."""
+        ray counts of stats() differ (include/crisoptix.h, cx_frame_stats)."""
         self.ctx.check(lib().cx_renderer_set_exec_mode(self.h, abi.EXEC_MODES[mode]), "cx_renderer_set_exec_mode")
 
     def set_queue_grid(self, max_blocks: int):

@@ -235,11 +235,11 @@ typedef struct cx_scene_info {
 } cx_scene_info;
 
 /* Per-pass timing of the last frame, ms (src/Renderer.cpp:396-402), plus the counts of the rays that
- * were traced.  Closest-hit counts are the same in either execution mode.  CX_EXEC_WAVEFRONT
- * evaluates what a path or shift would contribute before its last shadow ray, and neither traces nor
- * counts the ray if that is nothing whatever the answer (no BSDF density towards the light or across
- * the reconnection, a contribution of zero), so its shadow-ray counts are smaller than those of
- * CX_EXEC_MEGAKERNEL, which traces first. */
+ * were traced.  CX_EXEC_WAVEFRONT traces fewer rays than CX_EXEC_MEGAKERNEL for the same results and
+ * counts what it traces: it keeps a prefix vertex's hit that the reference traces again for NEE
+ * (path_gen.h:165-187), and it evaluates what a path or shift would contribute before its last
+ * shadow ray and leaves the ray out if that is nothing whatever the answer (no BSDF density towards
+ * the light or across the reconnection, a contribution of zero). */
 typedef struct cx_frame_stats {
     float passMs[CX_PASS_COUNT];
     float totalMs;
@@ -368,7 +368,7 @@ int cx_renderer_begin_frame(cx_renderer* r, const cx_camera* cam, int cameraChan
 int cx_pass_launch(cx_renderer* r, cx_pass pass, const cx_launch_params* params, void* stream);
 /*
  * Execution strategy of the passes; both give identical images, reservoirs and neighbour lists
- * (their counts of shadow rays differ, cx_frame_stats).  No counterpart in the reference, whose
+ * (their ray counts differ, cx_frame_stats).  No counterpart in the reference, whose
  * passes are single OptiX raygen launches.
  *   CX_EXEC_WAVEFRONT (default): path generation and shifts run as state machines whose
  *     rays are answered by separate traversal kernels, several launches per pass, with no
