@@ -12,6 +12,14 @@ static_assert(BLOCK == TRACE_BLOCK, "the traversal stack's column stride");
 static constexpr int TILE_X = 16;
 static constexpr int TILE_Y = 8;
 
+// The pass kernels need 225 to 320 registers left to themselves: past 256 one wavefront runs per SIMD
+// where two do at 256 (their stacks' LDS allows five blocks, ten wavefronts, per CU).  Held to two, 18
+// to 64 values are spilled.  1000x600 on 271 k triangles, ms without and with the hold: path tracer
+// 4.09 and 2.28, ReSTIR PT 7.25 and 4.23 (5.64 with the spatial pass alone left at one wavefront),
+// Conditional ReSTIR with 16 gathered suffixes, whose 32-slot gather goes from 320 registers to 256,
+// 23.4 with it.
+#define CX_PASS_WAVES __attribute__((amdgpu_waves_per_eu(2, 8)))
+
 #define CX_STACK_DECL                                  \
     __shared__ int s_stack[STACK_DEPTH * BLOCK];       \
     TraceCtx tc;                                       \
@@ -80,7 +88,7 @@ __device__ __forceinline__ void store_gbuf(const FrameArgs& A, uint32_t p, uint6
 // ------------------------------------------------------------------------------------------
 // prefix_gen_temp_reuse (shader/prefix_gen_temp_reuse.cu:11-193)
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void k_prefix_gen_temp(FrameArgs A) {
+__global__ __launch_bounds__(BLOCK) CX_PASS_WAVES void k_prefix_gen_temp(FrameArgs A) {
     CX_STACK_DECL
     uint32_t x, y, p;
     if (tile_pixel(A, x, y, p)) {
@@ -162,7 +170,7 @@ __global__ __launch_bounds__(BLOCK) void k_prefix_gen_temp(FrameArgs A) {
 // back buffer, which nothing writes during the pass (pass-entry snapshot); the front->back
 // copy of :162-163 is a separate copy after the kernel.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void k_prefix_spatial(FrameArgs A) {
+__global__ __launch_bounds__(BLOCK) CX_PASS_WAVES void k_prefix_spatial(FrameArgs A) {
     CX_STACK_DECL
     uint32_t x, y, p;
     if (tile_pixel(A, x, y, p)) {
@@ -247,7 +255,7 @@ __device__ __forceinline__ void invalidate(SuffixRes& r) {   // suffix_gen_temp_
 // suffix_gen_temp_reuse (shader/suffix_gen_temp_reuse.cu:19-134), with the unconditional
 // front->back copy of :132-133 fused into the store.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void k_suffix_gen_temp(FrameArgs A) {
+__global__ __launch_bounds__(BLOCK) CX_PASS_WAVES void k_suffix_gen_temp(FrameArgs A) {
     CX_STACK_DECL
     uint32_t x, y, p;
     if (tile_pixel(A, x, y, p)) {
@@ -318,7 +326,7 @@ __global__ __launch_bounds__(BLOCK) void k_suffix_gen_temp(FrameArgs A) {
 // suffix_spatial_reuse (shader/suffix_spatial_reuse.cu:16-167).  Both neighbour loops read the
 // back buffer (equal to the front buffer at pass entry); the copy of :165-166 follows the kernel.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void k_suffix_spatial(FrameArgs A) {
+__global__ __launch_bounds__(BLOCK) CX_PASS_WAVES void k_suffix_spatial(FrameArgs A) {
     CX_STACK_DECL
     uint32_t x, y, p;
     if (tile_pixel(A, x, y, p)) {
@@ -887,7 +895,7 @@ __device__ __forceinline__ V3 gather_not_canon(const FrameArgs& A, TraceCtx& tc,
 }
 
 template <int KR>
-__global__ __launch_bounds__(BLOCK) void k_final_gather(FrameArgs A) {
+__global__ __launch_bounds__(BLOCK) CX_PASS_WAVES void k_final_gather(FrameArgs A) {
     CX_STACK_DECL
     uint32_t x, y, p;
     if (tile_pixel(A, x, y, p)) {
