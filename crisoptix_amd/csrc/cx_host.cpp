@@ -930,6 +930,7 @@ int cx_scene_build(cx_ctx* ctx, const cx_scene_desc* d, cx_scene** out) {
     for (int a = 0; a < 3; a++) {
         s->info.boundsMin[a] = mn[a];
         s->info.boundsMax[a] = mx[a];
+        s->d.reach = std::max({s->d.reach, -mn[a], mx[a]});
     }
     s->info.numTriangles = d->numTriangles;
     s->info.numVertices = d->numVertices;
@@ -1019,6 +1020,7 @@ int cx_bvh_host_trace(const cx_scene_desc* d, const float* rays, uint32_t n, int
         width = wantWidth;
     if (widthUsed) *widthUsed = width;
     DScene S{};
+    for (size_t i = 0; i < 3 * (size_t)d->numVertices; i++) S.reach = std::max(S.reach, std::fabs(d->positions[i]));
     S.nodes = bvh.nodes.data();
     S.wnodes = width > 2 ? wide.data() : nullptr;
     S.tris = bvh.tris.data();
@@ -1044,7 +1046,7 @@ int cx_bvh_host_trace(const cx_scene_desc* d, const float* rays, uint32_t n, int
     auto run = [&](auto widthTag, auto anyTag, TravRay& tr, HostStack& st) {
         constexpr int Wd = decltype(widthTag)::value;
         constexpr bool Any = decltype(anyTag)::value;
-        while (!trav_step<Any, Wd>(S, tr, st)) {
+        while (!trav_step<Any, Wd, true>(S, tr, st)) {
         }
     };
     for (uint32_t i = 0; i < n; i++) {
@@ -1054,13 +1056,13 @@ int cx_bvh_host_trace(const cx_scene_desc* d, const float* rays, uint32_t n, int
         const V3 o{r[0], r[1], r[2]}, dir{r[3], r[4], r[5]};
         auto go = [&](auto anyTag) {
             if (width == 4) {
-                trav_init<4>(S, tr, o, dir, r[6], r[7]);
+                trav_init<4, true>(S, tr, o, dir, r[6], r[7]);
                 run(std::integral_constant<int, 4>{}, anyTag, tr, st);
             } else if (width == 8) {
-                trav_init<8>(S, tr, o, dir, r[6], r[7]);
+                trav_init<8, true>(S, tr, o, dir, r[6], r[7]);
                 run(std::integral_constant<int, 8>{}, anyTag, tr, st);
             } else {
-                trav_init<2>(S, tr, o, dir, r[6], r[7]);
+                trav_init<2, true>(S, tr, o, dir, r[6], r[7]);
                 run(std::integral_constant<int, 2>{}, anyTag, tr, st);
             }
         };

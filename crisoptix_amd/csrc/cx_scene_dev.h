@@ -60,7 +60,8 @@ struct DScene {
     int32_t wroot;        // root of `wnodes`
     uint32_t width;       // 2: traverse `nodes`; 4 or 8: traverse `wnodes`
     uint32_t numTextures;
-    uint32_t pad[2];
+    float reach;          // largest coordinate of any vertex, by magnitude
+    uint32_t pad;
     const float* __restrict__ uv;         // [V][2], or null (all zero)
     const uint32_t* __restrict__ texels;  // RGBA8 texels of every texture, one word each
     const uint4* __restrict__ texInfo;    // [textures]: first texel, width, height, -
@@ -133,10 +134,18 @@ struct Hit {
 // rounding of the fma is relative and covered by the far plane's slack; every box the ray enters
 // is so reported as entered.  A ray with d_i = 0 never changes x_i: its inv_i is a large power of
 // two (the product is then exact) and its interval is widened by 2^-40 in x_i, so that a box
-// whose face holds the origin is entered.  A component that overflows makes nn_i or nf_i infinite
-// or NaN, which fmaxf / fminf pass over: the axis then constrains nothing.
+// whose face holds the origin is entered.
+//
+// Where an interval is not finite (a reciprocal or a product overflows: a subnormal component, an
+// origin of 1e30, a direction of 1e-37) it would constrain nothing, for fmaxf / fminf pass over it, and
+// the ray would visit most of the tree: 100 k rays on 1.06 M triangles took 59 ms with one component of
+// 1e-40 and 1.3 s with directions of 1e-37, 0.17 and 0.35 ms as it is.  In the caller's ray arrays (ODD:
+// rays of any floats) such a ray is `odd`: a node's planes are moved to its origin first, so that its
+// intervals are those of o = 0.  A frame's rays, of unit length from points of the scene, do without:
+// asking for odd rays in their steps took 2.7 % of the 1080p frame.
 struct RaySlab {
     V3 inv, nn, nf;
+    bool odd;
 };
 
 CX_HD void slab_axis(float o, float d, float big, float& inv, float& nn, float& nf) {
@@ -147,17 +156,59 @@ CX_HD void slab_axis(float o, float d, float big, float& inv, float& nn, float& 
     nf = noi + e;
 }
 
-CX_HD RaySlab slab_init(V3 o, V3 d) {
+// An axis of an odd ray.  An infinite reciprocal (d = 0 or below 3e-39) is taken as the largest
+// number, and its interval is widened by `cover`, a time that no hit lies beyond.
+CX_HD void slab_axis_odd(float d, float cover, float& inv, float& nn, float& nf) {
+    const float most = 3.4028235e38f, q = 1.0f / d;
+    const bool beyond = fabsf(q) > most;
+    inv = beyond ? copysignf(most, d) : q;
+    nf = beyond ? cover : 1e-30f;
+    nn = -nf;
+}
+
+template <bool ODD>
+CX_HD RaySlab slab_init(const DScene& S, V3 o, V3 d) {
     const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
     // 2^96 over the power of two at or below the largest component (0 and denormals as they are)
     const float p = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, m) & 0x7f800000u);
     const float big = 7.9228163e28f / (p > 0.0f ? p : 1.0f);
     RaySlab r;
+    r.odd = false;
     slab_axis(o.x, d.x, big, r.inv.x, r.nn.x, r.nf.x);
     slab_axis(o.y, d.y, big, r.inv.y, r.nn.y, r.nf.y);
     slab_axis(o.z, d.z, big, r.inv.z, r.nn.z, r.nf.z);
+    // 2^96 over a subnormal p says nothing of the ray's times, so such a ray is odd as well
+    if (ODD && !(p > 0.0f && fabsf(r.nn.x) < INFINITY && fabsf(r.nf.x) < INFINITY && fabsf(r.nn.y) < INFINITY &&
+                 fabsf(r.nf.y) < INFINITY && fabsf(r.nn.z) < INFINITY && fabsf(r.nf.z) < INFINITY)) {
+        if (!(fabsf(o.x) < INFINITY && fabsf(o.y) < INFINITY && fabsf(o.z) < INFINITY) || d.x != d.x || d.y != d.y ||
+            d.z != d.z || m == 0.0f) {
+            // every triangle's t is a NaN (tri_hit): no box is entered
+            r.inv.x = 1.0f;
+            r.nn.x = INFINITY;
+            r.nf.x = -INFINITY;
+        } else {
+            // along the largest component no vertex is farther than the origin and the scene reach
+            const float far = fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + S.reach;
+            const float cover = fminf(4.0f * far / p, 3.4028235e38f);
+            r.odd = true;
+            slab_axis_odd(d.x, cover, r.inv.x, r.nn.x, r.nf.x);
+            slab_axis_odd(d.y, cover, r.inv.y, r.nn.y, r.nf.y);
+            slab_axis_odd(d.z, cover, r.inv.z, r.nn.z, r.nf.z);
+        }
+    }
     return r;
 }
+
+// Whether any lane that asks has an odd ray, and what a plane of this lane's ray is moved by.
+CX_HD bool slab_any_odd(const RaySlab& r) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __ballot(r.odd) != 0ull;
+#else
+    return r.odd;
+#endif
+}
+
+CX_HD V3 slab_shift(V3 o, const RaySlab& r) { return r.odd ? o : V3{0.0f, 0.0f, 0.0f}; }
 
 // Entry distance of a box whose near and far planes (by the signs of inv) are given, and whether
 // the ray enters it in [tmin, tcap].  The far plane carries a relative slack so that a triangle
@@ -373,6 +424,16 @@ CX_HD WideLoads wide_load(const float4* nodes, uint32_t off, const RaySlab& r) {
     return w;
 }
 
+// Moves a node's planes to the origin of an odd ray.
+CX_HD void wide_shift(WideLoads& w, V3 by) {
+    w.nx -= by.x;
+    w.fx -= by.x;
+    w.ny -= by.y;
+    w.fy -= by.y;
+    w.nz -= by.z;
+    w.fz -= by.z;
+}
+
 CX_HD void wide_keys(const WideLoads& w, const RaySlab& r, float tmin, float tcap, double* k) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -384,8 +445,9 @@ CX_HD void wide_keys(const WideLoads& w, const RaySlab& r, float tmin, float tca
 }
 
 // wide_visit of a 4-wide node whose float4 are loaded.
-template <typename Stack>
-CX_HD bool wide_visit4(const WideLoads& w, int& ref, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
+template <bool ODD, typename Stack>
+CX_HD bool wide_visit4(WideLoads& w, int& ref, V3 o, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
+    if (ODD && slab_any_odd(r)) wide_shift(w, slab_shift(o, r));
     double k[4];
     wide_keys(w, r, tmin, tcap, k);
     key_cswap(k[0], k[1]);
@@ -399,14 +461,19 @@ CX_HD bool wide_visit4(const WideLoads& w, int& ref, const RaySlab& r, float tmi
     return true;
 }
 
-template <int N, typename Stack>
-CX_HD bool wide_visit(const DScene& S, int& ref, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
+template <int N, bool ODD, typename Stack>
+CX_HD bool wide_visit(const DScene& S, int& ref, V3 o, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
     if constexpr (N == 4) {
-        return wide_visit4(wide_load(S.wnodes, (uint32_t)ref * 128u, r), ref, r, tmin, tcap, st, sp);
+        WideLoads w = wide_load(S.wnodes, (uint32_t)ref * 128u, r);
+        return wide_visit4<ODD>(w, ref, o, r, tmin, tcap, st, sp);
     } else {
         double k[8];
-        const WideLoads w0 = wide_load(S.wnodes, (uint32_t)ref * 256u, r);
-        const WideLoads w1 = wide_load(S.wnodes, (uint32_t)ref * 256u + 128u, r);
+        WideLoads w0 = wide_load(S.wnodes, (uint32_t)ref * 256u, r);
+        WideLoads w1 = wide_load(S.wnodes, (uint32_t)ref * 256u + 128u, r);
+        if (ODD && slab_any_odd(r)) {
+            wide_shift(w0, slab_shift(o, r));
+            wide_shift(w1, slab_shift(o, r));
+        }
         wide_keys(w0, r, tmin, tcap, k);
         wide_keys(w1, r, tmin, tcap, k + 4);
         // Batcher's odd-even merge sort of 8 keys (19 compare-exchanges).
@@ -429,11 +496,17 @@ CX_HD bool wide_visit(const DScene& S, int& ref, const RaySlab& r, float tmin, f
 
 // One binary node: the nearer hit child in ref (the farther one pushed); false when neither
 // child box is hit.
-template <typename Stack>
-CX_HD bool bin_visit(const DScene& S, int& ref, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
+template <bool ODD, typename Stack>
+CX_HD bool bin_visit(const DScene& S, int& ref, V3 o, const RaySlab& r, float tmin, float tcap, Stack& st, int& sp) {
     const float4* n = S.nodes + 4 * (size_t)ref;
-    const float4 a = n[0], b = n[1], c = n[2];
+    float4 a = n[0], b = n[1], c = n[2];
     const int4 dd = __builtin_bit_cast(int4, n[3]);
+    if (ODD && slab_any_odd(r)) {
+        const V3 by = slab_shift(o, r);
+        a = make_float4(a.x - by.x, a.y - by.x, a.z - by.y, a.w - by.y);
+        b = make_float4(b.x - by.x, b.y - by.x, b.z - by.y, b.w - by.y);
+        c = make_float4(c.x - by.z, c.y - by.z, c.z - by.z, c.w - by.z);
+    }
     const bool sx = __builtin_signbitf(r.inv.x), sy = __builtin_signbitf(r.inv.y), sz = __builtin_signbitf(r.inv.z);
     bool h0, h1;
     const float t0 = slab_box(sx ? a.y : a.x, sx ? a.x : a.y, sy ? a.w : a.z, sy ? a.z : a.w, sz ? c.y : c.x,
@@ -452,16 +525,16 @@ CX_HD bool bin_visit(const DScene& S, int& ref, const RaySlab& r, float tmin, fl
     return false;
 }
 
-template <bool ANY, int N, typename Stack>
+template <bool ANY, int N, bool ODD, typename Stack>
 CX_HD bool traverse_wide(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& best,
                                               Stack& st) {
     const RayPre rp = ray_pre(d);
-    const RaySlab sl = slab_init(o, d);
+    const RaySlab sl = slab_init<ODD>(S, o, d);
     int sp = 0;
     int ref = S.wroot;
     while (true) {
         if (ref >= 0) {
-            if (wide_visit<N>(S, ref, sl, tmin, best.t, st, sp)) continue;
+            if (wide_visit<N, ODD>(S, ref, o, sl, tmin, best.t, st, sp)) continue;
         } else {
             if (leaf_hits<ANY>(S, ref, o, rp, tmin, best)) return true;
         }
@@ -471,7 +544,7 @@ CX_HD bool traverse_wide(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hi
     return best.prim != INVALID_PRIM;
 }
 
-template <bool ANY, typename Stack>
+template <bool ANY, bool ODD, typename Stack>
 CX_HD bool traverse_bin(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& best,
                                              Stack& st) {
     best.prim = INVALID_PRIM;
@@ -480,12 +553,12 @@ CX_HD bool traverse_bin(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit
     best.v = 0.0f;
     if (S.numTris == 0) return false;
     const RayPre rp = ray_pre(d);
-    const RaySlab sl = slab_init(o, d);
+    const RaySlab sl = slab_init<ODD>(S, o, d);
     int sp = 0;
     int ref = S.root;
     while (true) {
         if (ref >= 0) {
-            if (bin_visit(S, ref, sl, tmin, best.t, st, sp)) continue;
+            if (bin_visit<ODD>(S, ref, o, sl, tmin, best.t, st, sp)) continue;
         } else {
             if (leaf_hits<ANY>(S, ref, o, rp, tmin, best)) return true;
         }
@@ -510,10 +583,10 @@ struct TravRay {
 };
 
 
-template <int WIDTH>
+template <int WIDTH, bool ODD>
 CX_HD void trav_init(const DScene& S, TravRay& r, V3 o, V3 d, float tmin, float tmax) {
     r.o = o;
-    r.sl = slab_init(o, d);
+    r.sl = slab_init<ODD>(S, o, d);
     r.rp = ray_pre(d);
     r.tmin = tmin;
     r.best = Hit{INVALID_PRIM, tmax, 0.0f, 0.0f};
@@ -529,7 +602,7 @@ CX_HD void trav_init(const DScene& S, TravRay& r, V3 o, V3 d, float tmin, float 
 // leaves issue their fetches (7 and 3 float4) before either kind is processed, so a wavefront
 // split between the two waits once per step; a leaf step tests one triangle and leaves the lane
 // on the rest of the leaf, so the leaf branch costs one triangle test per step.
-template <int WIDTH, typename Stack>
+template <int WIDTH, bool ODD, typename Stack>
 CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& st, bool any) {
     if (S.numTris == 0) return true;
     const int top = st.peek(r.sp);
@@ -556,7 +629,7 @@ CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& st, bool any) {
         asm("" : "+v"(w.nx), "+v"(w.fx), "+v"(w.ny), "+v"(w.fy), "+v"(w.nz), "+v"(w.fz), "+v"(w.ref));
 #endif
         if (inner) {
-            if (wide_visit4(w, r.ref, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
+            if (wide_visit4<ODD>(w, r.ref, r.o, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
         } else {
             if (tri_hits_q(w.nx, w.fx, w.ny, r.o, r.rp, r.tmin, r.best, any)) return true;
             if ((code & 15u) > 1u) {
@@ -566,9 +639,9 @@ CX_HD bool trav_step_rt(const DScene& S, TravRay& r, Stack& st, bool any) {
         }
     } else if (r.ref >= 0) {
         if constexpr (WIDTH == 2) {
-            if (bin_visit(S, r.ref, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
+            if (bin_visit<ODD>(S, r.ref, r.o, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
         } else {
-            if (wide_visit<WIDTH>(S, r.ref, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
+            if (wide_visit<WIDTH, ODD>(S, r.ref, r.o, r.sl, r.tmin, r.best.t, st, r.sp)) return false;
         }
     } else {
         if (leaf_hits_rt(S, r.ref, r.o, r.rp, r.tmin, r.best, any)) return true;
@@ -612,12 +685,14 @@ __device__ __forceinline__ void quad_best(Hit& h) {
 // Traces one ray per quad to its end; `col` is the quad's stack column in LDS (STACK_DEPTH entries,
 // `stride` apart).  The whole quad calls it with the same ray.  Closest hit in best (prim
 // INVALID_PRIM: a miss), occlusion as best.prim != INVALID_PRIM.
+template <bool ODD>
 __device__ __forceinline__ void quad_trace(const DScene& S, V3 o, V3 d, float tmin, float tmax, bool any, Hit& best,
                                            int* col, int stride) {
     best = Hit{INVALID_PRIM, tmax, 0.0f, 0.0f};
     if (S.numTris == 0) return;
     const RayPre rp = ray_pre(d);
-    const RaySlab r = slab_init(o, d);
+    const RaySlab r = slab_init<ODD>(S, o, d);
+    const bool anyOdd = ODD && slab_any_odd(r);
     const uint32_t j = threadIdx.x & 3u;
     const uint32_t ax = 4u * j + ((__builtin_bit_cast(uint32_t, r.inv.x) >> 27) & 16u);
     const uint32_t ay = 4u * j + ((__builtin_bit_cast(uint32_t, r.inv.y) >> 27) & 16u) + 32u;
@@ -628,10 +703,19 @@ __device__ __forceinline__ void quad_trace(const DScene& S, V3 o, V3 d, float tm
         const int top = col[(sp > 0 ? sp - 1 : 0) * stride];
         if (ref >= 0) {
             const uint32_t off = (uint32_t)ref * 128u;
-            const float nx = *(const float*)(nodes + (off | ax)), fx = *(const float*)(nodes + ((off | ax) ^ 16u));
-            const float ny = *(const float*)(nodes + (off | ay)), fy = *(const float*)(nodes + ((off | ay) ^ 16u));
-            const float nz = *(const float*)(nodes + (off | az)), fz = *(const float*)(nodes + ((off | az) ^ 16u));
+            float nx = *(const float*)(nodes + (off | ax)), fx = *(const float*)(nodes + ((off | ax) ^ 16u));
+            float ny = *(const float*)(nodes + (off | ay)), fy = *(const float*)(nodes + ((off | ay) ^ 16u));
+            float nz = *(const float*)(nodes + (off | az)), fz = *(const float*)(nodes + ((off | az) ^ 16u));
             const int child = *(const int*)(nodes + (off | (96u + 4u * j)));
+            if (anyOdd) {
+                const V3 by = slab_shift(o, r);
+                nx -= by.x;
+                fx -= by.x;
+                ny -= by.y;
+                fy -= by.y;
+                nz -= by.z;
+                fz -= by.z;
+            }
             bool h;
             const float t = slab_box(nx, fx, ny, fy, nz, fz, r, tmin, best.t, h);
             h = h && child != WIDE_EMPTY;
@@ -688,29 +772,29 @@ __device__ __forceinline__ void quad_trace(const DScene& S, V3 o, V3 d, float tm
     }
 }
 
-template <bool ANY, int WIDTH, typename Stack>
+template <bool ANY, int WIDTH, bool ODD, typename Stack>
 CX_HD bool trav_step(const DScene& S, TravRay& r, Stack& st) {
-    return trav_step_rt<WIDTH>(S, r, st, ANY);
+    return trav_step_rt<WIDTH, ODD>(S, r, st, ANY);
 }
 
 // Traversal at a BVH width fixed at compile time (WIDTH = S.width; the caller dispatches).
-template <bool ANY, int WIDTH, typename Stack>
+template <bool ANY, int WIDTH, bool ODD, typename Stack>
 CX_HD bool traverse_w(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& best, Stack& st) {
     best.prim = INVALID_PRIM;
     best.t = tmax;
     best.u = 0.0f;
     best.v = 0.0f;
     if (S.numTris == 0) return false;
-    if constexpr (WIDTH == 2) return traverse_bin<ANY>(S, o, d, tmin, tmax, best, st);
-    else return traverse_wide<ANY, WIDTH>(S, o, d, tmin, tmax, best, st);
+    if constexpr (WIDTH == 2) return traverse_bin<ANY, ODD>(S, o, d, tmin, tmax, best, st);
+    else return traverse_wide<ANY, WIDTH, ODD>(S, o, d, tmin, tmax, best, st);
 }
 
 // Dispatch on the scene's BVH width (uniform across a launch).
 template <bool ANY, typename Stack>
 CX_HD bool traverse_s(const DScene& S, V3 o, V3 d, float tmin, float tmax, Hit& best, Stack& st) {
-    if (S.width == 4) return traverse_w<ANY, 4>(S, o, d, tmin, tmax, best, st);
-    if (S.width == 8) return traverse_w<ANY, 8>(S, o, d, tmin, tmax, best, st);
-    return traverse_w<ANY, 2>(S, o, d, tmin, tmax, best, st);
+    if (S.width == 4) return traverse_w<ANY, 4, false>(S, o, d, tmin, tmax, best, st);
+    if (S.width == 8) return traverse_w<ANY, 8, false>(S, o, d, tmin, tmax, best, st);
+    return traverse_w<ANY, 2, false>(S, o, d, tmin, tmax, best, st);
 }
 
 // Traversal with the whole stack in a per-thread LDS column (stack[i * TRACE_BLOCK]).

@@ -123,6 +123,7 @@ __device__ __forceinline__ uint32_t chunk_ray(const ChunkRange& c, uint32_t v, u
 // {direction, tmax} and the place of its answer; store: the answer of a closest-hit ray or, any, of
 // a shadow ray.
 struct QueueRays {
+    static constexpr bool ODD = false;
     const Queue& q;
     const QIndex& qi;
     const FinalArgs& F;
@@ -145,6 +146,7 @@ struct QueueRays {
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 struct ArrayRays {
+    static constexpr bool ODD = true;   // any floats (RaySlab)
     const float* rays;
     uint32_t* prim;   // occlusion: the flags
     float *t, *u, *v;
@@ -194,7 +196,7 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Rays& rays, 
                         const uint32_t i = any ? chunk_ray(cs, v - cc.cnt, w, waves) : chunk_ray(cc, v, w, waves);
                         float4 a, b;
                         slot = rays.fetch(i, a, b);
-                        trav_init<WIDTH>(S, r, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w);
+                        trav_init<WIDTH, Rays::ODD>(S, r, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w);
                         has = true;
                     }
                 }
@@ -205,7 +207,7 @@ __device__ __forceinline__ void trace_chunks(const DScene& S, const Rays& rays, 
             if (cursor >= cnt) break;
             continue;
         }
-        if (trav_step_rt<WIDTH>(S, r, st, any)) {
+        if (trav_step_rt<WIDTH, Rays::ODD>(S, r, st, any)) {
             rays.store(slot, any, r.best);
             has = false;
         }
@@ -231,7 +233,7 @@ __device__ __forceinline__ void trace_quads(const DScene& S, const Rays& rays, u
         float4 a, b;
         const uint32_t slot = rays.fetch(i, a, b);
         Hit h;
-        quad_trace(S, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w, any, h, lds + (threadIdx.x >> 2), WBLOCK / 4);
+        quad_trace<Rays::ODD>(S, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w, any, h, lds + (threadIdx.x >> 2), WBLOCK / 4);
         if ((threadIdx.x & 3u) == 0u) rays.store(slot, any, h);
     }
 }
@@ -312,7 +314,7 @@ __global__ __launch_bounds__(WBLOCK) void k_trace_few(DScene S, ArrayRays rays, 
     float4 a, b;
     rays.fetch(i, a, b);
     Hit h;
-    const bool hit = traverse_w<ANY, WIDTH>(S, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w, h, st);
+    const bool hit = traverse_w<ANY, WIDTH, true>(S, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, a.w, b.w, h, st);
     if (ANY) h.prim = hit ? 0u : INVALID_PRIM;
     rays.store(i, ANY, h);
 }
@@ -1469,10 +1471,10 @@ __device__ __forceinline__ void tail_job(const WaveArgs& W, const Queue& q, cons
         Hit h;
         const bool any = e.kind != EMIT_CLOSEST;
         if constexpr (QUADS) {
-            quad_trace(S, e.o, e.d, e.tmin, e.tmax, any, h, lds + (threadIdx.x >> 2), WBLOCK / 4);
+            quad_trace<false>(S, e.o, e.d, e.tmin, e.tmax, any, h, lds + (threadIdx.x >> 2), WBLOCK / 4);
         } else {
-            if (any) traverse_w<true, WIDTH>(S, e.o, e.d, e.tmin, e.tmax, h, st);
-            else traverse_w<false, WIDTH>(S, e.o, e.d, e.tmin, e.tmax, h, st);
+            if (any) traverse_w<true, WIDTH, false>(S, e.o, e.d, e.tmin, e.tmax, h, st);
+            else traverse_w<false, WIDTH, false>(S, e.o, e.d, e.tmin, e.tmax, h, st);
         }
         const bool hit = h.prim != INVALID_PRIM;
         const uint4 r = any ? uint4{hit ? 1u : 0u, 0u, 0u, 0u}

@@ -60,6 +60,53 @@ def shadow_rays(scene, n, seed):
     return rays
 
 
+def float_rays(sc, n, seed):
+    """{name: rays}: the same n rays with one thing about them at the ends of the float range."""
+    base = random_rays(sc, n, seed=seed)
+    size = np.float32(sc.scene_size())
+    with np.errstate(over="ignore", under="ignore", invalid="ignore"):
+        def d(axis, v):
+            r = base.copy()
+            r[:, 3 + axis] = v
+            return r
+
+        def o(axis, v, back=False):
+            r = base.copy()
+            r[:, axis] = v
+            if back:   # still through the scene
+                r[:, 3:6] = 0.0
+                r[:, 3 + axis] = -np.sign(v)
+            return r
+
+        def scale(v, zero=None):
+            r = base.copy()
+            r[:, 3:6] *= np.float32(v)
+            r[:, 6] = 0.0
+            r[:, 7] = np.inf if v > 1e-36 else 3.4e38   # below, the t of a hit may be infinite itself
+            if zero is not None:
+                r[:, 3 + zero] = 0.0
+            return r
+
+        out = {"as they are": base, "x 1e-40": d(0, 1e-40), "y 1e-40": d(1, 1e-40), "z -1e-42": d(2, -1e-42),
+               "x 1e-26": d(0, 1e-26), "x 0": d(0, 0.0), "x inf": d(0, np.inf), "x nan": d(0, np.nan),
+               "1e-20": scale(1e-20), "1e-30": scale(1e-30), "1e-37": scale(1e-37), "1e-39": scale(1e-39),
+               "1e30": scale(1e30), "1e-6, z 0": scale(1e-6, 2), "1e-30, y 0": scale(1e-30, 1),
+               "1e-37, x 0": scale(1e-37, 0), "1e30, x 0": scale(1e30, 0)}
+        for v in (1e5, 1e10, -1e15, 1e30, 3e38, np.inf, -np.inf, np.nan):
+            out[f"origin x {v}"] = o(0, v)
+            out[f"origin z {v}, back"] = o(2, v, True)
+        far = d(2, 0.0)
+        far[:, 2] += np.float32(1e10)
+        out["z 0, origin z 1e10"] = far
+        behind = base.copy()
+        behind[:, 6] = -10.0 * size
+        out["from behind the origin"] = behind
+        anywhere = base.copy()
+        anywhere[:, 6:8] = -np.inf, np.inf
+        out["the whole line"] = anywhere
+    return out
+
+
 def bits(a):
     return np.ascontiguousarray(a).view(np.uint32)
 

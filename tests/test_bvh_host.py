@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from crisoptix_amd import runtime, scenes
-from parity_util import bits, random_rays, random_soup, shadow_rays, small_grid_scene
+from parity_util import bits, float_rays, random_rays, random_soup, shadow_rays, small_grid_scene
 
 pytestmark = pytest.mark.skipif(not __import__("os").path.exists(runtime.LIB_PATH), reason="HIP library not built")
 
@@ -74,6 +74,50 @@ def test_axis_parallel_and_far_rays_match_brute_force(name, orc):
             assert np.array_equal(bits(x), bits(y)), width
         og, _ = runtime.host_trace(sc, rays, any_hit=True, width=width)
         assert np.array_equal(occ, og), width
+
+
+@pytest.mark.parametrize("name", ["cornell", "grid3"])
+def test_rays_of_any_floats_match_brute_force(name, orc):
+    """Directions, origins and intervals at the ends of the float range: closest hits and occlusion of
+    every width equal the oracle's loop over all triangles, bit for bit."""
+    sc = scenes.cornell_box(1, 8) if name == "cornell" else small_grid_scene()
+    brute = orc.OracleScene(sc, brute_force=True)
+    hits = 0
+    for what, rays in float_rays(sc, 300, seed=29).items():
+        ref, occ = brute.trace_closest(rays), brute.trace_occluded(rays).astype(np.uint32)
+        hits += int(np.sum(ref[0] != 0xFFFFFFFF))
+        for width in (2, 4, 8):
+            *got, _ = runtime.host_trace(sc, rays, width=width)
+            for x, y in zip(ref, got):
+                assert np.array_equal(bits(x), bits(y)), (what, width)
+            og, _ = runtime.host_trace(sc, rays, any_hit=True, width=width)
+            assert np.array_equal(occ, og), (what, width)
+    assert hits > 1500
+
+
+def test_rays_of_any_floats_visit_few_nodes():
+    """Such rays do not visit most of the tree.  A call's time beyond the tree's build stands for its
+    visits: on 70 k triangles 4000 plain rays take 7 to 30 ms, and 250 ms (one component of 1e-40) to
+    minutes (directions of 1e-39) where an interval of the box test overflowed and constrained nothing."""
+    import time
+    sc = scenes.object_grid(4, 2, ground_quads=40)
+
+    def best(rays):
+        t = []
+        for _ in range(3):
+            t0 = time.perf_counter()
+            runtime.host_trace(sc, rays, width=4)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    kinds = float_rays(sc, 4000, seed=31)
+    build = best(kinds["as they are"][:8])
+    took = {what: best(rays) - build for what, rays in kinds.items()}
+    print({k: round(v, 3) for k, v in took.items()})
+    # a direction of 1e-39 reaches less than one unit before its t overflows, and a box test of such times
+    # is that much blurred
+    assert took.pop("1e-39") < 2.0
+    assert max(took.values()) < 3 * max(took["as they are"], 0.02) + 0.08, took
 
 
 def test_wide8_collapse_falls_back_to_greedy_on_large_scene():

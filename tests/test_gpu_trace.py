@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from crisoptix_amd import scenes
-from parity_util import bits, random_rays, random_soup, shadow_rays, small_grid_scene
+from parity_util import bits, float_rays, random_rays, random_soup, shadow_rays, small_grid_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -242,6 +242,26 @@ def test_ray_counts_and_alignment(width, orc, cx_runtime, cx_ctx):
             for x, y in zip(ref, outs):
                 assert np.array_equal(np.resize(bits(x), n), bits(y.numpy())), (n, shift)
             assert np.array_equal(np.resize(occ, n), flags.numpy()), (n, shift)
+
+
+@pytest.mark.parametrize("width,most", [(2, 700_001), (4, 130_001), (8, 200_001)])
+@pytest.mark.parametrize("name", ["cornell", "grid3"])
+def test_rays_of_any_floats(name, width, most, orc, cx_runtime, cx_ctx):
+    """Directions, origins and intervals at the ends of the float range, few and many (the kernels of
+    short and long arrays): the bits of the oracle's loop over all triangles."""
+    sc = scenes.cornell_box(1, 8) if name == "cornell" else small_grid_scene()
+    gscene = cx_runtime.Scene(cx_ctx, sc, width=width)
+    assert gscene.info.bvhWidth == width
+    rays = np.concatenate(list(float_rays(sc, 150, seed=37).values()))
+    brute = orc.OracleScene(sc, brute_force=True)
+    ref, occ = brute.trace_closest(rays), brute.trace_occluded(rays)
+    for n in (len(rays), most):
+        print(f"{name} width {width} rays {n}", flush=True)
+        got = gscene.trace_closest(np.resize(rays, (n, 8)))
+        flags = gscene.trace_occluded(np.resize(rays, (n, 8)))
+        for x, y in zip(ref, got):
+            assert np.array_equal(np.resize(bits(x), n), bits(y)), n
+        assert np.array_equal(np.resize(occ, n), flags), n
 
 
 @pytest.mark.parametrize("k", [1023, 1024, 1025, 1100, 2304])
