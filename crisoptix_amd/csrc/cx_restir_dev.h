@@ -654,8 +654,10 @@ __device__ __forceinline__ float box_distance2(V3 q, float4 lo, float4 hi) {
 
 // A number that no squared distance whose rounded root is at most d exceeds: the root, the square
 // and the sum of roundings are within 2^-22 of d^2, or within the smallest normal number where
-// d^2 underflows.  Infinite for a d whose square overflows, NaN for NaN.
-__device__ __forceinline__ float square_limit(float d) { return d * d * 1.000001f + 2e-38f; }
+// d^2 underflows.  Infinite for a d whose square overflows, NaN for NaN, and below 0 for a d below
+// -1.5e-19, which no distance is within: entries of negative or (the largest of none) NaN radius are
+// left out by node.
+__device__ __forceinline__ float square_limit(float d) { return d * fabsf(d) * 1.000001f + 2e-38f; }
 
 // Deferred siblings of the entry query: (child reference, its distance bound).  The first SHORT
 // entries live in a per-thread LDS column (two ints per entry, lds[(2 i) * stride] and

@@ -98,3 +98,32 @@ def test_sizes_ties_and_extremes(n, k, orc, cx_runtime, cx_ctx):
     assert np.array_equal(io[held], ig[held])
     assert np.array_equal(do[held].view(np.uint32), dg[held].view(np.uint32))
     assert np.all(ig[~held] == 0xFFFFFFFF) and np.all(dg[~held].view(np.uint32) == 0)
+
+
+@pytest.mark.parametrize("k", [8, 31])
+def test_entries_without_a_reach_are_left_out_by_node(k, cx_runtime, cx_ctx):
+    """Entries of negative, NaN or -inf radius are no candidates, and a query does not visit them one
+    by one: with no other entries it finds nothing, in no more time than it takes to find its k among
+    entries of a usual radius (it took 3 to 250 times as long where a square lost the radius's sign)."""
+    import time
+    n = 100_000
+    pos, radius, _, q = make_entries(n, seed=3)
+    q = np.resize(q, (40_000, 3))
+    E = cx_runtime.Entries(cx_ctx, n)
+
+    def best(radius):
+        E.build(pos, radius, np.ones(n, np.uint8), pos.min(0), pos.max(0))
+        t = []
+        for _ in range(5):
+            t0 = time.perf_counter()
+            count = E.query(q, k)[2]
+            t.append(time.perf_counter() - t0)
+        return min(t), count
+
+    plain, count = best(radius)
+    assert count.any()
+    for r in (-1.0, -np.inf, np.nan):
+        took, count = best(np.full(n, r, np.float32))
+        print(f"k {k} radius {r}: {took * 1e3:.2f} ms against {plain * 1e3:.2f}", flush=True)
+        assert not count.any()
+        assert took < 1.5 * plain + 1e-3
