@@ -18,12 +18,13 @@ W, H = 40, 24
 
 
 def _params(name, size):
-    """The settings whose frames take the most machines: two gathers, prefix spatial reuse."""
-    mode = {"gather2": "conditional_restir", "prefix_spatial": "conditional_restir"}.get(name, name)
+    """The settings whose frames take the most machines: two gathers, prefix spatial reuse; eight gathers
+    take more than there are sets of counters (16)."""
+    mode = "conditional_restir" if name in ("gather2", "gather8", "prefix_spatial") else name
     p = abi.workload_params(mode, W, H, size)
     if mode == "conditional_restir":
         p.gatherRadius = 0.6
-        p.gatherN = 2 if name == "gather2" else 1
+        p.gatherN = {"gather2": 2, "gather8": 8}.get(name, 1)
         p.prefixEnableSpatial = 1 if name == "prefix_spatial" else 0
         p.prefixSpatialRounds = 2
     if mode == "path_tracer":
@@ -75,7 +76,7 @@ def _same_records(ref, ren, tag):
 
 
 @pytest.mark.parametrize("rounds", [abi.CX_WAVE_ROUNDS_DEFAULT, 1])
-@pytest.mark.parametrize("name", ["path_tracer", "restir_pt_cornell", "gather2", "prefix_spatial"])
+@pytest.mark.parametrize("name", ["path_tracer", "restir_pt_cornell", "gather2", "gather8", "prefix_spatial"])
 def test_recorded_passes_replay(name, rounds, cx_runtime, cx_ctx):
     """One frame's passes recorded into a caller's graph and replayed four times, with eager work and
     synchronisations between, against the same passes launched eagerly as often."""
@@ -118,7 +119,7 @@ def test_recorded_passes_replay(name, rounds, cx_runtime, cx_ctx):
 
 
 @pytest.mark.parametrize("rounds", [abi.CX_WAVE_ROUNDS_DEFAULT, 1])
-@pytest.mark.parametrize("name", ["gather2", "prefix_spatial"])
+@pytest.mark.parametrize("name", ["gather2", "gather8", "prefix_spatial"])
 def test_hand_driven_frames_between_graph_replays(name, rounds, cx_runtime, cx_ctx):
     """Graph-mode frames, frames driven pass by pass and frames of another renderer type, which
     takes fewer machines, in turn on one renderer."""
