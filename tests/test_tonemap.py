@@ -96,3 +96,26 @@ def test_gpu_tonemap_every_float_of_the_curve(orc, cx_runtime, cx_ctx):
             bad = np.flatnonzero(got != ref)
             print(f"part {i}: {part.size} floats, {bad.size} differ", flush=True)
             assert bad.size == 0, part[bad[:8]]
+
+
+@pytest.mark.gpu
+def test_gpu_tonemap_of_a_white_image_takes_little_longer(orc, cx_runtime, cx_ctx):
+    """A clamped image is 1.0 over whole regions, a value next to a step of the byte whose power is known:
+    it takes less than twice as long as a grey one (5 times where every value took the double power)."""
+    import time
+    times = {}
+    for v in (0.5, 1.0):
+        d = cx_runtime.DeviceArray.from_numpy(np.full(8_000_000, v, np.float32))
+        out = cx_runtime.DeviceArray((8_000_000,), np.uint8)
+        t = []
+        for _ in range(8):
+            cx_runtime.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                cx_ctx.check(cx_runtime.lib().cx_tonemap(cx_ctx.h, d.ptr, out.ptr, 8_000_000, None), "cx_tonemap")
+            cx_runtime.synchronize()
+            t.append(time.perf_counter() - t0)
+        times[v] = min(t)
+        assert np.all(out.numpy() == orc.tonemap(np.float32([v]))[0])
+    print({k: f"{x / 20 * 1e6:.1f} us" for k, x in times.items()})
+    assert times[1.0] < 2.0 * times[0.5], times
