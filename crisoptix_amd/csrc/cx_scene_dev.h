@@ -139,7 +139,7 @@ struct Hit {
 // Where an interval is not finite (a reciprocal or a product overflows: a subnormal component, an
 // origin of 1e30, a direction of 1e-37) it would constrain nothing, for fmaxf / fminf pass over it, and
 // the ray would visit most of the tree: 100 k rays on 1.06 M triangles took 59 ms with one component of
-// 1e-40 and 1.3 s with directions of 1e-37, 0.17 and 0.35 ms as it is.  In the caller's ray arrays (ODD:
+// 1e-40 and 1.3 s with directions of 1e-37, 0.13 and 0.37 ms as it is.  In the caller's ray arrays (ODD:
 // rays of any floats) such a ray is `odd`: a node's planes are moved to its origin first, so that its
 // intervals are those of o = 0.  A frame's rays, of unit length from points of the scene, do without:
 // asking for odd rays in their steps took 2.7 % of the 1080p frame.

@@ -96,28 +96,28 @@ def test_rays_of_any_floats_match_brute_force(name, orc):
 
 
 def test_rays_of_any_floats_visit_few_nodes():
-    """Such rays do not visit most of the tree.  A call's time beyond the tree's build stands for its
-    visits: on 70 k triangles 4000 plain rays take 7 to 30 ms, and 250 ms (one component of 1e-40) to
+    """Such rays do not visit most of the tree.  A call's processor time beyond the tree's build stands for
+    its visits: on 70 k triangles 30000 plain rays take 0.05 s, and 2 s (one component of 1e-40) to many
     minutes (directions of 1e-39) where an interval of the box test overflowed and constrained nothing."""
     import time
     sc = scenes.object_grid(4, 2, ground_quads=40)
 
     def best(rays):
         t = []
-        for _ in range(3):
-            t0 = time.perf_counter()
+        for _ in range(2):
+            t0 = time.process_time()
             runtime.host_trace(sc, rays, width=4)
-            t.append(time.perf_counter() - t0)
+            t.append(time.process_time() - t0)
         return min(t)
 
-    kinds = float_rays(sc, 4000, seed=31)
+    kinds = float_rays(sc, 30_000, seed=31)
+    # a direction of 1e-39 reaches less than one unit before its t overflows, and a box test of such times
+    # is that much blurred
+    kinds["1e-39"] = kinds["1e-39"][:1000]
     build = best(kinds["as they are"][:8])
     took = {what: best(rays) - build for what, rays in kinds.items()}
     print({k: round(v, 3) for k, v in took.items()})
-    # a direction of 1e-39 reaches less than one unit before its t overflows, and a box test of such times
-    # is that much blurred
-    assert took.pop("1e-39") < 2.0
-    assert max(took.values()) < 3 * max(took["as they are"], 0.02) + 0.08, took
+    assert max(took.values()) < 5 * max(took["as they are"], 0.1) + 0.5, took
 
 
 def test_wide8_collapse_falls_back_to_greedy_on_large_scene():
